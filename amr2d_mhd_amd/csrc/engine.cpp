@@ -375,8 +375,6 @@ enum { PF_STAGE = 0, PF_FILL, PF_CT, PF_CFL, PF_REGRID, PF_HOST_TOPO, PF_HOST_RE
 
 }  // namespace
 
-// stage-kernel tuner: trials per variant and leaf-count bucket
-constexpr int kTuneTrials = 3;
 
 struct amr_ctx {
   int NT = 20, ng = 2, nxi = 16;
@@ -459,26 +457,17 @@ struct amr_ctx {
   // compiled fill programs kept per instance besides the current one (LRU)
   int prog_cache_max = 4;
   // a step launched by step_begin and not yet completed by step_end
-  bool in_flight = false, step_trial = false;
+  bool in_flight = false;
   uint64_t prog_clock = 0;
-  // stage-kernel variant: fixed (0..kStageVariants-1) or chosen per leaf-count
-  // bucket by the tuner (-1): the first launches in a bucket try every variant
-  // kTuneTrials times, timed by the kernel's own device-clock span, then the
-  // one with the fastest trial per leaf is kept for that bucket
+  // stage-kernel variant: fixed (0..kStageVariants-1), or (-1) by stage_rule
+  // unless one was imported for the bucket of the leaf count
   int stage_variant = -1;
-  struct TuneBucket {
-    double us_per_leaf[kStageVariants] = {0};          // sum over the trials (reported as a mean)
-    double trial_us[kStageVariants][kTuneTrials] = {};  // each timed trial, us per leaf (decides: median)
-    int nval[kStageVariants] = {0};                     // timed trials
-    int n[kStageVariants] = {0};                        // trials launched
-    int chosen = -1;
+  struct StageBucket {
+    int chosen = -1;    // imported
+    bool used = false;  // stages have been launched in the bucket
   };
-  TuneBucket tune_by_spec[kStageSpecs][24];  // per stage-kernel specialisation
+  StageBucket stage_buckets[kStageSpecs][24];  // per stage-kernel specialisation
   int stage_spec = kStageGeneric;   // of the running instances (set at each topology rebuild)
-  TuneBucket* tune = tune_by_spec[0];
-  unsigned long long* d_span = nullptr;  // [stage 1 start, end, stage 2 start, end]
-  unsigned long long* h_span = nullptr;
-  int span_variant[2] = {-1, -1};
   double wall_khz = 0;
   hipGraphExec_t gexec = nullptr;
   // persistent step kernel (kernels.hpp): 0 = per-phase launches (the
@@ -2017,24 +2006,25 @@ int graph_capacity(int cur, int n, int hard_max) {
   return std::max(n, std::min(g, hard_max));
 }
 
-// A specialised stage kernel serves launches whose running instances all use
-// HLLD with a MUSCL-family limiter, or all HLLD with WENO5 (24x24 tiles).
-int stage_spec_of(const amr_ctx* c) {
-  bool hlld_muscl = true, hlld_weno5 = c->NT == 24 && c->ng == 4;
-  for (const Instance& I : c->inst) {
-    if (I.done) continue;
-    if (!(I.solver == kFluxHLLD && I.lim < kLimWENO3)) hlld_muscl = false;
-    if (!(I.solver == kFluxHLLD && I.lim == kLimWENO5)) hlld_weno5 = false;
-  }
-  return hlld_muscl ? kStageHLLDMuscl : hlld_weno5 ? kStageHLLDWeno5 : kStageGeneric;
-}
-
 // stage specialisation an instance's leaves can run with on their own
 int stage_class_of(const amr_ctx* c, const Instance& I) {
   if (I.solver == kFluxHLLD && I.lim < kLimWENO3) return kStageHLLDMuscl;
   if (I.solver == kFluxHLLD && I.lim == kLimWENO5 && c->NT == 24 && c->ng == 4) return kStageHLLDWeno5;
   if (I.solver == kFluxHLLC && I.lim < kLimWENO3) return kStageHLLCMuscl;
   return kStageGeneric;
+}
+
+// A specialised stage kernel serves launches whose running instances are all
+// of its class.
+int stage_spec_of(const amr_ctx* c) {
+  int spec = -1;
+  for (const Instance& I : c->inst) {
+    if (I.done) continue;
+    const int k = stage_class_of(c, I);
+    if (spec >= 0 && k != spec) return kStageGeneric;
+    spec = k;
+  }
+  return spec < 0 ? kStageHLLDMuscl : spec;
 }
 
 // when the running instances fall into more than one class, order the leaf
@@ -2101,7 +2091,6 @@ int rebuild_topology(amr_ctx* c) {
   c->nleaf = (int)c->h_leaves.size();
   {
     c->stage_spec = stage_spec_of(c);
-    c->tune = c->tune_by_spec[c->stage_spec];
     plan_stage_split(c);
   }
   // programs of instances whose tree changed: the current one if the tree is
@@ -2280,113 +2269,39 @@ void run_fill(amr_ctx* c, const FillSet& s) {
               c->launch_counts);
 }
 
-int tune_bucket(int nleaf) {
+int leaf_bucket(int nleaf) {
   int b = 0;
   while ((2 << b) <= nleaf && b < 23) b++;
   return b;
 }
 
-// variant of the next stage launch; sets *timed when the launch is a trial
-// (trials run only inside full steps, whose spans are collected)
-// The strip variants split a leaf over several workgroups, so they cannot run
-// a stage that reads and writes the same field (SSP-RK3's second stage reads
-// Us and writes Us: one strip's update would race with another's loads of
-// its halo rows).  The tuner leaves them out of RK3 contexts, and a fixed
-// strip variant runs such a stage as the whole-leaf 768-lane variant.
-bool strip_variant(int v) { return v == 6 || v == 7; }
-bool strips_allowed(const amr_ctx* c) { return c->rk != 3; }
-int stage_variant_for(const amr_ctx* c, int v, int step) {
-  return strip_variant(v) && c->rk == 3 && step == 2 ? 2 : v;
+// The strips split a leaf over several workgroups, so they cannot run a stage
+// that reads and writes the same field (SSP-RK3's second stage reads Us and
+// writes Us: one strip's update would race with another's loads of its halo
+// rows); such a stage runs as the wide kernel instead.
+int stage_variant_for(const amr_ctx* c, int step) {
+  const int b = c->stage_buckets[c->stage_spec][leaf_bucket(c->nleaf)].chosen;
+  const int v = c->stage_variant >= 0 ? c->stage_variant : b >= 0 ? b : stage_rule(c->nleaf);
+  return stage_kernel_of(v) == kStageStrips && c->rk == 3 && step == 2 ? kVariantWide : v;
 }
 
-int stage_choice(amr_ctx* c, bool* timed, bool allow_trial = true) {
-  *timed = false;
-  if (c->stage_variant >= 0) return c->stage_variant;
-  const auto& B = c->tune[tune_bucket(c->nleaf)];
-  if (B.chosen >= 0) return B.chosen;
-  if (!allow_trial) return 0;
-  // round robin over the variants (the one with the fewest trials), so that
-  // every variant's trials fall on about the same leaf counts
-  int next = -1;
-  for (int v = 0; v < kStageVariants; v++)
-    if ((strips_allowed(c) || !strip_variant(v)) && B.n[v] < kTuneTrials && (next < 0 || B.n[v] < B.n[next]))
-      next = v;
-  if (next >= 0) {
-    *timed = true;
-    return next;
-  }
-  return 0;
-}
-
-bool tuning(amr_ctx* c) {
-  if (c->stage_split) return false;  // split launches make no trials
-  bool t;
-  stage_choice(c, &t);
-  return t;
-}
-
-void run_stage(amr_ctx* c, int step, bool allow_trial = true) {
+void run_stage(amr_ctx* c, int step) {
+  const int v = stage_variant_for(c, step);
+  c->stage_buckets[c->stage_spec][leaf_bucket(c->nleaf)].used = true;
   if (c->stage_split) {
     // one launch per class of instances, each with its specialisation
-    // (the HLLC one exists for kSplitVariant only); no tuner trials
-    const int v = stage_variant_for(c, c->stage_variant >= 0 ? c->stage_variant : kSplitVariant, step);
-    c->span_variant[step - 1] = -1;
     for (int k = 0; k < c->split_n; k++) {
       const int n = c->split_off[k + 1] - c->split_off[k];
       if (n <= 0) continue;
       Timed tm(c, PF_STAGE, true);
       launch_stage(c->NT, c->ng, v, c->split_spec[k], c->F, c->d_split_leaves + c->split_off[k], n, c->d_ip, step,
-                   c->d_err, c->stream, tm.start(), tm.stop(), nullptr, nullptr);
+                   c->d_err, c->stream, tm.start(), tm.stop());
     }
     return;
   }
   Timed tm(c, PF_STAGE, true);
-  bool timed;
-  const int v = stage_variant_for(c, stage_choice(c, &timed, allow_trial), step);
-  unsigned long long* span = timed ? c->d_span + 2 * (step - 1) : nullptr;
-  c->span_variant[step - 1] = timed ? v : -1;
-  if (timed) {
-    // the trial counts as pending until the step's results come back
-    c->tune[tune_bucket(c->nleaf)].n[v] += 1;
-  }
   launch_stage(c->NT, c->ng, v, c->stage_spec, c->F, c->d_leaves, c->grid_leaves, c->d_ip, step, c->d_err, c->stream,
-               tm.start(), tm.stop(), span, c->launch_counts);
-}
-
-// fold the spans of this step's trial launches into the tuner
-void tune_collect(amr_ctx* c) {
-  auto& B = c->tune[tune_bucket(c->nleaf)];
-  for (int q = 0; q < 2; q++) {
-    const int v = c->span_variant[q];
-    if (v < 0) continue;
-    c->span_variant[q] = -1;
-    const unsigned long long t0 = ~c->h_span[2 * q], t1 = c->h_span[2 * q + 1];
-    if (t1 > t0 && c->wall_khz > 0) {
-      const double us = (double)(t1 - t0) / (c->wall_khz * 1e-3) / c->nleaf;
-      B.us_per_leaf[v] += us;
-      if (B.nval[v] < kTuneTrials) B.trial_us[v][B.nval[v]++] = us;
-    }
-  }
-  bool all = true;
-  for (int v = 0; v < kStageVariants; v++) all &= B.n[v] >= kTuneTrials || (!strips_allowed(c) && strip_variant(v));
-  if (all && B.chosen < 0) {
-    // the variant with the smallest median trial (one slow or fast outlier
-    // does not decide)
-    int best = -1;
-    double best_us = 0.;
-    for (int v = 0; v < kStageVariants; v++) {
-      if (!B.nval[v]) continue;
-      double t[kTuneTrials];
-      std::copy(B.trial_us[v], B.trial_us[v] + B.nval[v], t);
-      std::sort(t, t + B.nval[v]);
-      const double med = t[(B.nval[v] - 1) / 2];
-      if (best < 0 || med < best_us) {
-        best = v;
-        best_us = med;
-      }
-    }
-    B.chosen = best < 0 ? 0 : best;
-  }
+               tm.start(), tm.stop(), c->launch_counts);
 }
 
 // CT2D.cpp:11-124
@@ -2726,8 +2641,6 @@ int enqueue_step_persistent(amr_ctx* c) {
 // bounds, indicators and error records: stream-ordered launches only, so it
 // can be captured into a graph.
 int enqueue_step(amr_ctx* c) {
-  const bool trial = tuning(c);
-  if (trial) HIPCHK(hipMemsetAsync(c->d_span, 0, 4 * sizeof(unsigned long long), c->stream));
   {
     // the step's parameters (dt) ride on the first fill launch
     FillSet s0 = make_set(c, {{kU, kFillCell}, {kBi, kFillFace}});
@@ -2768,8 +2681,6 @@ int enqueue_step(amr_ctx* c) {
   run_fill(c, make_set(c, {{kU, kFillCell}}));
   launch_cfl_regrid(c, nullptr, c->grid_leaves);
   if (int e = download_results(c, c->grid_leaves, c->regrid_device)) return e;
-  if (trial)
-    HIPCHK(hipMemcpyAsync(c->h_span, c->d_span, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
   return 0;
 }
 
@@ -2825,21 +2736,18 @@ int step_begin(amr_ctx* c) {
   fill_params(c);
   const bool device_timing = (c->prof_mask & 0x1fu) != 0;
   if (persistent_step(c)) {
-    c->step_trial = false;
     if (int e = enqueue_step_persistent(c)) return e;
     c->steps_same_topo++;
     c->in_flight = true;
     return 0;
   }
-  c->step_trial = tuning(c);
-  if (c->graph_on && !device_timing && !c->step_trial && !c->dma_since_direct) {
+  if (c->graph_on && !device_timing && !c->dma_since_direct) {
     // the captured step serves this tree when its grids cover the counts
-    bool trial;
     amr_ctx::GraphKey k;
     k.epoch = c->topo_epoch;
     k.leaves = graph_capacity(c->gkey.leaves, c->nleaf, (int)std::min<int64_t>(c->cap_slots, INT32_MAX));
     k.chunks = graph_capacity(c->gkey.chunks, c->nchunks, INT32_MAX);
-    k.variant = stage_choice(c, &trial, false);
+    k.variant = stage_variant_for(c, 1);
     k.spec = c->stage_spec;
     c->grid_leaves = k.leaves;
     c->grid_chunks = k.chunks;
@@ -2879,7 +2787,6 @@ int step_end(amr_ctx* c, int* n_active) {
   }
   c->in_flight = false;
   if (int e = wait_errors(c)) return e;
-  if (c->step_trial) tune_collect(c);
   int active = 0;
   for (size_t q = 0; q < c->inst.size(); q++) {
     Instance& I = c->inst[q];
@@ -3038,8 +2945,6 @@ int amr_create(int n_inst, const amr_sim_config* cfgs, int64_t slot_capacity, am
       hipMalloc((void**)&c->dtree.leafs, 4 * tree_blocks) != hipSuccess ||
       hipMemset(c->dtree.leafs, 0, 4 * tree_blocks) != hipSuccess ||
       hipHostMalloc((void**)&c->h_rec, rec_bytes) != hipSuccess ||
-      hipMalloc((void**)&c->d_span, 4 * sizeof(unsigned long long)) != hipSuccess ||
-      hipHostMalloc((void**)&c->h_span, 4 * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc((void**)&c->d_sync, sizeof(GridSync)) != hipSuccess ||
       hipMemset(c->d_sync, 0, sizeof(GridSync)) != hipSuccess ||
       hipMalloc((void**)&c->d_stamps, sizeof(unsigned long long) * (kMaxPhases + 1)) != hipSuccess ||
@@ -3067,7 +2972,6 @@ int amr_create(int n_inst, const amr_sim_config* cfgs, int64_t slot_capacity, am
     int dev = 0, khz = 0;
     if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess)
       c->wall_khz = khz;
-    if (c->wall_khz <= 0) c->stage_variant = 0;  // no device clock: no tuning
   }
   std::vector<int32_t> mU, mB;
   coarsen_maps(c->NT, c->ng, mU, mB);
@@ -3111,11 +3015,9 @@ int amr_destroy(amr_ctx* c) {
     hipEventDestroy(e[1]);
   }
   if (c->gexec) hipGraphExecDestroy(c->gexec);
-  hipFree(c->d_span);
   hipFree(c->d_sync);
   hipFree(c->d_stamps);
   if (c->h_stamps) hipHostFree(c->h_stamps);
-  if (c->h_span) hipHostFree(c->h_span);
   if (c->own_stream) hipStreamDestroy(c->own_stream);
   delete c;
   return AMR_OK;
@@ -3602,7 +3504,7 @@ int amr_stage(amr_ctx* c, int step) {
   if (c->topo_dirty)
     if (int e = rebuild_topology(c)) return e;
   if (int e = upload_params(c)) return e;
-  run_stage(c, step, false);
+  run_stage(c, step);
   return finish_call(c);
   AMR_CATCH
 }
@@ -3689,7 +3591,7 @@ int amr_set_stage_variant(amr_ctx* c, int variant) {
   AMR_TRY
   fill_touched(c);
   if (!c || variant < -1 || variant >= kStageVariants) return AMR_ERR_CONFIG;
-  c->stage_variant = (variant < 0 && c->wall_khz <= 0) ? 0 : variant;
+  c->stage_variant = variant;
   c->graph_dirty = true;
   return AMR_OK;
   AMR_CATCH
@@ -3698,11 +3600,10 @@ int amr_set_stage_variant(amr_ctx* c, int variant) {
 int amr_stage_tuning(amr_ctx* c, int nbuckets, int32_t* chosen, double* us_per_leaf) {
   AMR_TRY
   if (!c || nbuckets < 0) return AMR_ERR_CONFIG;
-  const auto* tune = c->tune_by_spec[stage_spec_of(c)];
+  const auto* buckets = c->stage_buckets[stage_spec_of(c)];
   for (int b = 0; b < nbuckets && b < 24; b++) {
-    if (chosen) chosen[b] = tune[b].chosen;
-    for (int v = 0; v < kStageVariants && us_per_leaf; v++)
-      us_per_leaf[b * kStageVariants + v] = tune[b].n[v] ? tune[b].us_per_leaf[v] / tune[b].n[v] : 0.0;
+    if (chosen) chosen[b] = buckets[b].chosen >= 0 || !buckets[b].used ? buckets[b].chosen : stage_rule(1 << b);
+    for (int v = 0; v < kStageVariants && us_per_leaf; v++) us_per_leaf[b * kStageVariants + v] = 0.0;
   }
   return AMR_OK;
   AMR_CATCH
@@ -3714,9 +3615,9 @@ int amr_set_stage_tuning(amr_ctx* c, int nbuckets, const int32_t* chosen) {
   if (!c || nbuckets < 0 || nbuckets > 24 || (nbuckets && !chosen)) return AMR_ERR_CONFIG;
   for (int b = 0; b < nbuckets; b++)
     if (chosen[b] < -1 || chosen[b] >= kStageVariants) return AMR_ERR_CONFIG;
-  auto* tune = c->tune_by_spec[stage_spec_of(c)];
+  auto* buckets = c->stage_buckets[stage_spec_of(c)];
   for (int b = 0; b < nbuckets; b++)
-    if (chosen[b] >= 0) tune[b].chosen = chosen[b];
+    if (chosen[b] >= 0) buckets[b].chosen = chosen[b];
   c->graph_dirty = true;
   return AMR_OK;
   AMR_CATCH

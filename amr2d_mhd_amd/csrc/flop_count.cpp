@@ -52,6 +52,7 @@ inline bool isnan(Counted a) { return std::isnan(a.v); }
 
 }  // namespace amr
 
+#define AMR_COUNT_OPS
 #define double Counted
 #include "physics.hpp"
 #undef double

@@ -37,34 +37,51 @@ struct RegridOp {
 
 bool tile_supported(int NT, int ng);
 
-// stage kernel variants (identical results): lanes per leaf block and where
-// the face fluxes live for the RK update --
-//   0: 256 lanes, fluxes in LDS      1: 512 lanes, LDS      2: 768 lanes, LDS
-//   3: 256 lanes, fluxes read back from ff/gg, compiled for 4 waves per SIMD
-//   4: 512 lanes, read back, 4 waves per SIMD   5: 512 lanes, LDS, 4 waves per SIMD
-//   6: each leaf split into 2 row strips, one workgroup per strip (fluxes in LDS)
-//   7: 4 row strips per leaf
-// The fewer-lane variants suit large leaf counts (throughput), the wide ones
-// and the strips small leaf counts (per-block latency, filling the device).
-// A non-null `span` receives the launch's device wall-clock span (see
-// stamp_start/stamp_end).
+// Stage kernels (identical results), and the variant numbers of the interface
+// that select them:
+//   wide    768 lanes a leaf block, face fluxes in LDS (1, 2, 5): one pass over
+//           the block's 578 faces, the shortest time of a single block
+//   narrow  256 lanes, fluxes read back from ff/gg (0, 3, 4): 25.6 KB of LDS and
+//           168 VGPRs, three blocks on a CU at a time whose load, face and
+//           update phases overlap
+//   strips  each block split into 4 row strips of 192 lanes (6, 7): four times
+//           the workgroups where the blocks alone leave CUs idle
+// stage_rule chooses by the number of leaf blocks of a launch.  Microseconds a
+// launch, rotor HLLD + MC (strips, wide, narrow): 52 blocks 10.9, 15.2, 19.3;
+// 136: 16.2, 16.0, 20.5; 196: 17.2, 16.5, 20.4; 340: 24.4, 25.7, 27.4; 436: 28.5,
+// 27.1, 28.3; 757: 41.2, 41.2, 34.3; 2352: 110, 117, 90.  HLLC + VanLeer at 100
+// blocks 15.1, 17.0, 23.6, HLLE at 340 25.7, 27.1, 28.4.
+enum { kStageWide, kStageNarrow, kStageStrips };
+constexpr int stage_kernel_of(int variant) {
+  return variant >= 6 ? kStageStrips : variant == 0 || variant == 3 || variant == 4 ? kStageNarrow : kStageWide;
+}
+constexpr int kVariantWide = 2, kVariantNarrow = 3, kVariantStrips = 7;
+inline int stage_rule(int nleaf) { return nleaf < 128 ? kVariantStrips : nleaf < 512 ? kVariantWide : kVariantNarrow; }
 constexpr int kStageVariants = 8;
 // stage-kernel specialisations: generic (solver and limiter read per leaf), or
 // HLLD with a MUSCL-family limiter, or HLLD with WENO5 (24x24 tiles, the only
 // ones with the ghost depth WENO5 needs), fixed at compile time
-// (kStageHLLCMuscl: HLLC with a MUSCL-family limiter, used for the HLLC part of
-// a launch split by specialisation; variant 5 only)
+// or HLLC with a MUSCL-family limiter.  The specialised kernels are 2-7% faster
+// than the generic one with the same settings (rotor5 at 340 blocks: 25.7 and
+// 26.7 us; WENO5 narrow 28 and 40 us: the generic code overruns the
+// instruction cache).
 enum { kStageGeneric = 0, kStageHLLDMuscl = 1, kStageHLLDWeno5 = 2, kStageHLLCMuscl = 3, kStageSpecs = 4 };
-// the variant a launch split by specialisation uses unless one is fixed
-constexpr int kSplitVariant = 5;
 // Work-list counts on the device (counts[kCountLeaves], counts[kCountChunks]):
 // a launch given `counts` may have a larger grid than its work (a captured
 // step replayed over changing trees) and its surplus workgroups exit; with
 // counts = null the grid is the work.
 enum { kCountLeaves = 0, kCountChunks = 1 };
+// one specialisation for one tile size (stage.hip, step.hip): 20 and 12 cells
+// a side for every specialisation but HLLD + WENO5, 24 for all
+template <int SPEC, int TILE>
+void launch_stage_tile(int variant, const FieldPtrs& F, const LeafItem* leaves, int nleaf, const InstParams* ip,
+                       int step, DevError* err, hipStream_t s, hipEvent_t ev_start, hipEvent_t ev_stop,
+                       const int32_t* counts);
+template <int SPEC, int TILE>
+const void* step_kernel_tile(int lanes_idx);
 void launch_stage(int NT, int ng, int variant, int spec, const FieldPtrs& F, const LeafItem* leaves, int nleaf,
                   const InstParams* ip, int step, DevError* err, hipStream_t s, hipEvent_t ev_start = nullptr,
-                  hipEvent_t ev_stop = nullptr, unsigned long long* span = nullptr, const int32_t* counts = nullptr);
+                  hipEvent_t ev_stop = nullptr, const int32_t* counts = nullptr);
 // corner EMF of RK stage `step` of an `rk`-stage scheme (CTtype per instance)
 void launch_emf(int NT, const FieldPtrs& F, const LeafItem* leaves, int nleaf, const InstParams* ip, int step,
                 int rk, DevError* err, hipStream_t s, const int32_t* counts = nullptr);

@@ -1,0 +1,444 @@
+// Device code of the other phases of a step: constrained transport, ghost
+// fills, the CFL bound and the refinement indicators.
+#pragma once
+#include "device.hpp"
+
+namespace amr {
+
+namespace {
+
+// --------------------------------------------------------------------- CT
+// CT2D.cpp:28-75 (CTtype 2) gas pressure and fast speed of one cell of the
+// stage state q (the reference's per-block p and C arrays, formed here per
+// corner for the four cells around it, by the same expressions)
+__device__ inline void ct2_pc(const double* q, int N2, int c, double g, double& p, double& C) {
+  const double q0 = q[c], q1 = q[N2 + c], q2 = q[2 * N2 + c], q3 = q[3 * N2 + c], q4 = q[4 * N2 + c],
+               q5 = q[5 * N2 + c], q6 = q[6 * N2 + c], q7 = q[7 * N2 + c];
+  p = (g - 1) * (q4 - 0.5 * ((q1 * q1 + q2 * q2 + q3 * q3) / q0 + (q5 * q5 + q6 * q6 + q7 * q7)));
+  C = sqrt((g * p + (q5 * q5 + q6 * q6 + q7 * q7)) / q0);
+}
+
+// CT2D.cpp:15-75: corner EMF from the face fluxes for i,j in [1,NT-1].
+// CTtype 1: the mean of the four face values.  CTtype 2 ("upwind"): the
+// y-flux and x-flux pairs weighted 1 - psi and psi, psi = dPx / (dPx + dPy)
+// where the pressure jump around the corner exceeds half the smallest
+// pressure (sw1) and the flow is compressive beyond a tenth of the smallest
+// fast speed (sw2), else psi = 0.5; the velocity divergence keeps the
+// reference's terms as written (two y-velocity quotients divide q2 by
+// itself, CT2D.cpp:45).  q is the stage state (Us, or U on the last stage).
+template <int NT>
+__device__ inline void emf_cell(const FieldPtrs& F, const LeafItem L, const InstParams* __restrict__ ip, int last,
+                                DevError* err, int step, int c) {
+  constexpr int N2 = NT * NT;
+  const int i = c % NT, j = c / NT;
+  if (i < 1 || j < 1) return;
+  const double* gg5 = F.f[kGG] + (size_t)L.gs * 8 * N2 + 5 * N2;
+  const double* ff6 = F.f[kFF] + (size_t)L.gs * 8 * N2 + 6 * N2;
+  const InstParams& P = ip[L.inst];
+  if (P.ct_type != 2) {
+    F.f[kEMF][(size_t)L.gs * N2 + c] = 0.25 * ((gg5[c - 1] + gg5[c]) - (ff6[c - NT] + ff6[c]));
+    return;
+  }
+  const double* q = F.f[last ? kU : kUs] + (size_t)L.gs * 8 * N2;
+  // cells (i, j), (i, j-1), (i-1, j), (i-1, j-1) of the reference's [i][j]
+  const int c00 = c, c0m = c - NT, cm0 = c - 1, cmm = c - 1 - NT;
+  double p00, p0m, pm0, pmm, C00, C0m, Cm0, Cmm;
+  ct2_pc(q, N2, c00, P.gamma, p00, C00);
+  ct2_pc(q, N2, c0m, P.gamma, p0m, C0m);
+  ct2_pc(q, N2, cm0, P.gamma, pm0, Cm0);
+  ct2_pc(q, N2, cmm, P.gamma, pmm, Cmm);
+  const double beta = 0.5, delta = 0.1;
+  const double dPx = 0.5 * fabs(p00 + p0m - pm0 - pmm);
+  const double dPy = 0.5 * fabs(p00 + pm0 - p0m - pmm);
+  const double* q0 = q;
+  const double* q1 = q + N2;
+  const double* q2 = q + 2 * N2;
+  const double divV = 0.5 * (q1[c00] / q0[c00] + q1[c0m] / q0[c0m] - q1[cm0] / q0[cm0] - q1[cmm] / q0[cmm]) +
+                      0.5 * (q2[c00] / q0[c00] + q2[cm0] / q2[cm0] - q2[c0m] / q2[c0m] - q2[cmm] / q0[cmm]);
+  double tP = pmm < p0m ? pmm : p0m;
+  const double tP1 = pm0 < p00 ? pm0 : p00;
+  tP = tP < tP1 ? tP : tP1;
+  const bool sw1 = (dPx + dPy) > beta * tP;
+  double tC = Cmm < C0m ? Cmm : C0m;
+  const double tC1 = Cm0 < C00 ? Cm0 : C00;
+  tC = tC < tC1 ? tC : tC1;
+  const bool sw2 = (-delta * tC) > divV;
+  double psi = 0.5;
+  if (sw1 && sw2) psi = dPx / (dPx + dPy);
+  if (psi < 0 || psi > 1) report(err, L.inst, error_key(step, kSeqCt | L.nb, 0, i, j, 0, L.nb, kErrCtPsi));
+  F.f[kEMF][(size_t)L.gs * N2 + c] = 0.5 * (1. - psi) * (gg5[c - 1] + gg5[c]) - 0.5 * psi * (ff6[c - NT] + ff6[c]);
+}
+
+template <int NT>
+__global__ __launch_bounds__(kThreads) void emf_kernel(FieldPtrs F, const LeafItem* __restrict__ leaves,
+                                                       const InstParams* __restrict__ ip, int last, DevError* err,
+                                                       int step, const int32_t* __restrict__ counts) {
+  if (counts && (int)blockIdx.y >= counts[kCountLeaves]) return;
+  const int c = blockIdx.x * kThreads + threadIdx.x;
+  if (c < NT * NT) emf_cell<NT>(F, leaves[blockIdx.y], ip, last, err, step, c);
+}
+
+// CT2D.cpp:78-92: face-B RK update from the edge EMF.  Stage input B (Bi for
+// step 1, else Bis), written array Bn (Bi on the last stage, else Bis) and
+// the step's starting value B0 = Bi; SSP-RK3 stages 2-3 are build-defined.
+__device__ inline double face_rk(int rk, int step, double B, double Bn, double B0, double dt, double res) {
+  if (step == 1) return B - dt * res;
+  if (rk == 2) return 0.5 * (B + Bn - dt * res);
+  if (step == 2) return 0.75 * B0 + 0.25 * (B - dt * res);
+  return (1. / 3.) * B0 + (2. / 3.) * (B - dt * res);
+}
+
+template <int NT>
+__device__ inline void bupdate_cell(const FieldPtrs& F, const LeafItem L, const InstParams* __restrict__ ip, int step,
+                                    int rk, int c) {
+  constexpr int N2 = NT * NT;
+  const int i = c % NT, j = c / NT;
+  const InstParams& P = ip[L.inst];
+  const double dt = P.dt, dxl = P.dx[L.lev];
+  const double* E = F.f[kEMF] + (size_t)L.gs * N2;
+  const double* B = F.f[step == 1 ? kBi : kBis] + (size_t)L.gs * 2 * N2;
+  const double* B0 = F.f[kBi] + (size_t)L.gs * 2 * N2;
+  double* Bn = F.f[step == rk ? kBi : kBis] + (size_t)L.gs * 2 * N2;
+  const int cjp = j < NT - 1 ? c + NT : c;
+  const int cip = i < NT - 1 ? c + 1 : c;
+  const double rx = (1. / dxl) * (E[cjp] - E[c]);
+  const double ry = -(1. / dxl) * (E[cip] - E[c]);
+  const double bx = face_rk(rk, step, B[c], Bn[c], B0[c], dt, rx);
+  const double by = face_rk(rk, step, B[N2 + c], Bn[N2 + c], B0[N2 + c], dt, ry);
+  Bn[c] = bx;
+  Bn[N2 + c] = by;
+}
+
+template <int NT>
+__global__ __launch_bounds__(kThreads) void bupdate_kernel(FieldPtrs F, const LeafItem* __restrict__ leaves,
+                                                           const InstParams* __restrict__ ip, int step, int rk,
+                                                           const int32_t* __restrict__ counts) {
+  if (counts && (int)blockIdx.y >= counts[kCountLeaves]) return;
+  const int c = blockIdx.x * kThreads + threadIdx.x;
+  if (c < NT * NT) bupdate_cell<NT>(F, leaves[blockIdx.y], ip, step, rk, c);
+}
+
+// CT2D.cpp:95-123: cell-centred B from the updated faces + energy correction
+template <int NT>
+__device__ inline void bsync_cell(const FieldPtrs& F, const LeafItem L, int last, int c) {
+  constexpr int N2 = NT * NT;
+  const int i = c % NT, j = c / NT;
+  const double* Bn = F.f[last ? kBi : kBis] + (size_t)L.gs * 2 * N2;
+  double* q = F.f[last ? kU : kUs] + (size_t)L.gs * 8 * N2;
+  const int ip = i < NT - 1 ? i + 1 : i, jp = j < NT - 1 ? j + 1 : j;
+  const double bx = 0.5 * (Bn[j * NT + ip] + Bn[j * NT + ip - 1]);
+  const double by = 0.5 * (Bn[N2 + jp * NT + i] + Bn[N2 + (jp - 1) * NT + i]);
+  const double q5 = q[5 * N2 + c], q6 = q[6 * N2 + c];
+  q[4 * N2 + c] = q[4 * N2 + c] + 0.5 * ((bx * bx + by * by) - ((q5 * q5) + (q6 * q6)));
+  q[5 * N2 + c] = bx;
+  q[6 * N2 + c] = by;
+}
+
+template <int NT>
+__global__ __launch_bounds__(kThreads) void bsync_kernel(FieldPtrs F, const LeafItem* __restrict__ leaves, int last,
+                                                         const int32_t* __restrict__ counts) {
+  if (counts && (int)blockIdx.y >= counts[kCountLeaves]) return;
+  const int c = blockIdx.x * kThreads + threadIdx.x;
+  if (c < NT * NT) bsync_cell<NT>(F, leaves[blockIdx.y], last, c);
+}
+
+// -------------------------------------------------------------- ghost fill
+// Single-pass execution of a compiled fill program.  Every destination's value
+// is a function of the pre-fill state only; a workgroup evaluates all values
+// of its chunk of ops, synchronises, then writes them.  The compiler places
+// each op that reads an element some other op writes in the same chunk as
+// that writer, so reads always see pre-fill values.
+struct FillCtx {
+  const double* base;
+  int nv, kind, N2, NT;
+  const FillGen* gen;
+};
+
+__device__ inline double fill_elem(const FillCtx& f, int64_t gs, int cell, int k) {
+  return f.base[((size_t)gs * f.nv + k) * f.N2 + cell];
+}
+
+// explicit operand of a general restriction (always a pre-fill element)
+__device__ inline double fill_ref(const FillCtx& f, int64_t ref, int k) {
+  return fill_elem(f, ref >> 16, (int)(ref & 0xffff), k);
+}
+
+// boundary.cpp (0.25 x 2x2 sum in misc.cpp:35-48 order), boundaryfc.cpp
+// (0.5 x face pair: along j for component 0, along i otherwise) and
+// boundaryec.cpp (injection); v[] holds (i1,j1),(i1,j1+1),(i1+1,j1),(i1+1,j1+1)
+__device__ inline double restrict_combine(int kind, int k, double v00, double v01, double v10, double v11) {
+  double v = 0.;
+  if (kind == kFillCell) {
+    v += v00;
+    v += v01;
+    v += v10;
+    v += v11;
+    return 0.25 * v;
+  }
+  if (kind == kFillFace) {
+    v += v00;
+    v += k == 0 ? v01 : v10;
+    return 0.5 * v;
+  }
+  return v00;
+}
+
+__device__ inline double gen_value(const FillCtx& f, const FillGen& g, int k) {
+  return restrict_combine(f.kind, k, fill_ref(f, g.ref[0], k), fill_ref(f, g.ref[1], k), fill_ref(f, g.ref[2], k),
+                          fill_ref(f, g.ref[3], k));
+}
+
+__device__ inline double fill_value(const FillCtx& f, const FillOp& op, int k) {
+  if (op.op == kFillCopy) return fill_elem(f, op.src, op.src_cell, k);
+  if (op.op == kFillRestrict) {
+    const int a = op.src_cell;
+    return restrict_combine(f.kind, k, fill_elem(f, op.src, a, k), fill_elem(f, op.src, a + f.NT, k),
+                            fill_elem(f, op.src, a + 1, k), fill_elem(f, op.src, a + 1 + f.NT, k));
+  }
+  return gen_value(f, f.gen[op.src], k);
+}
+
+// The program is a concatenation of per-instance segments of whole chunks:
+// chunk w belongs to the instance q with cprefix[q] <= w < cprefix[q+1].
+struct FillProgram {
+  const FillOp* const* ops;
+  const FillGen* const* gen;
+  const int32_t* cprefix;
+  int ninst;
+};
+
+__device__ inline int find_segment(const FillProgram& P, int w) {
+  int lo = 0, hi = P.ninst;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (P.cprefix[mid] <= w) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+
+template <int NV>
+__device__ inline void fill_field(const FillCtx& f, double* base, const FillOp& op, bool live) {
+  double v[NV];
+#pragma unroll
+  for (int k = 0; k < NV; k++) v[k] = live ? fill_value(f, op, k) : 0.;
+  __syncthreads();  // every read of the chunk precedes every write
+  if (live) {
+#pragma unroll
+    for (int k = 0; k < NV; k++) base[((size_t)op.dst_gs * NV + k) * f.N2 + op.dst_cell] = v[k];
+  }
+}
+
+// One chunk of the program per kFillChunk lanes (`lane` within the chunk); a
+// workgroup may run several chunks side by side, and every lane of it calls
+// this together (it synchronises the workgroup).  valid = false: no chunk.
+__device__ inline void fill_chunk(const FillProgram& P, const FillSet& set, int NT, int w, int lane, bool valid) {
+  FillOp op{};
+  op.op = kFillNop;
+  int q = 0;
+  if (valid) {
+    q = find_segment(P, w);
+    op = P.ops[q][(w - P.cprefix[q]) * kFillChunk + lane];
+  }
+  const bool live = op.op != kFillNop;
+  for (int fi = 0; fi < set.n; fi++) {
+    const FillCtx f{set.base[fi], set.nv[fi], set.kind[fi], NT * NT, NT, valid ? P.gen[q] : nullptr};
+    if (set.nv[fi] == 8) fill_field<8>(f, set.base[fi], op, live);
+    else if (set.nv[fi] == 2) fill_field<2>(f, set.base[fi], op, live);
+    else fill_field<1>(f, set.base[fi], op, live);
+  }
+}
+
+// restrict_combine for a kind fixed at compile time (the same IEEE
+// operations, no branch on the kind between an op's loads)
+template <int KIND>
+__device__ inline double restrict_kind(int k, double v00, double v01, double v10, double v11) {
+  double v = 0.;
+  if constexpr (KIND == kFillCell) {
+    v += v00;
+    v += v01;
+    v += v10;
+    v += v11;
+    return 0.25 * v;
+  } else if constexpr (KIND == kFillFace) {
+    v += v00;
+    v += k == 0 ? v01 : v10;
+    return 0.5 * v;
+  } else {
+    return v00;
+  }
+}
+
+// the NV components of one field of combine kind KIND for an op whose
+// operands are the elements e[t] (block slot << 16 | cell): one (copy) or
+// four (restriction, 2x2 order)
+template <int NV, int KIND, bool COPY>
+__device__ inline void fill_gather(const double* __restrict__ base, int N2, const int64_t* e, double* v) {
+  if constexpr (COPY) {
+    const double* p = base + (size_t)(e[0] >> 16) * NV * N2 + (e[0] & 0xffff);
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] = p[(size_t)k * N2];
+  } else {
+    const double* p0 = base + (size_t)(e[0] >> 16) * NV * N2 + (e[0] & 0xffff);
+    const double* p1 = base + (size_t)(e[1] >> 16) * NV * N2 + (e[1] & 0xffff);
+    const double* p2 = base + (size_t)(e[2] >> 16) * NV * N2 + (e[2] & 0xffff);
+    const double* p3 = base + (size_t)(e[3] >> 16) * NV * N2 + (e[3] & 0xffff);
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+      v[k] = restrict_kind<KIND>(k, p0[(size_t)k * N2], p1[(size_t)k * N2], p2[(size_t)k * N2], p3[(size_t)k * N2]);
+  }
+}
+
+// The same for a set of up to three fields with NV0, NV1, NV2 components
+// (0: absent) and combine kinds K0, K1, K2, fixed at compile time: every value
+// of every field of the chunk is read before the one barrier, then all are
+// written.  The op's kind and operand elements are decoded once, outside the
+// loops over fields and components, so that all of an op's loads are in
+// flight together (branches per component made each component's loads wait
+// for the previous ones).
+template <int NV0, int NV1, int NV2, int K0, int K1, int K2>
+__device__ inline void fill_chunk_nv(const FillProgram& P, const FillSet& set, int NT, int w, int lane, bool valid) {
+  FillOp op{};
+  op.op = kFillNop;
+  int q = 0;
+  if (valid) {
+    q = find_segment(P, w);
+    op = P.ops[q][(w - P.cprefix[q]) * kFillChunk + lane];
+  }
+  const bool live = op.op != kFillNop;
+  const int N2 = NT * NT;
+  double v0[NV0 > 0 ? NV0 : 1], v1[NV1 > 0 ? NV1 : 1], v2[NV2 > 0 ? NV2 : 1];
+  if (live) {
+    int64_t e[4];
+    if (op.op == kFillCopy) {
+      e[0] = src_ref(op.src, op.src_cell);
+      if constexpr (NV0 > 0) fill_gather<NV0, K0, true>(set.base[0], N2, e, v0);
+      if constexpr (NV1 > 0) fill_gather<NV1, K1, true>(set.base[1], N2, e, v1);
+      if constexpr (NV2 > 0) fill_gather<NV2, K2, true>(set.base[2], N2, e, v2);
+    } else {
+      if (op.op == kFillRestrict) {
+        const int a = op.src_cell;
+        e[0] = src_ref(op.src, a);
+        e[1] = src_ref(op.src, a + NT);
+        e[2] = src_ref(op.src, a + 1);
+        e[3] = src_ref(op.src, a + 1 + NT);
+      } else {
+        const FillGen& g = P.gen[q][op.src];
+#pragma unroll
+        for (int t = 0; t < 4; t++) e[t] = g.ref[t];
+      }
+      if constexpr (NV0 > 0) fill_gather<NV0, K0, false>(set.base[0], N2, e, v0);
+      if constexpr (NV1 > 0) fill_gather<NV1, K1, false>(set.base[1], N2, e, v1);
+      if constexpr (NV2 > 0) fill_gather<NV2, K2, false>(set.base[2], N2, e, v2);
+    }
+  }
+  __syncthreads();  // every read of the chunk precedes every write
+  if (live) {
+#pragma unroll
+    for (int k = 0; k < NV0; k++) set.base[0][((size_t)op.dst_gs * NV0 + k) * N2 + op.dst_cell] = v0[k];
+#pragma unroll
+    for (int k = 0; k < NV1; k++) set.base[1][((size_t)op.dst_gs * NV1 + k) * N2 + op.dst_cell] = v1[k];
+#pragma unroll
+    for (int k = 0; k < NV2; k++) set.base[2][((size_t)op.dst_gs * NV2 + k) * N2 + op.dst_cell] = v2[k];
+  }
+}
+
+// field sets of the step (engine.cpp) with their combine kinds: {U, Bi},
+// {Bi, ff, gg}, {ff, gg}, one cell field, one face field, EMF; any other set
+// takes the per-field path
+template <int NV0, int NV1, int NV2, int K0, int K1, int K2>
+__global__ __launch_bounds__(kThreads) void fill_kernel_nv(FillProgram P, FillSet set, int NT,
+                                                           const int32_t* __restrict__ counts) {
+  for (int i = blockIdx.x * kThreads + threadIdx.x; i < set.copy_words; i += gridDim.x * kThreads)
+    set.copy_dst[i] = set.copy_src[i];
+  if (counts && (int)blockIdx.x >= counts[kCountChunks]) return;
+  fill_chunk_nv<NV0, NV1, NV2, K0, K1, K2>(P, set, NT, blockIdx.x, threadIdx.x, true);
+}
+
+// ------------------------------------------------------ CFL and criteria
+// main.cpp:209-230 (per-leaf wave-speed bound, with the reference's
+// |rho|+c_fx and |u|+c_fy terms) fused with criteria.cpp:6-44 (maximum of
+// the max4diff/|w| ratio over p, rho, Bx, By on the interior).  One leaf, all
+// TPB lanes (a power of two); sW: 8 NT^2 doubles and sRed: 2 TPB doubles of
+// the workgroup's LDS.  The maxima never hold a NaN (std_max keeps its first
+// operand against one), so the reduction order does not change them.
+template <int NT, int NG, int TPB>
+__device__ inline void cfl_block(const FieldPtrs& F, const double* __restrict__ Win, const LeafItem L, int leaf,
+                                 const InstParams* __restrict__ ip, double* lam_grad, DevError* err, double* sW,
+                                 double* sRed) {
+  constexpr int N2 = NT * NT;
+  constexpr int LO = NG, HI = NT - 1 - NG;
+  const double g = ip[L.inst].gamma;
+  const int tid = threadIdx.x;
+  if (Win) {
+    const double* W = Win + (size_t)leaf * 8 * N2;
+    for (int q = tid; q < 8 * N2; q += TPB) sW[q] = W[q];
+  } else {
+    const double* U = F.f[kU] + (size_t)L.gs * 8 * N2;
+    for (int c = tid; c < N2; c += TPB) {
+      double u[8], w[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) u[k] = U[k * N2 + c];
+      cons_to_prim(u, g, w);
+#pragma unroll
+      for (int k = 0; k < 8; k++) sW[k * N2 + c] = w[k];
+      const int i = c % NT, j = c / NT;
+      if (w[4] <= 0 && i > LO - 1 && i < HI + 1 && j > LO - 1 && j < HI + 1)
+        report(err, L.inst, error_key(kOrdCfl, L.nb, 0, i, j, 0, L.nb, kErrPressure));
+    }
+  }
+  __syncthreads();
+  double lam = 0., grad = 0.;
+  constexpr int NI = HI - LO + 1;
+  for (int q = tid; q < NI * NI; q += TPB) {
+    const int i = LO + q % NI, j = LO + q / NI, c = j * NT + i;
+    double w[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) w[k] = sW[k * N2 + c];
+    if (!Win) {
+      lam = std_max(lam, fabs(w[0]) + fast_speed(w, g, 5));
+      lam = std_max(lam, fabs(w[1]) + fast_speed(w, g, 6));
+    }
+    const int vars[4] = {4, 0, 5, 6};
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const double* Wk = sW + vars[v] * N2;
+      const double x = Wk[c];
+      double m = fabs(Wk[c + 1] - x);
+      m = mac_max(m, fabs(Wk[c - 1] - x));
+      m = mac_max(m, fabs(Wk[c + NT] - x));
+      m = mac_max(m, fabs(Wk[c - NT] - x));
+      grad = std_max(grad, m / mac_max(kEps, fabs(x)));
+    }
+  }
+  sRed[tid] = lam;
+  sRed[TPB + tid] = grad;
+  __syncthreads();
+  for (int w = TPB / 2; w > 0; w >>= 1) {
+    if (tid < w) {
+      sRed[tid] = std_max(sRed[tid], sRed[tid + w]);
+      sRed[TPB + tid] = std_max(sRed[TPB + tid], sRed[TPB + tid + w]);
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    const double dxl = ip[L.inst].dx[L.lev];
+    lam_grad[2 * leaf] = std_min(dxl, dxl) / sRed[0];
+    lam_grad[2 * leaf + 1] = sRed[TPB];
+  }
+}
+
+template <int NT, int NG>
+__global__ __launch_bounds__(kThreads) void cfl_criteria_kernel(FieldPtrs F, const double* __restrict__ Win,
+                                                                const LeafItem* __restrict__ leaves,
+                                                                const InstParams* __restrict__ ip, double* lam_grad,
+                                                                DevError* err, const int32_t* __restrict__ counts) {
+  __shared__ double sW[8 * NT * NT];
+  __shared__ double sRed[2 * kThreads];
+  if (counts && (int)blockIdx.x >= counts[kCountLeaves]) return;
+  cfl_block<NT, NG, kThreads>(F, Win, leaves[blockIdx.x], blockIdx.x, ip, lam_grad, err, sW, sRed);
+}
+
+}  // namespace
+
+}  // namespace amr

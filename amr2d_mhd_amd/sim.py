@@ -224,20 +224,19 @@ class Simulation:
         _check(self.h, lib().amr_set_fill_cache(self.h, int(entries)))
 
     def set_stage_variant(self, variant):
-        """Select the stage-kernel variant (0 to STAGE_VARIANTS - 1, identical results; -1 = tuned per
-        leaf-count bucket)."""
+        """Select the stage-kernel variant (0 to STAGE_VARIANTS - 1, identical results; -1 = chosen by
+        the number of leaf blocks)."""
         _check(self.h, lib().amr_set_stage_variant(self.h, int(variant)))
 
     def stage_tuning(self, nbuckets=24):
-        """Tuner decisions: {bucket: (chosen variant, [mean us per leaf of each variant])}."""
+        """Variants in use: {leaf-count bucket: (variant, [zeros])}."""
         chosen = np.zeros(nbuckets, np.int32)
         us = np.zeros((nbuckets, STAGE_VARIANTS))
         _check(self.h, lib().amr_stage_tuning(self.h, nbuckets, chosen.ctypes.data, us.ctypes.data))
         return {b: (int(chosen[b]), us[b].tolist()) for b in range(nbuckets) if chosen[b] >= 0 or us[b].any()}
 
     def set_stage_tuning(self, chosen):
-        """Import tuner decisions {bucket: variant} (as stage_tuning() returns
-        them, or plain ints): those buckets run no trial launches."""
+        """Import variants {bucket: variant} (as stage_tuning() returns them, or plain ints)."""
         arr = np.full(24, -1, np.int32)
         for b, v in chosen.items():
             arr[int(b)] = v[0] if isinstance(v, (tuple, list)) else int(v)

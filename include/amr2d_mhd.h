@@ -201,7 +201,7 @@ int amr_set_graph(amr_ctx *ctx, int on);
  * separated by grid-wide barriers -- instead of one launch per phase.  Same
  * results bit for bit.  mode 1: 256 lanes per workgroup, 2: 512 lanes,
  * 0 and -1 (the default): per-phase launches (graph replay and the
- * stage-kernel tuner apply to these only) -- on MI355X a grid-wide barrier
+ * stage-kernel variants apply to these only) -- on MI355X a grid-wide barrier
  * over the 8 XCDs costs more than the kernel boundary it replaces, so per-phase
  * launches are faster for these workloads.  The step kernel runs only where
  * the device keeps its whole grid resident (else per-phase launches); a
@@ -224,30 +224,25 @@ int amr_set_step_kernel(amr_ctx *ctx, int mode);
 int amr_set_regrid_device(amr_ctx *ctx, int on);
 
 /* Stage-kernel variant (no counterpart in the reference; all variants give
- * identical results): lanes per leaf block and where the face fluxes live
- * for the RK update -- 0: 256 lanes, fluxes in LDS; 1: 512 lanes, LDS;
- * 2: 768 lanes, LDS; 3: 256 lanes, fluxes read back from ff/gg, 4 waves per
- * SIMD; 4: 512 lanes, read back, 4 waves per SIMD; 5: 512 lanes, LDS, 4 waves
- * per SIMD; 6: each leaf split into 2 row strips, one workgroup per strip;
- * 7: 4 row strips (a stage that reads and writes the same field, SSP-RK3's
- * second, runs as variant 2 instead, and the tuner does not try strips with
- * RK3).  Each variant exists generic (solver and limiter read per
- * instance), specialised to HLLD with a MUSCL-family limiter, and, for
- * nghosts 4, specialised to HLLD with WENO5; launches use a specialisation
- * when every running instance has its pair.  -1 (the default)
- * tunes per specialisation and leaf-count bucket (bucket b holds
- * 2^b <= nleaf < 2^(b+1)): the first stage launches in a bucket try the
- * variants in turn, three times each, timed by the kernel's device-clock
- * span, and the one with the smallest median time per leaf block is kept. */
+ * identical results).  Three kernels serve the variant numbers: 1, 2, 5 a
+ * wide workgroup per leaf block with the face fluxes in LDS, 0, 3, 4 a narrow
+ * one that reads them back from ff/gg, 6, 7 four row strips per leaf block, one
+ * workgroup each (a stage that reads and writes the same field, SSP-RK3's
+ * second, runs as the wide kernel instead).  Each exists generic (solver and
+ * limiter read per instance), specialised to HLLD or HLLC with a MUSCL-family
+ * limiter, and, for nghosts 4, specialised to HLLD with WENO5; launches use a
+ * specialisation when every running instance has its pair.  -1 (the default)
+ * chooses by the number of leaf blocks: strips below 128, wide below 512,
+ * narrow from there. */
 int amr_set_stage_variant(amr_ctx *ctx, int variant);
-/* Tuner state of the specialisation in use: chosen[b] (-1 = not decided) and
- * the mean measured microseconds per leaf block of each variant,
- * us_per_leaf[b][6]. */
+/* Variants in use, per leaf-count bucket (bucket b holds 2^b <= nleaf <
+ * 2^(b+1)) of the specialisation in use: chosen[b] is the imported variant,
+ * or the default's where stages have run in the bucket, or -1.  us_per_leaf[b][8]
+ * is filled with zeros (no launch is timed for the choice). */
 int amr_stage_tuning(amr_ctx *ctx, int nbuckets, int32_t *chosen, double *us_per_leaf);
-/* Import tuner decisions (e.g. from an earlier run of the same workload):
- * chosen[b] >= 0 fixes bucket b's variant for the specialisation the
- * context's running instances select, so later launches in it run no trials;
- * -1 leaves a bucket as it is. */
+/* Import variants: chosen[b] >= 0 fixes bucket b's variant for the
+ * specialisation the context's running instances select; -1 leaves a bucket
+ * as it is. */
 int amr_set_stage_tuning(amr_ctx *ctx, int nbuckets, const int32_t *chosen);
 
 /* Fill-program cache (no counterpart in the reference): after a tree change

@@ -1,0 +1,108 @@
+"""The stage arithmetic over the whole exponent range.
+
+The device forms quotients with shared reciprocals and unscaled square roots
+where the face's or tile's values lie in a checked range of exponents, and
+with the full sequences elsewhere: values on both sides of every limit, exact
+zeros of both signs, infinities and NaN must give the oracle's bits."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# around the limits 2^60 (faces), 2^-800 (numerators, tiles), 2^-860 (momenta), and the underflow threshold
+EXPONENTS = [0, 30, 59, 60, 61, 100, 101, 300, 480, 799, 800, 801, 859, 861, 968, 1000, 1021, 1060]
+
+
+def _same_bits(a, b):
+    return (a.view(np.int64) == b.view(np.int64)) | (np.isnan(a) & np.isnan(b))
+
+
+@pytest.mark.parametrize("method", ["RUSA", "HLLE", "HLLC", "HLLD"])
+@pytest.mark.parametrize("direction", ["x", "y"])
+def test_riemann_batch_exponents(method, direction):
+    torch = pytest.importorskip("torch")
+    import amr2d_mhd_amd as A
+
+    rng = np.random.default_rng(77 + len(method) + (direction == "y"))
+    n = 512
+    L, R = [], []
+    for e in EXPONENTS:
+        w = np.zeros((2, n, 8))
+        w[:, :, 0] = rng.uniform(0.1, 3.0, (2, n))
+        w[:, :, 4] = rng.uniform(0.05, 3.0, (2, n))
+        w[:, :, 1:4] = rng.normal(0, 1, (2, n, 3))
+        w[:, :, 5:8] = rng.normal(0, 1, (2, n, 3))
+        # each of the six vector components of each state: kept, scaled down by 2^-e, +0 or -0
+        pick = rng.integers(0, 4, (2, n, 6))
+        v = w[:, :, [1, 2, 3, 5, 6, 7]]
+        v = np.where(pick == 1, v * 2.0 ** -e, np.where(pick == 2, 0.0, np.where(pick == 3, -0.0, v)))
+        w[:, :, [1, 2, 3, 5, 6, 7]] = v
+        w[1, : n // 4] = w[0, : n // 4]  # equal states: numerators cancel
+        if e < 300:  # density or pressure on either side of the range
+            k = slice(n // 2, n // 2 + 32)
+            w[:, k, 0] *= 2.0 ** -e
+            k = slice(n // 2 + 32, n // 2 + 64)
+            w[:, k, 4] *= 2.0 ** -e
+            k = slice(n // 2 + 64, n // 2 + 96)
+            w[:, k, 0] *= 2.0 ** e
+            w[:, k, 4] *= 2.0 ** e
+            k = slice(n // 2 + 96, n // 2 + 128)
+            w[0, k, 1:4] *= 2.0 ** e
+        w[0, -1, 4] = -1.0
+        w[0, -2, 2] = np.nan
+        w[0, -3, 6] = np.inf
+        L.append(w[0])
+        R.append(w[1])
+    wL, wR = np.concatenate(L), np.concatenate(R)
+    with np.errstate(all="ignore"):
+        fo, so = O.riemann(method, direction, 1.4, wL, wR)
+    fg, sg = A.riemann_batch(method, direction, 1.4, torch.from_numpy(wL).cuda(), torch.from_numpy(wR).cuda())
+    fg, sg = fg.cpu().numpy(), sg.cpu().numpy()
+    assert np.array_equal(so != 0, sg != 0)
+    ok = so == 0
+    same = _same_bits(fg[ok], fo[ok])
+    assert same.all(), f"{method} {direction}: {int((~same).sum())} flux components differ"
+
+
+@pytest.mark.parametrize("lim,ng", [("1st", 2), ("noSL", 2), ("minmod", 2), ("VanLeer", 2), ("Superbee", 2),
+                                    ("MC", 2), ("Koren", 2), ("Cada3rd", 2), ("WENO3", 2), ("WENO5", 4)])
+@pytest.mark.parametrize("variant", [2, 3, 7])
+@pytest.mark.parametrize("planar", [True, False])
+def test_stage_exponents(lim, ng, variant, planar):
+    """Stage 1 of four blocks whose velocities and fields span the range, each
+    stage kernel, with and without z components, against the oracle's stage."""
+    import amr2d_mhd_amd as A
+
+    cfg = dict(ic="rotor", limiter=lim, flux="HLLD", cfl=0.4, nx=16, nghosts=ng, maxlevs=1)
+    sim, dom = A.Simulation(cfg), O.Domain(**cfg)
+    sim.init()
+    assert dom.init() == 0
+    sim.set_stage_variant(variant)
+    rng = np.random.default_rng(5)
+    NT = 16 + 2 * ng
+    for lo in (60, 805, 1020):  # inside the tiles' range, across its end, into underflow
+        U = np.zeros((4, 8, NT, NT))
+        e = rng.integers(0, lo, (4, 6, NT, NT)).astype(np.float64)
+        U[:, 0] = rng.uniform(0.5, 2, (4, NT, NT))
+        U[:, 4] = rng.uniform(5, 9, (4, NT, NT))
+        vec = rng.normal(0, 0.3, (4, 6, NT, NT)) * np.exp2(-e) * (rng.random((4, 6, NT, NT)) < 0.8)
+        if planar:
+            vec[:, [2, 5]] = 0.0
+        U[:, [1, 2, 3, 5, 6, 7]] = vec
+        U[3, 1:4], U[3, 5:8] = 0.0, 0.0  # a block at rest
+        Bi = np.ascontiguousarray(U[:, 5:7])
+        sim.upload("U", U)
+        sim.upload("Bi", Bi)
+        dom.set_field(O.U, U)
+        dom.set_field(O.BI, Bi)
+        sim.set_time(0.0, 1e-3, 1e-3, 1)
+        dom.set_time(0.0, 1e-3, 1e-3, 1)
+        sim.stage(1)
+        assert dom.stage(1) == 0
+        for f, of in (("Us", O.US), ("ff", O.FF), ("gg", O.GG)):
+            a, b = sim.download(f, nslots=4), dom.get_field(of, 4)
+            same = _same_bits(np.ascontiguousarray(a), np.ascontiguousarray(b))
+            assert same.all(), f"{lim} below 2^-{lo}: {f} differs in {int((~same).sum())} values"
+    sim.close()

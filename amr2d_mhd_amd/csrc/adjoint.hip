@@ -24,6 +24,7 @@
 #include "../../include/amr2d_mhd.h"
 #include "abi_guard.hpp"
 #include "adjoint_math.hpp"
+#include "stage.hpp"
 
 using namespace amr;
 
@@ -42,13 +43,145 @@ struct Grid {
 };
 
 // -------------------------------------------------------------- forward
-__global__ __launch_bounds__(kT) void k_prim(Grid G, const double* __restrict__ U, double* __restrict__ W) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  double u[8], w[8];
-  for (int k = 0; k < 8; k++) u[k] = U[k * G.n2 + c];
-  prim_of(u, G.g, w);
-  for (int k = 0; k < 8; k++) W[k * G.n2 + c] = w[k];
+// A stage is two launches.  k_fwd_faces: primitives and face fluxes of a tile
+// of T x T cells, whose lower x and y faces it owns -- the primitives of the
+// tile and of the three more columns and rows its faces read go through LDS,
+// with the AMR stage's reconstruction, solver and range flags (stage.hpp).
+// k_fwd_update: everything that follows the fluxes, a lane a cell: the stage
+// update, the four corner EMFs around the cell, its two faces and the far ones
+// its field averages read (formed twice rather than stored and read back), and
+// the cell sync.  (Primitives, fluxes, update, EMF, faces and sync as a launch
+// each took 70 us a stage at 512 x 512, HLLD, and six launch gaps.)
+// T = 8 (128 lanes, the x faces on the first wavefront, the y faces on the
+// second) up to kSmallN cells a side, where 16 x 16 tiles leave CUs idle;
+// T = 16 (256 lanes, x then y faces) beyond.
+template <int T, int SOLVER>
+__global__ __launch_bounds__(T == 16 ? 256 : 128) __attribute__((amdgpu_waves_per_eu(3))) void k_fwd_faces(
+    Grid G, const double* __restrict__ Q, const double* __restrict__ Bx, const double* __restrict__ By,
+    double* __restrict__ W, double* __restrict__ Fx, double* __restrict__ Fy) {
+  constexpr int P = T + 3, VS = P * P, TPB = T == 16 ? 256 : 128;
+  __shared__ double sW[8 * VS];
+  __shared__ int sFlags;
+  const int tid = threadIdx.x, i0 = blockIdx.x * T, j0 = blockIdx.y * T;
+  if (tid == 0) sFlags = 0;
+  __syncthreads();
+  for (int c = tid; c < VS; c += TPB) {
+    const int ti = c % P, tj = c / P;  // cell (i0 + ti - 2, j0 + tj - 2)
+    const bool ci = ti >= 2 && ti < 2 + T, cj = tj >= 2 && tj < 2 + T;
+    if (!ci && !cj) continue;  // no face reads the corners
+    const size_t e = (size_t)wrap_any(j0 + tj - 2, G.n) * G.n + wrap_any(i0 + ti - 2, G.n);
+    double u[8], w[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) u[k] = Q[k * G.n2 + e];
+    const int tile = tile_prim(u, G.g, w);
+    if (tile) atomicOr(&sFlags, tile);
+#pragma unroll
+    for (int k = 0; k < 8; k++) sW[k * VS + c] = w[k];
+    if (ci && cj && i0 + ti - 2 < G.n && j0 + tj - 2 < G.n) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) W[k * G.n2 + e] = w[k];
+    }
+  }
+  __syncthreads();
+  const int tile = sFlags;
+  for (int q = tid; q < 2 * T * T; q += TPB) {
+    const int dir = q >= T * T, r = q - dir * T * T;
+    const int ci = r % T, cj = r / T;
+    if (i0 + ci >= G.n || j0 + cj >= G.n) continue;
+    const size_t f = (size_t)(j0 + cj) * G.n + i0 + ci;
+    const double* Wl = sW + (cj + 2 - dir) * P + ci + 1 + dir;  // the cell below the face
+    double fl[8];
+    tile_face_flux<kStageHLLDMuscl>(Wl, VS, dir ? P : 1, kLimMinmod, SOLVER, G.g, 1., dir ? By[f] : Bx[f], tile, dir,
+                                    fl);
+    double* F = dir ? Fy : Fx;
+#pragma unroll
+    for (int k = 0; k < 8; k++) F[k * G.n2 + f] = fl[k];
+  }
+}
+
+constexpr int kUx = 64, kUy = 4;  // cells of one workgroup of the per-cell kernels
+
+struct FwdFaces {
+  const double *B0x, *B0y;  // the step's input faces
+  const double *Bsx, *Bsy;  // the first stage's (stage 2)
+  double *Bnx, *Bny;        // the stage's faces
+  double *Bcx, *Bcy;        // a copy of them, or null
+};
+
+// STAGE 1: out = U - dt res, Bn = B0 - dt r; 2: out = 0.5 (U + Us - dt res),
+// Bn = 0.5 (Bs + B0 - dt r).  pre: the cell B before the sync.
+template <int STAGE>
+__global__ __launch_bounds__(kUx* kUy) void k_fwd_update(Grid G, const double* __restrict__ U,
+                                                         const double* __restrict__ Us, const double* __restrict__ Fx,
+                                                         const double* __restrict__ Fy, FwdFaces B, double dt,
+                                                         double* __restrict__ out, double* __restrict__ pre) {
+  const int i = blockIdx.x * kUx + threadIdx.x % kUx, j = blockIdx.y * kUy + threadIdx.x / kUx;
+  if (i >= G.n || j >= G.n) return;
+  const int n = G.n, ip = wrap(i + 1, n), im = wrap(i - 1, n), jp = wrap(j + 1, n), jm = wrap(j - 1, n);
+  const size_t n2 = G.n2, c = (size_t)j * n + i, cx = (size_t)j * n + ip, cy = (size_t)jp * n + i;
+  double dF[8], dG[8], u[8], us[8], res[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const size_t o = k * n2;
+    u[k] = U[o + c];
+    if (STAGE == 2) us[k] = Us[o + c];
+    dF[k] = Fx[o + cx] - Fx[o + c];
+    dG[k] = Fy[o + cy] - Fy[o + c];
+  }
+  // corner EMF at (i, j), (i + 1, j), (i, j + 1), (i + 1, j + 1)
+  const double* gy5 = Fy + 5 * n2;
+  const double* fx6 = Fx + 6 * n2;
+  auto emf = [&](int a, int am, int b, int bm) {
+    return 0.25 * ((gy5[(size_t)b * n + am] + gy5[(size_t)b * n + a]) - (fx6[(size_t)bm * n + a] + fx6[(size_t)b * n + a]));
+  };
+  const double E00 = emf(i, im, j, jm), E10 = emf(ip, i, j, jm), E01 = emf(i, im, jp, j), E11 = emf(ip, i, jp, j);
+  const double rdx = 1. / G.dx;
+  auto face = [&](const double* B0, const double* Bs, size_t f, double r) {
+    return STAGE == 1 ? B0[f] - dt * r : 0.5 * (Bs[f] + B0[f] - dt * r);
+  };
+  const double bx = face(B.B0x, B.Bsx, c, rdx * (E01 - E00)), bxp = face(B.B0x, B.Bsx, cx, rdx * (E11 - E10));
+  const double by = face(B.B0y, B.Bsy, c, -rdx * (E10 - E00)), byp = face(B.B0y, B.Bsy, cy, -rdx * (E11 - E01));
+  stage_residual(dF, dG, G.dx, res);
+  double q[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) q[k] = STAGE == 1 ? u[k] - dt * res[k] : 0.5 * (u[k] + us[k] - dt * res[k]);
+  const double mx = 0.5 * (bxp + bx), my = 0.5 * (byp + by);
+  pre[c] = q[5];
+  pre[n2 + c] = q[6];
+  q[4] = q[4] + 0.5 * ((mx * mx + my * my) - ((q[5] * q[5]) + (q[6] * q[6])));
+  q[5] = mx;
+  q[6] = my;
+#pragma unroll
+  for (int k = 0; k < 8; k++) out[k * n2 + c] = q[k];
+  B.Bnx[c] = bx;
+  B.Bny[c] = by;
+  if (STAGE == 2 && B.Bcx) {
+    B.Bcx[c] = bx;
+    B.Bcy[c] = by;
+  }
+}
+
+// -------------------------------------------------------------- adjoint
+// Tape of one step (doubles, N2 = N*N each unless stated): the primitive
+// states the two flux passes read (W1 = prim(U), W2 = prim(Us), 8 N2 each),
+// the stage-1 faces (Bxs, Bys), the pre-sync cell B of both stages (2 N2
+// each) and the output faces (Bxo, Byo).
+struct Tape {
+  double *W1, *W2, *Bxs, *Bys, *pre1, *pre2, *Bxo, *Byo;
+};
+constexpr size_t kTapePerCell = 24;
+
+Tape tape_at(double* base, size_t n2) {
+  Tape t;
+  t.W1 = base;
+  t.W2 = base + 8 * n2;
+  t.Bxs = base + 16 * n2;
+  t.Bys = base + 17 * n2;
+  t.pre1 = base + 18 * n2;
+  t.pre2 = base + 20 * n2;
+  t.Bxo = base + 22 * n2;
+  t.Byo = base + 23 * n2;
+  return t;
 }
 
 // edge states of one face: x faces (dir 0) take Bx as the normal component,
@@ -76,209 +209,104 @@ __device__ inline void face_states(const Grid& G, const double* W, const double*
   }
 }
 
-template <int SOLVER>
-__global__ __launch_bounds__(kT) void k_flux(Grid G, const double* __restrict__ W, const double* __restrict__ Bx,
-                                             const double* __restrict__ By, double* __restrict__ Fx,
-                                             double* __restrict__ Fy) {
-  const size_t f = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (f >= G.n2) return;
-  const int dir = blockIdx.y;
-  const int i = (int)(f % G.n), j = (int)(f / G.n);
-  double wl[8], wr[8], fl[8];
-  size_t cell[4];
-  face_states(G, W, dir ? By : Bx, dir, i, j, wl, wr, cell);
-  if (SOLVER == kFluxHLLD) {
-    for (int k = 0; k < 8; k++) fl[k] = 0.;
-    flux_hlld(wl, wr, G.g, fl);
+// Reverse of a stage, two launches: k_rev_faces takes the adjoint Q of the
+// synced state and of the faces back through the cell sync and the face update
+// to the corner EMF (adjoint Eb) and the earlier faces; the face reverse
+// (k_stage_vjp, or k_flux_vjp and k_gather_prim_vjp) forms the flux adjoints it
+// needs from Q and Eb as it goes and passes Q on to the stage's inputs.  (The
+// sync, the faces, the EMF and the flux adjoints as launches of their own, with
+// 16 flux adjoints a cell written and read back, took 37 us a stage at
+// 512 x 512.)
+//
+// Cell sync: E += 0.5 ((bx^2 + by^2) - (q5^2 + q6^2)), q5 <- bx, q6 <- by, so the
+// averages' adjoints are bb = (Q5 + Q4 bx, Q6 + Q4 by) and the pre-sync state's
+// are Q but -Q4 pre in components 5 and 6.  Faces: the updated faces' adjoint
+// Bb = Bin + 0.5 (bb of both adjacent cells); stage 2 (Bn = 0.5 (Bs + B0 - dt r))
+// assigns B0b = Bsb = 0.5 Bb, stage 1 (Bn = B0 - dt r) adds Bb to B0b.  EMF:
+// rx_b = -s dt Bbx, ry_b = -s dt Bby (s = 1 or 0.5), rx = (1/dx) (E[j+1] - E[j]),
+// ry = -(1/dx) (E[i+1] - E[i]).  Face values a corner needs beside the cell's own
+// are formed again from the inputs, which no lane writes.
+template <int STAGE>
+__global__ __launch_bounds__(kUx* kUy) void k_rev_faces(Grid G, const double* __restrict__ Q,
+                                                        const double* __restrict__ Bx, const double* __restrict__ By,
+                                                        const double* __restrict__ Binx,
+                                                        const double* __restrict__ Biny, double dt,
+                                                        double* __restrict__ B0bx, double* __restrict__ B0by,
+                                                        double* __restrict__ Bsbx, double* __restrict__ Bsby,
+                                                        double* __restrict__ Eb) {
+  const int i = blockIdx.x * kUx + threadIdx.x % kUx, j = blockIdx.y * kUy + threadIdx.x / kUx;
+  if (i >= G.n || j >= G.n) return;
+  const int n = G.n, ip = wrap(i + 1, n), im = wrap(i - 1, n), jp = wrap(j + 1, n), jm = wrap(j - 1, n);
+  const size_t n2 = G.n2;
+  auto at = [n](int a, int b) { return (size_t)b * n + a; };
+  auto bbx = [&](int a, int ap, int b) {  // adjoint of the x average of cell (a, b)
+    const size_t c = at(a, b);
+    return Q[5 * n2 + c] + Q[4 * n2 + c] * (0.5 * (Bx[at(ap, b)] + Bx[c]));
+  };
+  auto bby = [&](int a, int b, int bp) {
+    const size_t c = at(a, b);
+    return Q[6 * n2 + c] + Q[4 * n2 + c] * (0.5 * (By[at(a, bp)] + By[c]));
+  };
+  const size_t c = at(i, j);
+  const double x = Binx[c] + 0.5 * (bbx(i, ip, j) + bbx(im, i, j));
+  const double y = Biny[c] + 0.5 * (bby(i, j, jp) + bby(i, jm, j));
+  const double x_jm = Binx[at(i, jm)] + 0.5 * (bbx(i, ip, jm) + bbx(im, i, jm));
+  const double y_im = Biny[at(im, j)] + 0.5 * (bby(im, j, jp) + bby(im, jm, j));
+  if (STAGE == 2) {
+    B0bx[c] = 0.5 * x;
+    B0by[c] = 0.5 * y;
+    Bsbx[c] = 0.5 * x;
+    Bsby[c] = 0.5 * y;
   } else {
-    flux_hlle(wl, wr, G.g, fl);
+    B0bx[c] += x;
+    B0by[c] += y;
   }
-  if (dir) swap_xy(fl);
-  double* F = dir ? Fy : Fx;
-  for (int k = 0; k < 8; k++) F[k * G.n2 + f] = fl[k];
-}
-
-// stage update: mode 1 out = U - dt res; mode 2 out = 0.5 (U + Us - dt res)
-__global__ __launch_bounds__(kT) void k_update(Grid G, const double* __restrict__ U, const double* __restrict__ Us,
-                                               const double* __restrict__ Fx, const double* __restrict__ Fy,
-                                               double dt, int mode, double* __restrict__ out) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  const int i = (int)(c % G.n), j = (int)(c / G.n);
-  const size_t cx = (size_t)j * G.n + wrap(i + 1, G.n), cy = (size_t)wrap(j + 1, G.n) * G.n + i;
-  for (int k = 0; k < 8; k++) {
-    const size_t o = k * G.n2;
-    const double res = (Fx[o + cx] - Fx[o + c]) / G.dx + (Fy[o + cy] - Fy[o + c]) / G.dx;
-    out[o + c] = mode == 1 ? U[o + c] - dt * res : 0.5 * (U[o + c] + Us[o + c] - dt * res);
-  }
-}
-
-__global__ __launch_bounds__(kT) void k_emf(Grid G, const double* __restrict__ Fx, const double* __restrict__ Fy,
-                                            double* __restrict__ E) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  const int i = (int)(c % G.n), j = (int)(c / G.n);
-  const double* gy5 = Fy + 5 * G.n2;
-  const double* fx6 = Fx + 6 * G.n2;
-  E[c] = 0.25 * ((gy5[(size_t)j * G.n + wrap(i - 1, G.n)] + gy5[c]) - (fx6[(size_t)wrap(j - 1, G.n) * G.n + i] + fx6[c]));
-}
-
-// face update: mode 1 Bn = B0 - dt r; mode 2 Bn = 0.5 (Bs + B0 - dt r); the
-// result also goes to (Bcx, Bcy) when given
-__global__ __launch_bounds__(kT) void k_faces(Grid G, const double* __restrict__ B0x, const double* __restrict__ B0y,
-                                              const double* __restrict__ Bsx, const double* __restrict__ Bsy,
-                                              const double* __restrict__ E, double dt, int mode,
-                                              double* __restrict__ Bnx, double* __restrict__ Bny,
-                                              double* __restrict__ Bcx, double* __restrict__ Bcy) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  const int i = (int)(c % G.n), j = (int)(c / G.n);
-  const double rx = (1. / G.dx) * (E[(size_t)wrap(j + 1, G.n) * G.n + i] - E[c]);
-  const double ry = -(1. / G.dx) * (E[(size_t)j * G.n + wrap(i + 1, G.n)] - E[c]);
-  const double bx = mode == 1 ? B0x[c] - dt * rx : 0.5 * (Bsx[c] + B0x[c] - dt * rx);
-  const double by = mode == 1 ? B0y[c] - dt * ry : 0.5 * (Bsy[c] + B0y[c] - dt * ry);
-  Bnx[c] = bx;
-  Bny[c] = by;
-  if (Bcx) {
-    Bcx[c] = bx;
-    Bcy[c] = by;
-  }
-}
-
-// cell sync; saves the pre-sync cell B (q5, q6) when `pre` is given
-__global__ __launch_bounds__(kT) void k_bsync(Grid G, double* __restrict__ Q, const double* __restrict__ Bx,
-                                              const double* __restrict__ By, double* __restrict__ pre) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  const int i = (int)(c % G.n), j = (int)(c / G.n);
-  const double bx = 0.5 * (Bx[(size_t)j * G.n + wrap(i + 1, G.n)] + Bx[c]);
-  const double by = 0.5 * (By[(size_t)wrap(j + 1, G.n) * G.n + i] + By[c]);
-  const double q5 = Q[5 * G.n2 + c], q6 = Q[6 * G.n2 + c];
-  if (pre) {
-    pre[c] = q5;
-    pre[G.n2 + c] = q6;
-  }
-  Q[4 * G.n2 + c] = Q[4 * G.n2 + c] + 0.5 * ((bx * bx + by * by) - ((q5 * q5) + (q6 * q6)));
-  Q[5 * G.n2 + c] = bx;
-  Q[6 * G.n2 + c] = by;
-}
-
-// -------------------------------------------------------------- adjoint
-// Tape of one step (doubles, N2 = N*N each unless stated): the primitive
-// states the two flux passes read (W1 = prim(U), W2 = prim(Us), 8 N2 each),
-// the stage-1 faces (Bxs, Bys), the pre-sync cell B of both stages (2 N2
-// each) and the output faces (Bxo, Byo).
-struct Tape {
-  double *W1, *W2, *Bxs, *Bys, *pre1, *pre2, *Bxo, *Byo;
-};
-constexpr size_t kTapePerCell = 24;
-
-Tape tape_at(double* base, size_t n2) {
-  Tape t;
-  t.W1 = base;
-  t.W2 = base + 8 * n2;
-  t.Bxs = base + 16 * n2;
-  t.Bys = base + 17 * n2;
-  t.pre1 = base + 18 * n2;
-  t.pre2 = base + 20 * n2;
-  t.Bxo = base + 22 * n2;
-  t.Byo = base + 23 * n2;
-  return t;
-}
-
-// bsync reverse.  Qb (adjoint of the synced state; read from Qin, written to
-// Qout, which may alias) -> adjoint of the pre-sync state and of the cell
-// averages bx, by of the faces (bb[2][N2]); E += 0.5 ((bx^2 + by^2) - (q5^2 +
-// q6^2)), q5 <- bx, q6 <- by
-__global__ __launch_bounds__(kT) void k_bsync_vjp(Grid G, const double* Qin, double* Qout,
-                                                  const double* __restrict__ pre, const double* __restrict__ Bx,
-                                                  const double* __restrict__ By, double* __restrict__ bb) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  const int i = (int)(c % G.n), j = (int)(c / G.n);
-  const double bx = 0.5 * (Bx[(size_t)j * G.n + wrap(i + 1, G.n)] + Bx[c]);
-  const double by = 0.5 * (By[(size_t)wrap(j + 1, G.n) * G.n + i] + By[c]);
-  const double e = Qin[4 * G.n2 + c];
-  const double q5 = Qin[5 * G.n2 + c], q6 = Qin[6 * G.n2 + c];
-  bb[c] = q5 + e * bx;
-  bb[G.n2 + c] = q6 + e * by;
-  if (Qout != Qin) {
-    for (int k = 0; k < 8; k++)
-      if (k != 5 && k != 6) Qout[k * G.n2 + c] = Qin[k * G.n2 + c];
-  }
-  Qout[5 * G.n2 + c] = -e * pre[c];
-  Qout[6 * G.n2 + c] = -e * pre[G.n2 + c];
-}
-
-// face reverse of one stage fused with the cell-average reverse of the bsync
-// that follows it.  Bb = Bin + 0.5 (bb of both adjacent cells) is the adjoint
-// of the updated faces (written to Bb, which may alias Bin).  Mode 2 (Bn =
-// 0.5 (Bs + B0 - dt r)): B0b = 0.5 Bb and Bsb = 0.5 Bb are assigned; mode 1
-// (Bn = B0 - dt r): B0b += Bb.
-__global__ __launch_bounds__(kT) void k_faces_vjp(Grid G, const double* Binx, const double* Biny,
-                                                  const double* __restrict__ bb, int mode, double* Bbx, double* Bby,
-                                                  double* __restrict__ B0bx, double* __restrict__ B0by,
-                                                  double* __restrict__ Bsbx, double* __restrict__ Bsby) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  const int i = (int)(c % G.n), j = (int)(c / G.n);
-  const double bxb = Binx[c] + 0.5 * (bb[c] + bb[(size_t)j * G.n + wrap(i - 1, G.n)]);
-  const double byb = Biny[c] + 0.5 * (bb[G.n2 + c] + bb[G.n2 + (size_t)wrap(j - 1, G.n) * G.n + i]);
-  Bbx[c] = bxb;
-  Bby[c] = byb;
-  if (mode == 2) {
-    B0bx[c] = 0.5 * bxb;
-    B0by[c] = 0.5 * byb;
-    Bsbx[c] = 0.5 * bxb;
-    Bsby[c] = 0.5 * byb;
-  } else {
-    B0bx[c] += bxb;
-    B0by[c] += byb;
-  }
-}
-
-// adjoint of E at every corner from the face adjoints: rx_b = -s dt Bbx,
-// ry_b = -s dt Bby (s = 1 or 0.5), rx = (1/dx)(E[j+1] - E[j]),
-// ry = -(1/dx)(E[i+1] - E[i])
-__global__ __launch_bounds__(kT) void k_emf_b(Grid G, const double* __restrict__ Bbx, const double* __restrict__ Bby,
-                                              double dt, int mode, double* __restrict__ Eb) {
-  const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (c >= G.n2) return;
-  const int i = (int)(c % G.n), j = (int)(c / G.n);
-  const double s = mode == 1 ? -dt : -0.5 * dt;
-  const double rxb_jm = s * Bbx[(size_t)wrap(j - 1, G.n) * G.n + i], rxb = s * Bbx[c];
-  const double ryb_im = s * Bby[(size_t)j * G.n + wrap(i - 1, G.n)], ryb = s * Bby[c];
+  const double s = STAGE == 1 ? -dt : -0.5 * dt;
+  const double rxb_jm = s * x_jm, rxb = s * x, ryb_im = s * y_im, ryb = s * y;
   Eb[c] = (1. / G.dx) * (rxb_jm - rxb) - (1. / G.dx) * (ryb_im - ryb);
 }
 
-// adjoint of the face fluxes from the stage update (residual adjoint
-// resb = -s dt Qb, s = 1 or 0.5) and from the EMF (components 6 of Fx, 5 of
-// Fy), fused with the pass-through of Qb to the stage inputs: mode 2
-// (out = 0.5 (U + Us - dt res)) assigns Ub = Usb = 0.5 Qb; mode 1 (out = U -
-// dt res) adds Qb to Ub
-__global__ __launch_bounds__(kT) void k_flux_b(Grid G, const double* __restrict__ Qb, const double* __restrict__ Eb,
-                                               double dt, int mode, double* __restrict__ Fbx,
-                                               double* __restrict__ Fby, double* __restrict__ Ub,
-                                               double* __restrict__ Usb) {
-  const size_t f = (size_t)blockIdx.x * kT + threadIdx.x;
-  if (f >= G.n2) return;
-  const int i = (int)(f % G.n), j = (int)(f / G.n);
-  const double s = mode == 1 ? -dt : -0.5 * dt;
-  const size_t lx = (size_t)j * G.n + wrap(i - 1, G.n), ly = (size_t)wrap(j - 1, G.n) * G.n + i;
+// what the face reverse reads: the stage's synced-state adjoint, the cell B
+// before the sync, the corner EMF's adjoint, and where Q goes on to -- stage 2
+// (out = 0.5 (U + Us - dt res)) assigns Ub = 0.5 Q and Qb = 0.5 Q + ..., stage 1
+// (out = U - dt res) adds Q and the face contributions to Qb = Ub
+struct RevIn {
+  const double *Q, *pre, *Eb;
+  double s;  // residual adjoint = s Q: -dt, or -0.5 dt in stage 2
+};
+
+// pre-sync state adjoint, component k
+__device__ inline double presync(const Grid& G, const RevIn& R, int k, size_t c) {
+  return k == 5 || k == 6 ? -R.Q[4 * G.n2 + c] * R.pre[(k - 5) * G.n2 + c] : R.Q[k * G.n2 + c];
+}
+
+// adjoints of the fluxes through the lower face of cell (i, j) in direction
+// DIR: from the update's residual and from the EMF (components 6 of x, 5 of y)
+template <int DIR>
+__device__ AMR_INLINE void flux_adjoint(const Grid& G, const RevIn& R, int i, int j, double* fb) {
+  const size_t f = (size_t)j * G.n + i;
+  const size_t l = DIR == 0 ? (size_t)j * G.n + wrap(i - 1, G.n) : (size_t)wrap(j - 1, G.n) * G.n + i;
+  const RDen dx = rden(G.dx);
+#pragma unroll
+  for (int k = 0; k < 8; k++) fb[k] = quot(R.s * presync(G, R, k, l) - R.s * presync(G, R, k, f), dx);
+  if (DIR == 0) fb[6] -= 0.25 * (R.Eb[f] + R.Eb[(size_t)wrap(j + 1, G.n) * G.n + i]);
+  else fb[5] += 0.25 * (R.Eb[f] + R.Eb[(size_t)j * G.n + wrap(i + 1, G.n)]);
+}
+
+// Q on to the stage's inputs, with the face contributions ub
+template <int STAGE>
+__device__ inline void pass_state(const Grid& G, const RevIn& R, size_t c, const double* ub, double* Ub, double* Qb) {
+#pragma unroll
   for (int k = 0; k < 8; k++) {
-    const size_t o = k * G.n2;
-    const double q = Qb[o + f];
-    Fbx[o + f] = (s * Qb[o + lx] - s * q) / G.dx;
-    Fby[o + f] = (s * Qb[o + ly] - s * q) / G.dx;
-    if (mode == 2) {
-      Ub[o + f] = 0.5 * q;
-      Usb[o + f] = 0.5 * q;
+    const double q = presync(G, R, k, c);
+    const size_t e = k * G.n2 + c;
+    if (STAGE == 2) {
+      Ub[e] = 0.5 * q;
+      Qb[e] = 0.5 * q + ub[k];
     } else {
-      Ub[o + f] += q;
+      Qb[e] = (Qb[e] + q) + ub[k];
     }
   }
-  Fby[5 * G.n2 + f] += 0.25 * (Eb[f] + Eb[(size_t)j * G.n + wrap(i + 1, G.n)]);
-  Fbx[6 * G.n2 + f] -= 0.25 * (Eb[f] + Eb[(size_t)wrap(j + 1, G.n) * G.n + i]);
 }
 
 // per-face reverse of reconstruction + HLLE for the faces of one direction
@@ -289,16 +317,12 @@ __global__ __launch_bounds__(kT) void k_flux_b(Grid G, const double* __restrict_
 // cells (i-2 .. i+1 along the normal) and the normal-B adjoint
 template <int DIR, int SOLVER>
 __device__ inline void face_reverse(const Grid& G, int i, int j, const double* __restrict__ W,
-                                    const double* __restrict__ Bn, const double* __restrict__ Fb, double* wlb,
-                                    double* wrb, size_t* cell) {
-  const size_t f = (size_t)j * G.n + i;
+                                    const double* __restrict__ Bn, const RevIn& R, double* wlb, double* wrb,
+                                    size_t* cell) {
   double wl[8], wr[8], fb[8];
   face_states(G, W, Bn, DIR, i, j, wl, wr, cell);
-  for (int k = 0; k < 8; k++) {
-    fb[k] = Fb[k * G.n2 + f];
-    wlb[k] = 0.;
-    wrb[k] = 0.;
-  }
+  flux_adjoint<DIR>(G, R, i, j, fb);
+  for (int k = 0; k < 8; k++) wlb[k] = wrb[k] = 0.;
   if (DIR) swap_xy(fb);  // adjoint of the output swap
   if (SOLVER == kFluxHLLD) hlld_vjp(wl, wr, G.g, fb, wlb, wrb);
   else hlle_vjp(wl, wr, G.g, fb, wlb, wrb);
@@ -339,12 +363,12 @@ __device__ inline void stencil_reverse(const Grid& G, const double* __restrict__
 
 template <int DIR, int SOLVER>
 __device__ inline void flux_vjp_face(const Grid& G, size_t f, const double* __restrict__ W,
-                                     const double* __restrict__ Bn, const double* __restrict__ Fb,
-                                     double* __restrict__ S, double* __restrict__ Bnb) {
+                                     const double* __restrict__ Bn, const RevIn& R, double* __restrict__ S,
+                                     double* __restrict__ Bnb) {
   const int i = (int)(f % G.n), j = (int)(f / G.n);
   double wlb[8], wrb[8];
   size_t cell[4];
-  face_reverse<DIR, SOLVER>(G, i, j, W, Bn, Fb, wlb, wrb, cell);
+  face_reverse<DIR, SOLVER>(G, i, j, W, Bn, R, wlb, wrb, cell);
   constexpr int nc = DIR ? 6 : 5;
   Bnb[f] += wlb[nc] + wrb[nc];
   stencil_reverse<DIR>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
@@ -354,18 +378,18 @@ __device__ inline void flux_vjp_face(const Grid& G, size_t f, const double* __re
 
 template <int DIR, int SOLVER>
 __global__ __launch_bounds__(kT) void k_flux_vjp(Grid G, const double* __restrict__ W, const double* __restrict__ Bn,
-                                                 const double* __restrict__ Fb, double* __restrict__ S,
-                                                 double* __restrict__ Bnb) {
+                                                 RevIn R, double* __restrict__ S, double* __restrict__ Bnb) {
   const size_t f = (size_t)blockIdx.x * kT + threadIdx.x;
   if (f >= G.n2) return;
-  flux_vjp_face<DIR, SOLVER>(G, f, W, Bn, Fb, S, Bnb);
+  flux_vjp_face<DIR, SOLVER>(G, f, W, Bn, R, S, Bnb);
 }
 
 // per-cell sum of the stencil contributions, then the cons->prim reverse
 // from the tape's primitive state: Qb += (dW/dQ)^T Wb
+template <int STAGE>
 __global__ __launch_bounds__(kT) void k_gather_prim_vjp(Grid G, const double* __restrict__ W,
                                                         const double* __restrict__ Sx, const double* __restrict__ Sy,
-                                                        double* __restrict__ Qb) {
+                                                        RevIn R, double* __restrict__ Ub, double* __restrict__ Qb) {
   const size_t c = (size_t)blockIdx.x * kT + threadIdx.x;
   if (c >= G.n2) return;
   const int i = (int)(c % G.n), j = (int)(c / G.n);
@@ -383,7 +407,7 @@ __global__ __launch_bounds__(kT) void k_gather_prim_vjp(Grid G, const double* __
     ub[k] = 0.;
   }
   prim_vjp_w(w, G.g, wb, ub);
-  for (int k = 0; k < 8; k++) Qb[k * G.n2 + c] += ub[k];
+  pass_state<STAGE>(G, R, c, ub, Ub, Qb);
 }
 
 // Fused face reverse + stencil sum + cons->prim reverse over a tile of
@@ -395,12 +419,11 @@ __global__ __launch_bounds__(kT) void k_gather_prim_vjp(Grid G, const double* __
 // tiles that read them; the normal-B adjoint of a face is added only by the
 // tile that owns the face.  Deterministic: fixed summation order, no
 // atomics.
-template <int TW, int TH, int TT, int SOLVER>
+template <int TW, int TH, int TT, int SOLVER, int STAGE>
 __global__ __launch_bounds__(TT) void k_stage_vjp(Grid G, const double* __restrict__ W,
-                                                  const double* __restrict__ Bx, const double* __restrict__ By,
-                                                  const double* __restrict__ Fbx, const double* __restrict__ Fby,
+                                                  const double* __restrict__ Bx, const double* __restrict__ By, RevIn R,
                                                   double* __restrict__ Bnbx, double* __restrict__ Bnby,
-                                                  double* __restrict__ Qb) {
+                                                  double* __restrict__ Ub, double* __restrict__ Qb) {
   static_assert(TH * (TW + 3) <= TT && (TH + 3) * TW <= TT, "one face per lane and direction");
   __shared__ double S[8][4][TT];  // [variable][stencil position][face of the tile]
   // x-face sums of the tile's cells, kept in LDS across the y-face reverse
@@ -419,7 +442,7 @@ __global__ __launch_bounds__(TT) void k_stage_vjp(Grid G, const double* __restri
     if (fj < G.n) {
       double wlb[8], wrb[8];
       size_t cell[4];
-      face_reverse<0, SOLVER>(G, fi, fj, W, Bx, Fbx, wlb, wrb, cell);
+      face_reverse<0, SOLVER>(G, fi, fj, W, Bx, R, wlb, wrb, cell);
       if (q >= 1 && q <= TW && i0 - 1 + q < G.n) Bnbx[(size_t)fj * G.n + fi] += wlb[5] + wrb[5];
       stencil_reverse<0>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
         for (int s = 0; s < 4; s++) S[k][s][tid] = vb[s];
@@ -443,7 +466,7 @@ __global__ __launch_bounds__(TT) void k_stage_vjp(Grid G, const double* __restri
     if (fi < G.n) {
       double wlb[8], wrb[8];
       size_t cell[4];
-      face_reverse<1, SOLVER>(G, fi, fj, W, By, Fby, wlb, wrb, cell);
+      face_reverse<1, SOLVER>(G, fi, fj, W, By, R, wlb, wrb, cell);
       if (r >= 1 && r <= TH && j0 - 1 + r < G.n) Bnby[(size_t)fj * G.n + fi] += wlb[6] + wrb[6];
       stencil_reverse<1>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
         for (int s = 0; s < 4; s++) S[k][s][tid] = vb[s];
@@ -462,15 +485,15 @@ __global__ __launch_bounds__(TT) void k_stage_vjp(Grid G, const double* __restri
       ub[k] = 0.;
     }
     prim_vjp_w(w, G.g, wb, ub);
-    for (int k = 0; k < 8; k++) Qb[k * G.n2 + c] += ub[k];
+    pass_state<STAGE>(G, R, c, ub, Ub, Qb);
   }
 }
 
-template <int TW, int TH, int TT, int SOLVER>
-void launch_stage_vjp(const Grid& G, const double* W, const double* Bx, const double* By, const double* Fbx,
-                      const double* Fby, double* Bnbx, double* Bnby, double* Qb, hipStream_t s) {
+template <int TW, int TH, int TT, int SOLVER, int STAGE>
+void launch_stage_vjp(const Grid& G, const double* W, const double* Bx, const double* By, const RevIn& R, double* Bnbx,
+                      double* Bnby, double* Ub, double* Qb, hipStream_t s) {
   const dim3 grid((unsigned)((G.n + TW - 1) / TW), (unsigned)((G.n + TH - 1) / TH));
-  k_stage_vjp<TW, TH, TT, SOLVER><<<grid, TT, 0, s>>>(G, W, Bx, By, Fbx, Fby, Bnbx, Bnby, Qb);
+  k_stage_vjp<TW, TH, TT, SOLVER, STAGE><<<grid, TT, 0, s>>>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb);
 }
 
 unsigned blocks(size_t n) { return (unsigned)((n + kT - 1) / kT); }
@@ -483,9 +506,9 @@ struct amr_adj {
   int fused = 1;  // face reverse + gather in one tiled kernel: 1 16x13 tiles of 256 lanes, 2 32x13 tiles of
                   // 512 lanes; 0: per-face kernels and a gather
   // forward scratch
-  double *Fx, *Fy, *E, *Us, *Uo, *Bxo, *Byo, *tape;
+  double *Fx, *Fy, *Us, *Uo, *Bxo, *Byo, *tape;
   // adjoint work
-  double *Qb2, *Usb, *Fbx, *Fby, *Eb, *Bsbx, *Bsby, *Bbx, *Bby, *bb, *Sx, *Sy;
+  double *Usb, *Eb, *Bsbx, *Bsby, *Sx, *Sy;
 };
 
 namespace {
@@ -500,89 +523,95 @@ namespace {
     }                                                                                          \
   } while (0)
 
-void launch_flux(amr_adj* a, const double* W, const double* Bx, const double* By, hipStream_t s) {
-  const dim3 b2(blocks(a->G.n2), 2);
-  if (a->solver == kFluxHLLD) k_flux<kFluxHLLD><<<b2, kT, 0, s>>>(a->G, W, Bx, By, a->Fx, a->Fy);
-  else k_flux<kFluxHLLE><<<b2, kT, 0, s>>>(a->G, W, Bx, By, a->Fx, a->Fy);
+constexpr int kSmallN = 256;  // 8 x 8 tiles up to this many cells a side (k_fwd_faces)
+
+template <int SOLVER>
+void launch_faces(amr_adj* a, const double* Q, const double* Bx, const double* By, double* W, hipStream_t s) {
+  const unsigned n = (unsigned)a->G.n;
+  if (a->G.n <= kSmallN) {
+    const dim3 grid((n + 7) / 8, (n + 7) / 8);
+    k_fwd_faces<8, SOLVER><<<grid, 128, 0, s>>>(a->G, Q, Bx, By, W, a->Fx, a->Fy);
+  } else {
+    const dim3 grid((n + 15) / 16, (n + 15) / 16);
+    k_fwd_faces<16, SOLVER><<<grid, 256, 0, s>>>(a->G, Q, Bx, By, W, a->Fx, a->Fy);
+  }
 }
 
+dim3 cell_grid(const Grid& G) { return dim3((unsigned)((G.n + kUx - 1) / kUx), (unsigned)((G.n + kUy - 1) / kUy)); }
+
 // forward stage sequence, writing the step's tape
-int forward(amr_adj* a, const double* U, const double* Bx, const double* By, double dt, double* Uo, double* Bxo,
-            double* Byo, const Tape& T, hipStream_t s) {
+template <int SOLVER>
+int forward_of(amr_adj* a, const double* U, const double* Bx, const double* By, double dt, double* Uo, double* Bxo,
+               double* Byo, const Tape& T, hipStream_t s) {
   const Grid& G = a->G;
-  const unsigned b1 = blocks(G.n2);
-  k_prim<<<b1, kT, 0, s>>>(G, U, T.W1);
-  launch_flux(a, T.W1, Bx, By, s);
-  k_update<<<b1, kT, 0, s>>>(G, U, nullptr, a->Fx, a->Fy, dt, 1, a->Us);
-  k_emf<<<b1, kT, 0, s>>>(G, a->Fx, a->Fy, a->E);
-  k_faces<<<b1, kT, 0, s>>>(G, Bx, By, nullptr, nullptr, a->E, dt, 1, T.Bxs, T.Bys, nullptr, nullptr);
-  k_bsync<<<b1, kT, 0, s>>>(G, a->Us, T.Bxs, T.Bys, T.pre1);
-  k_prim<<<b1, kT, 0, s>>>(G, a->Us, T.W2);
-  launch_flux(a, T.W2, T.Bxs, T.Bys, s);
-  k_update<<<b1, kT, 0, s>>>(G, U, a->Us, a->Fx, a->Fy, dt, 2, Uo);
-  k_emf<<<b1, kT, 0, s>>>(G, a->Fx, a->Fy, a->E);
-  k_faces<<<b1, kT, 0, s>>>(G, Bx, By, T.Bxs, T.Bys, a->E, dt, 2, Bxo, Byo, T.Bxo, T.Byo);
-  k_bsync<<<b1, kT, 0, s>>>(G, Uo, Bxo, Byo, T.pre2);
+  const dim3 cells = cell_grid(G);
+  launch_faces<SOLVER>(a, U, Bx, By, T.W1, s);
+  k_fwd_update<1><<<cells, kUx * kUy, 0, s>>>(G, U, nullptr, a->Fx, a->Fy,
+                                              FwdFaces{Bx, By, nullptr, nullptr, T.Bxs, T.Bys, nullptr, nullptr}, dt,
+                                              a->Us, T.pre1);
+  launch_faces<SOLVER>(a, a->Us, T.Bxs, T.Bys, T.W2, s);
+  k_fwd_update<2><<<cells, kUx * kUy, 0, s>>>(G, U, a->Us, a->Fx, a->Fy,
+                                              FwdFaces{Bx, By, T.Bxs, T.Bys, Bxo, Byo, T.Bxo, T.Byo}, dt, Uo, T.pre2);
   ADJ_CHK(hipGetLastError());
   return 0;
 }
 
-// face reverse of one stage from its flux adjoints (a->Fbx, a->Fby): normal-B
-// adjoints into Bnb*, cell adjoints added to Qb
-void face_and_gather(amr_adj* a, const double* W, const double* Bx, const double* By, double* Bnbx, double* Bnby,
-                     double* Qb, hipStream_t s) {
+int forward(amr_adj* a, const double* U, const double* Bx, const double* By, double dt, double* Uo, double* Bxo,
+            double* Byo, const Tape& T, hipStream_t s) {
+  return a->solver == kFluxHLLD ? forward_of<kFluxHLLD>(a, U, Bx, By, dt, Uo, Bxo, Byo, T, s)
+                                : forward_of<kFluxHLLE>(a, U, Bx, By, dt, Uo, Bxo, Byo, T, s);
+}
+
+// face reverse of one stage: normal-B adjoints into Bnb*, cell adjoints to
+// Ub (stage 2) and Qb
+template <int SOLVER, int STAGE>
+void face_and_gather(amr_adj* a, const double* W, const double* Bx, const double* By, const RevIn& R, double* Bnbx,
+                     double* Bnby, double* Ub, double* Qb, hipStream_t s) {
   const Grid& G = a->G;
-  const bool hlld = a->solver == kFluxHLLD;
   if (a->fused == 1) {
-    if (hlld) launch_stage_vjp<16, 13, 256, kFluxHLLD>(G, W, Bx, By, a->Fbx, a->Fby, Bnbx, Bnby, Qb, s);
-    else launch_stage_vjp<16, 13, 256, kFluxHLLE>(G, W, Bx, By, a->Fbx, a->Fby, Bnbx, Bnby, Qb, s);
+    launch_stage_vjp<16, 13, 256, SOLVER, STAGE>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb, s);
   } else if (a->fused == 2) {
-    if (hlld) launch_stage_vjp<32, 13, 512, kFluxHLLD>(G, W, Bx, By, a->Fbx, a->Fby, Bnbx, Bnby, Qb, s);
-    else launch_stage_vjp<32, 13, 512, kFluxHLLE>(G, W, Bx, By, a->Fbx, a->Fby, Bnbx, Bnby, Qb, s);
+    launch_stage_vjp<32, 13, 512, SOLVER, STAGE>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb, s);
   } else {
     const unsigned b1 = blocks(G.n2);
-    if (hlld) {
-      k_flux_vjp<0, kFluxHLLD><<<b1, kT, 0, s>>>(G, W, Bx, a->Fbx, a->Sx, Bnbx);
-      k_flux_vjp<1, kFluxHLLD><<<b1, kT, 0, s>>>(G, W, By, a->Fby, a->Sy, Bnby);
-    } else {
-      k_flux_vjp<0, kFluxHLLE><<<b1, kT, 0, s>>>(G, W, Bx, a->Fbx, a->Sx, Bnbx);
-      k_flux_vjp<1, kFluxHLLE><<<b1, kT, 0, s>>>(G, W, By, a->Fby, a->Sy, Bnby);
-    }
-    k_gather_prim_vjp<<<b1, kT, 0, s>>>(G, W, a->Sx, a->Sy, Qb);
+    k_flux_vjp<0, SOLVER><<<b1, kT, 0, s>>>(G, W, Bx, R, a->Sx, Bnbx);
+    k_flux_vjp<1, SOLVER><<<b1, kT, 0, s>>>(G, W, By, R, a->Sy, Bnby);
+    k_gather_prim_vjp<STAGE><<<b1, kT, 0, s>>>(G, W, a->Sx, a->Sy, R, Ub, Qb);
   }
 }
 
 // reverse sweep of one step from its tape and input faces
-int reverse(amr_adj* a, const Tape& T, const double* Bx, const double* By, double dt, const double* Uob,
-            const double* Bxob, const double* Byob, double* Ub, double* Bxb, double* Byb, hipStream_t s) {
+template <int SOLVER>
+int reverse_of(amr_adj* a, const Tape& T, const double* Bx, const double* By, double dt, const double* Uob,
+               const double* Bxob, const double* Byob, double* Ub, double* Bxb, double* Byb, hipStream_t s) {
   const Grid& G = a->G;
-  const unsigned b1 = blocks(G.n2);
-  // ---- stage 2
-  k_bsync_vjp<<<b1, kT, 0, s>>>(G, Uob, a->Qb2, T.pre2, T.Bxo, T.Byo, a->bb);
-  k_faces_vjp<<<b1, kT, 0, s>>>(G, Bxob, Byob, a->bb, 2, a->Bbx, a->Bby, Bxb, Byb, a->Bsbx, a->Bsby);
-  k_emf_b<<<b1, kT, 0, s>>>(G, a->Bbx, a->Bby, dt, 2, a->Eb);
-  k_flux_b<<<b1, kT, 0, s>>>(G, a->Qb2, a->Eb, dt, 2, a->Fbx, a->Fby, Ub, a->Usb);
-  face_and_gather(a, T.W2, T.Bxs, T.Bys, a->Bsbx, a->Bsby, a->Usb, s);
-  // ---- stage 1
-  k_bsync_vjp<<<b1, kT, 0, s>>>(G, a->Usb, a->Usb, T.pre1, T.Bxs, T.Bys, a->bb);
-  k_faces_vjp<<<b1, kT, 0, s>>>(G, a->Bsbx, a->Bsby, a->bb, 1, a->Bsbx, a->Bsby, Bxb, Byb, nullptr, nullptr);
-  k_emf_b<<<b1, kT, 0, s>>>(G, a->Bsbx, a->Bsby, dt, 1, a->Eb);
-  k_flux_b<<<b1, kT, 0, s>>>(G, a->Usb, a->Eb, dt, 1, a->Fbx, a->Fby, Ub, nullptr);
-  face_and_gather(a, T.W1, Bx, By, Bxb, Byb, Ub, s);
+  const dim3 cells = cell_grid(G);
+  k_rev_faces<2><<<cells, kUx * kUy, 0, s>>>(G, Uob, T.Bxo, T.Byo, Bxob, Byob, dt, Bxb, Byb, a->Bsbx, a->Bsby, a->Eb);
+  face_and_gather<SOLVER, 2>(a, T.W2, T.Bxs, T.Bys, RevIn{Uob, T.pre2, a->Eb, -0.5 * dt}, a->Bsbx, a->Bsby, Ub,
+                             a->Usb, s);
+  k_rev_faces<1><<<cells, kUx * kUy, 0, s>>>(G, a->Usb, T.Bxs, T.Bys, a->Bsbx, a->Bsby, dt, Bxb, Byb, nullptr, nullptr,
+                                             a->Eb);
+  face_and_gather<SOLVER, 1>(a, T.W1, Bx, By, RevIn{a->Usb, T.pre1, a->Eb, -dt}, Bxb, Byb, nullptr, Ub, s);
   ADJ_CHK(hipGetLastError());
   return 0;
 }
 
+int reverse(amr_adj* a, const Tape& T, const double* Bx, const double* By, double dt, const double* Uob,
+            const double* Bxob, const double* Byob, double* Ub, double* Bxb, double* Byb, hipStream_t s) {
+  return a->solver == kFluxHLLD ? reverse_of<kFluxHLLD>(a, T, Bx, By, dt, Uob, Bxob, Byob, Ub, Bxb, Byb, s)
+                                : reverse_of<kFluxHLLE>(a, T, Bx, By, dt, Uob, Bxob, Byob, Ub, Bxb, Byb, s);
+}
+
 // ------------------------------------------------- allocation-free step
-// Work memory of amr_adj_step_noalloc: the forward's face fluxes, corner EMF,
-// stage state and tape (8 + 8 + 1 + 8 + kTapePerCell doubles per cell) for
+// Work memory of amr_adj_step_noalloc: the forward's face fluxes,
+// stage state and tape (8 + 8 + 8 + kTapePerCell doubles per cell) for
 // grids of up to kNoAllocMaxN^2 cells, in one file-scope device array that
-// every GPU the library runs on holds until the process ends (25.7 MB).  Host
+// every GPU the library runs on holds until the process ends (25.2 MB).  Host
 // code never passes the array's name to a kernel (a host-side stand-in):
 // each device's address comes from hipGetSymbolAddress, taken once per
 // device on its first call, and only that address is used.
 constexpr int kNoAllocMaxN = 256;
-constexpr size_t kNoAllocPerCell = 8 + 8 + 1 + 8 + kTapePerCell;
+constexpr size_t kNoAllocPerCell = 8 + 8 + 8 + kTapePerCell;
 static __device__ __align__(256) double scratch[kNoAllocPerCell * kNoAllocMaxN * kNoAllocMaxN];
 
 constexpr int kMaxDevices = 64;
@@ -630,9 +659,8 @@ int amr_adj_step_noalloc(int n, double dx, double gamma, const char* flux, const
   const size_t n2 = a.G.n2;
   a.Fx = w;
   a.Fy = w + 8 * n2;
-  a.E = w + 16 * n2;
-  a.Us = w + 17 * n2;
-  a.tape = w + 25 * n2;
+  a.Us = w + 16 * n2;
+  a.tape = w + 24 * n2;
   return forward(&a, U, Bx, By, dt, Uo, Bxo, Byo, tape_at(a.tape, n2), (hipStream_t)stream);
   AMR_CATCH
 }
@@ -647,13 +675,12 @@ int amr_adj_create(int n, double dx, double gamma, const char* flux, amr_adj** o
   a->solver = solver;
   a->G = Grid{n, dx, gamma, (size_t)n * n};
   const size_t n2 = a->G.n2;
-  double** bufs8[] = {&a->Fx, &a->Fy, &a->Us, &a->Uo, &a->Qb2, &a->Usb, &a->Fbx, &a->Fby};
-  double** bufs1[] = {&a->E, &a->Bxo, &a->Byo, &a->Eb, &a->Bsbx, &a->Bsby, &a->Bbx, &a->Bby};
+  double** bufs8[] = {&a->Fx, &a->Fy, &a->Us, &a->Uo, &a->Usb};
+  double** bufs1[] = {&a->Bxo, &a->Byo, &a->Eb, &a->Bsbx, &a->Bsby};
   bool ok = true;
   for (auto p : bufs8) ok = ok && hipMalloc((void**)p, 8 * n2 * sizeof(double)) == hipSuccess;
   for (auto p : bufs1) ok = ok && hipMalloc((void**)p, n2 * sizeof(double)) == hipSuccess;
   ok = ok && hipMalloc((void**)&a->tape, kTapePerCell * n2 * sizeof(double)) == hipSuccess;
-  ok = ok && hipMalloc((void**)&a->bb, 2 * n2 * sizeof(double)) == hipSuccess;
   ok = ok && hipMalloc((void**)&a->Sx, 32 * n2 * sizeof(double)) == hipSuccess;
   ok = ok && hipMalloc((void**)&a->Sy, 32 * n2 * sizeof(double)) == hipSuccess;
   if (!ok) {
@@ -668,8 +695,8 @@ int amr_adj_create(int n, double dx, double gamma, const char* flux, amr_adj** o
 int amr_adj_destroy(amr_adj* a) {
   AMR_TRY
   if (!a) return AMR_OK;
-  double* all[] = {a->Fx,  a->Fy,  a->E,    a->Us,   a->Uo,  a->Bxo, a->Byo, a->tape, a->Qb2, a->Usb,
-                   a->Fbx, a->Fby, a->Eb,   a->Bsbx, a->Bsby, a->Bbx, a->Bby, a->bb,   a->Sx,  a->Sy};
+  double* all[] = {a->Fx,   a->Fy,   a->Us, a->Uo, a->Bxo, a->Byo, a->tape, a->Usb, a->Eb,
+                   a->Bsbx, a->Bsby, a->Sx, a->Sy};
   for (double* p : all)
     if (p) hipFree(p);
   delete a;

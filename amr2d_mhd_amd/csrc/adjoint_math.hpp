@@ -7,26 +7,38 @@
 // computed expression chain, including the branch taken at every min/max and
 // the 1e-15 guards, so the result is the exact derivative of the discrete
 // map away from branch switches.
+//
+// Quotients take the FAST forms of physics.hpp on the device (one refined
+// reciprocal a denominator): a reverse has several quotients by each of its
+// denominators, and the values it meets that lie outside the forms' range are
+// numerators below 1e-291, whose quotients are then right to an absolute
+// 1e-290.
 #pragma once
 #include "physics.hpp"
 
 namespace amr {
 
+using RDen = Den<true>;
+__host__ __device__ AMR_INLINE RDen rden(double d) { return den<true>(d); }
+__host__ __device__ AMR_INLINE double rdiv(double n, double d) { return quot(n, den<true>(d)); }
+__host__ __device__ AMR_INLINE double rroot(double x) { return root<true>(x); }
+
 // Hides x from the optimizer, so that values recomputed from it are not
 // merged with identical ones computed earlier and kept live in the
 // meantime (a register-pressure device; no effect in the host build).
-__host__ __device__ inline void opaque(double& x) {
+__host__ __device__ AMR_INLINE void opaque(double& x) {
 #ifdef __HIP_DEVICE_COMPILE__
   asm volatile("" : "+v"(x));
 #endif
 }
 
 // ------------------------------------------------------------ cons -> prim
-__host__ __device__ inline void prim_of(const double* u, double g, double* w) {
+__host__ __device__ AMR_INLINE void prim_of(const double* u, double g, double* w) {
   w[0] = u[0];
-  w[1] = u[1] / u[0];
-  w[2] = u[2] / u[0];
-  w[3] = u[3] / u[0];
+  const RDen r = rden(u[0]);
+  w[1] = quot(u[1], r);
+  w[2] = quot(u[2], r);
+  w[3] = quot(u[3], r);
   const double p = (g - 1) * (u[4] - 0.5 * w[0] * (w[1] * w[1] + w[2] * w[2] + w[3] * w[3]));
   w[5] = u[5];
   w[6] = u[6];
@@ -36,8 +48,8 @@ __host__ __device__ inline void prim_of(const double* u, double g, double* w) {
 
 // ub += (dw/du)^T wb, from the primitive state w = prim_of(u) (u0 = w0 and
 // u5..7 = w5..7; w1..3 = u1..3 / u0)
-__host__ __device__ inline void prim_vjp_w(const double* w, double g, const double* wb, double* ub) {
-  const double iw0 = 1. / w[0];
+__host__ __device__ AMR_INLINE void prim_vjp_w(const double* w, double g, const double* wb, double* ub) {
+  const double iw0 = rdiv(1., w[0]);
   const double pb = wb[4];
   const double sv = w[1] * w[1] + w[2] * w[2] + w[3] * w[3];
   double w0b = wb[0] + pb * (-(g - 1) * 0.5 * sv);
@@ -53,7 +65,7 @@ __host__ __device__ inline void prim_vjp_w(const double* w, double g, const doub
   for (int k = 5; k <= 7; k++) ub[k] += wb[k] - pb * (g - 1) * w[k];
 }
 
-__host__ __device__ inline void prim_vjp(const double* u, double g, const double* wb, double* ub) {
+__host__ __device__ AMR_INLINE void prim_vjp(const double* u, double g, const double* wb, double* ub) {
   double w[8];
   prim_of(u, g, w);
   prim_vjp_w(w, g, wb, ub);
@@ -62,27 +74,28 @@ __host__ __device__ inline void prim_vjp(const double* u, double g, const double
 // -------------------------------------------------- minmod MUSCL, one face
 // Edge states of the face between cells c (left) and c+1 of a 4-cell
 // stencil v = (c-1, c, c+1, c+2): muscl_plus/muscl_minus with minmod.
-__host__ __device__ inline void recon_minmod(const double* v, double& wl, double& wr) {
+__host__ __device__ AMR_INLINE void recon_minmod(const double* v, double& wl, double& wr) {
   const double a = v[1] - v[0], b = v[2] - v[1], d = v[3] - v[2];
-  wl = muscl_plus(kLimMinmod, v[1], a, b, 1.);
-  wr = muscl_minus(kLimMinmod, v[2], b, d, 1.);
+  wl = muscl_plus<true>(kLimMinmod, v[1], a, b, 1.);
+  wr = muscl_minus<true>(kLimMinmod, v[2], b, d, 1.);
 }
 
 // derivative of max(0, min(1, r)) (mac_max(0, mac_min(1, r))) along the
 // branch the forward takes: the value is r itself iff !(1 < r) and !(0 > r)
-__host__ __device__ inline bool minmod_slope(double r) { return !(1. < r) && !(0. > r); }
+__host__ __device__ AMR_INLINE bool minmod_slope(double r) { return !(1. < r) && !(0. > r); }
 
 // vb[0..3] += d(wl, wr)/dv ^T (wlb, wrb).  wl = v1 + 0.5 phi(rl) a with
 // rl = b / (a + eps): where phi = rl, d wl/da = 0.5 rl eps / (a + eps) and
 // d wl/db = 0.5 a / (a + eps); elsewhere phi is 0 or 1 and d wl/da = 0.5 phi.
 // wr = v2 - 0.5 phi(rr) d with rr = b / (d + eps) likewise.  rl and rr are
 // the forward's own quotients, so the branch is the one the forward took.
-__host__ __device__ inline void recon_minmod_vjp(const double* v, double wlb, double wrb, double* vb) {
+__host__ __device__ AMR_INLINE void recon_minmod_vjp(const double* v, double wlb, double wrb, double* vb) {
   const double a = v[1] - v[0], b = v[2] - v[1], d = v[3] - v[2];
-  const double rl = b / (a + kEps), rr = b / (d + kEps);
+  const RDen da = rden(a + kEps), dd = rden(d + kEps);
+  const double rl = quot(b, da), rr = quot(b, dd);
   double ab, bb, db;
   if (minmod_slope(rl)) {
-    const double il = 1. / (a + kEps);
+    const double il = quot(1., da);
     ab = 0.5 * wlb * rl * kEps * il;
     bb = 0.5 * wlb * a * il;
   } else {
@@ -90,7 +103,7 @@ __host__ __device__ inline void recon_minmod_vjp(const double* v, double wlb, do
     bb = 0.;
   }
   if (minmod_slope(rr)) {
-    const double ir = 1. / (d + kEps);
+    const double ir = quot(1., dd);
     db = -0.5 * wrb * rr * kEps * ir;
     bb -= 0.5 * wrb * d * ir;
   } else {
@@ -114,27 +127,28 @@ struct FastT {
   double ca2, a2, can2, s1, sq, cf;
 };
 
-__host__ __device__ inline double fast_fwd(const double* w, double g, FastT& t) {
-  const double ca = sqrt((w[5] * w[5] + w[6] * w[6] + w[7] * w[7]) / w[0]);
-  const double a = sqrt(g * w[4] / w[0]);
-  const double can = sqrt((w[5] * w[5]) / w[0]);
+__host__ __device__ AMR_INLINE double fast_fwd(const double* w, double g, FastT& t) {
+  const RDen r = rden(w[0]);
+  const double ca = rroot(quot(w[5] * w[5] + w[6] * w[6] + w[7] * w[7], r));
+  const double a = rroot(quot(g * w[4], r));
+  const double can = rroot(quot(w[5] * w[5], r));
   t.ca2 = ca * ca;
   t.a2 = a * a;
   t.can2 = can * can;
   const double s0 = t.ca2 + t.a2;
   t.s1 = t.ca2 - t.a2;
-  t.sq = sqrt(t.s1 * t.s1 + 4. * t.a2 * (t.ca2 - t.can2));
-  t.cf = sqrt(0.5 * (s0 + t.sq));
+  t.sq = rroot(t.s1 * t.s1 + 4. * t.a2 * (t.ca2 - t.can2));
+  t.cf = rroot(0.5 * (s0 + t.sq));
   return t.cf;
 }
 
 // cfb -> wb; each of ca^2, a^2, can^2 is sqrt(q)^2 of a quotient q over w0,
 // with derivative 1 in q wherever the root is positive
-__host__ __device__ inline void fast_bwd(const double* w, double g, const FastT& t, double iw0, double cfb,
+__host__ __device__ AMR_INLINE void fast_bwd(const double* w, double g, const FastT& t, double iw0, double cfb,
                                          double* wb) {
-  const double tb = cfb * 0.5 / t.cf;
+  const double tb = rdiv(cfb * 0.5, t.cf);
   const double s0b = 0.5 * tb, sqb = 0.5 * tb;
-  const double innerb = t.sq > 0. ? sqb * 0.5 / t.sq : 0.;
+  const double innerb = t.sq > 0. ? rdiv(sqb * 0.5, t.sq) : 0.;
   const double s1b = innerb * 2. * t.s1;
   const double a2b = innerb * 4. * (t.ca2 - t.can2) + s0b - s1b;
   const double ca2b = innerb * 4. * t.a2 + s0b + s1b;
@@ -158,16 +172,17 @@ __host__ __device__ inline void fast_bwd(const double* w, double g, const FastT&
 
 // the fast speed, energy density and enthalpy of one side (side_state's
 // cf, e and H)
-__host__ __device__ inline void side_fwd(const double* w, double g, FastT& f, double& e, double& H) {
+__host__ __device__ AMR_INLINE void side_fwd(const double* w, double g, FastT& f, double& e, double& H) {
   fast_fwd(w, g, f);
   const double b2 = w[5] * w[5] + w[6] * w[6] + w[7] * w[7];
-  e = (w[4] / (w[0] * (g - 1))) + 0.5 * (w[1] * w[1] + w[2] * w[2] + w[3] * w[3]) + 0.5 * b2 / w[0];
+  const RDen r = rden(w[0]);
+  e = rdiv(w[4], w[0] * (g - 1)) + 0.5 * (w[1] * w[1] + w[2] * w[2] + w[3] * w[3]) + quot(0.5 * b2, r);
   e = e * w[0];
-  H = (e + w[4] + 0.5 * b2) / w[0];
+  H = quot(e + w[4] + 0.5 * b2, r);
 }
 
 // component k of side_state's conserved state q and x-flux F
-__host__ __device__ inline void side_qF(const double* w, double e, double H, int k, double& q, double& F) {
+__host__ __device__ AMR_INLINE void side_qF(const double* w, double e, double H, int k, double& q, double& F) {
   const double vn = w[1], Bn = w[5];
   const double mv = w[0] * vn;
   switch (k) {
@@ -184,9 +199,9 @@ __host__ __device__ inline void side_qF(const double* w, double e, double H, int
 
 // side reverse: the adjoints of F and q are sF Nb and sQ Nb, of H Hb and of
 // the fast speed cfb; accumulates into wb
-__host__ __device__ inline void side_bwd(const double* w, double g, double e, double H, const FastT& f,
+__host__ __device__ AMR_INLINE void side_bwd(const double* w, double g, double e, double H, const FastT& f,
                                          const double* Nb, double sF, double sQ, double Hb, double cfb, double* wb) {
-  const double iw0 = 1. / w[0];
+  const double iw0 = rdiv(1., w[0]);
   const double vn = w[1], Bn = w[5];
   const double b2 = w[5] * w[5] + w[6] * w[6] + w[7] * w[7];
   const double mv = w[0] * vn;
@@ -232,8 +247,9 @@ __host__ __device__ inline void side_bwd(const double* w, double g, double e, do
   // e = e1 w0 with e1 = w4 / (w0 (g-1)) + 0.5 |v|^2 + 0.5 b2 / w0
   const double e1b = eb * w[0];
   wb[0] += eb * (e * iw0);
-  wb[4] += e1b * iw0 / (g - 1);
-  wb[0] -= e1b * (w[4] * iw0 / (g - 1)) * iw0;
+  const RDen dg = rden(g - 1);
+  wb[4] += quot(e1b * iw0, dg);
+  wb[0] -= e1b * quot(w[4] * iw0, dg) * iw0;
   wb[1] += e1b * w[1];
   wb[2] += e1b * w[2];
   wb[3] += e1b * w[3];
@@ -250,7 +266,7 @@ __host__ __device__ inline void side_bwd(const double* w, double g, double e, do
 
 // side reverse with q and F adjoints sQ Nb and sF Nb, plus adjoints of e
 // and pt used outside q and F (HLLD star states), H and the fast speed
-__host__ __device__ inline void side_bwd_vec(const double* w, double g, double e, double H, const FastT& f,
+__host__ __device__ AMR_INLINE void side_bwd_vec(const double* w, double g, double e, double H, const FastT& f,
                                              const double* Nb, double sF, double sQ, double Hb, double eb_x,
                                              double ptb_x, double cfb, double* wb) {
   double Fb[8], qb[8];
@@ -259,7 +275,7 @@ __host__ __device__ inline void side_bwd_vec(const double* w, double g, double e
     Fb[k] = sF * Nb[k];
     qb[k] = sQ * Nb[k];
   }
-  const double iw0 = 1. / w[0];
+  const double iw0 = rdiv(1., w[0]);
   const double vn = w[1], Bn = w[5];
   const double b2 = w[5] * w[5] + w[6] * w[6] + w[7] * w[7];
   const double mv = w[0] * vn;
@@ -295,8 +311,9 @@ __host__ __device__ inline void side_bwd_vec(const double* w, double g, double e
   wb[0] -= Hb * H * iw0;
   const double e1b = eb * w[0];
   wb[0] += eb * (e * iw0);
-  wb[4] += e1b * iw0 / (g - 1);
-  wb[0] -= e1b * (w[4] * iw0 / (g - 1)) * iw0;
+  const RDen dg = rden(g - 1);
+  wb[4] += quot(e1b * iw0, dg);
+  wb[0] -= e1b * quot(w[4] * iw0, dg) * iw0;
   wb[1] += e1b * w[1];
   wb[2] += e1b * w[2];
   wb[3] += e1b * w[3];
@@ -315,50 +332,52 @@ struct RoeT {
   double sl, sr, nrm, v[3], B[3], RT, d, d6, d7, X, Y, h, btsq, cY, vax2, a2raw, a2, ct2, tdif, sq, cfast;
 };
 
-__host__ __device__ inline void roe_fwd(const double* wL, const double* wR, double g, double HL, double HR, RoeT& t,
+__host__ __device__ AMR_INLINE void roe_fwd(const double* wL, const double* wR, double g, double HL, double HR, RoeT& t,
                                         double& lmin, double& lmax) {
-  t.sl = sqrt(wL[0]);
-  t.sr = sqrt(wR[0]);
-  t.nrm = sqrt(wL[0] + t.sr);
+  t.sl = rroot(wL[0]);
+  t.sr = rroot(wR[0]);
+  t.nrm = rroot(wL[0] + t.sr);
+  const RDen dn = rden(t.nrm);
 #pragma unroll
   for (int i = 0; i < 3; i++) {
-    t.v[i] = (t.sl * wL[i + 1] + t.sr * wR[i + 1]) / t.nrm;
-    t.B[i] = (t.sl * wL[i + 5] + t.sr * wR[i + 5]) / t.nrm;
+    t.v[i] = quot(t.sl * wL[i + 1] + t.sr * wR[i + 1], dn);
+    t.B[i] = quot(t.sl * wL[i + 5] + t.sr * wR[i + 5], dn);
   }
-  t.RT = sqrt(wR[0] / wL[0]);
-  t.d = sqrt(wR[0] * wL[0]);
+  t.RT = rroot(rdiv(wR[0], wL[0]));
+  t.d = rroot(wR[0] * wL[0]);
+  const RDen dd = rden(t.d);
   t.d6 = wL[6] - wR[6];
   t.d7 = wL[7] - wR[7];
-  t.X = 0.5 * ((t.d6 * t.d6) + (t.d7 * t.d7)) / (t.sl + t.sr);
-  t.Y = 0.5 * (wL[0] + wR[0]) / t.d;
-  t.h = (HL + t.RT * HR) / (1 + t.RT);
+  t.X = rdiv(0.5 * ((t.d6 * t.d6) + (t.d7 * t.d7)), t.sl + t.sr);
+  t.Y = quot(0.5 * (wL[0] + wR[0]), dd);
+  t.h = rdiv(HL + t.RT * HR, 1 + t.RT);
   const double vsq = t.v[0] * t.v[0] + t.v[1] * t.v[1] + t.v[2] * t.v[2];
   t.btsq = (t.B[1] * t.B[1]) + (t.B[2] * t.B[2]);
   t.cY = (g - 1. - (g - 2) * t.Y);
   const double bt2s = t.cY * t.btsq;
-  t.vax2 = (t.B[0] * t.B[0]) / t.d;
-  const double hp = t.h - (t.vax2 + t.btsq / t.d);
+  t.vax2 = quot(t.B[0] * t.B[0], dd);
+  const double hp = t.h - (t.vax2 + quot(t.btsq, dd));
   t.a2raw = ((g - 1.) * (hp - 0.5 * vsq) - (g - 2.) * t.X);
   t.a2 = mac_max(t.a2raw, kEps);
-  t.ct2 = bt2s / t.d;
+  t.ct2 = quot(bt2s, dd);
   const double tsum = t.vax2 + t.ct2 + t.a2;
   t.tdif = t.vax2 + t.ct2 - t.a2;
-  t.sq = sqrt(t.tdif * t.tdif + 4. * t.a2 * t.ct2);
-  t.cfast = sqrt(0.5 * (tsum + t.sq));
+  t.sq = rroot(t.tdif * t.tdif + 4. * t.a2 * t.ct2);
+  t.cfast = rroot(0.5 * (tsum + t.sq));
   lmin = t.v[0] - t.cfast;
   lmax = t.v[0] + t.cfast;
 }
 
 // (lminb, lmaxb) -> wL, wR, HL, HR adjoints (accumulated)
-__host__ __device__ inline void roe_bwd(const double* wL, const double* wR, double g, double HR, const RoeT& t,
+__host__ __device__ AMR_INLINE void roe_bwd(const double* wL, const double* wR, double g, double HR, const RoeT& t,
                                         double lminb, double lmaxb, double* wLb, double* wRb, double& HLb,
                                         double& HRb) {
-  const double id = 1. / t.d, inrm = 1. / t.nrm;
+  const double id = rdiv(1., t.d), inrm = rdiv(1., t.nrm);
   double vb[3] = {lminb + lmaxb, 0., 0.}, Bb[3] = {0., 0., 0.};
   const double cfb = lmaxb - lminb;
-  const double tb = cfb * 0.5 / t.cfast;
+  const double tb = rdiv(cfb * 0.5, t.cfast);
   const double tsumb = 0.5 * tb, sqb = 0.5 * tb;
-  const double inb = t.sq > 0. ? sqb * 0.5 / t.sq : 0.;
+  const double inb = t.sq > 0. ? rdiv(sqb * 0.5, t.sq) : 0.;
   const double tdifb = inb * 2. * t.tdif;
   const double a2b = inb * 4. * t.ct2 + tsumb - tdifb;
   const double ct2b = inb * 4. * t.a2 + tsumb + tdifb;
@@ -387,7 +406,7 @@ __host__ __device__ inline void roe_bwd(const double* wL, const double* wR, doub
 #pragma unroll
   for (int i = 0; i < 3; i++) vb[i] += vsqb * 2. * t.v[i];
   // h = (HL + RT HR) / (1 + RT)
-  const double i1 = 1. / (1 + t.RT);
+  const double i1 = rdiv(1., 1 + t.RT);
   HLb += hb * i1;
   HRb += hb * t.RT * i1;
   const double RTb = (hb * HR - hb * t.h) * i1;
@@ -396,7 +415,7 @@ __host__ __device__ inline void roe_bwd(const double* wL, const double* wR, doub
   wRb[0] += Yb * 0.5 * id;
   db -= Yb * t.Y * id;
   // X = 0.5 (d6^2 + d7^2) / (sl + sr)
-  const double iss = 1. / (t.sl + t.sr);
+  const double iss = rdiv(1., t.sl + t.sr);
   const double d6b = Xb * t.d6 * iss, d7b = Xb * t.d7 * iss;
   double slb = -Xb * t.X * iss, srb = slb;
   wLb[6] += d6b;
@@ -411,8 +430,8 @@ __host__ __device__ inline void roe_bwd(const double* wL, const double* wR, doub
   }
   // RT = sqrt(rhoR / rhoL)
   if (t.RT > 0.) {
-    const double qb = RTb * 0.5 / t.RT;
-    const double iL = 1. / wL[0];
+    const double qb = rdiv(RTb * 0.5, t.RT);
+    const double iL = rdiv(1., wL[0]);
     wRb[0] += qb * iL;
     wLb[0] -= qb * (wR[0] * iL) * iL;
   }
@@ -430,12 +449,12 @@ __host__ __device__ inline void roe_bwd(const double* wL, const double* wR, doub
   }
   // nrm = sqrt(rhoL + sr), sl = sqrt(rhoL), sr = sqrt(rhoR)
   const double inner_b = nrmb * 0.5 * inrm;
-  wLb[0] += inner_b + slb * 0.5 / t.sl;
-  wRb[0] += (inner_b + srb) * 0.5 / t.sr;
+  wLb[0] += inner_b + rdiv(slb * 0.5, t.sl);
+  wRb[0] += rdiv((inner_b + srb) * 0.5, t.sr);
 }
 
 // HLLE flux (flux_hlle) reverse: fb -> wLb, wRb (accumulated)
-__host__ __device__ inline void hlle_vjp(const double* wL, const double* wR, double g, const double* fb, double* wLb,
+__host__ __device__ AMR_INLINE void hlle_vjp(const double* wL, const double* wR, double g, const double* fb, double* wLb,
                                          double* wRb) {
   FastT fL, fR;
   double eL, HL, eR, HR;
@@ -448,7 +467,7 @@ __host__ __device__ inline void hlle_vjp(const double* wL, const double* wR, dou
   const double SL = mac_min(il, 0.);
   const double xr = wR[1] + fR.cf, ir = std_max(xr, lmax);
   const double SR = mac_max(ir, 0.);
-  const double iD = 1. / (SR - SL);
+  const double iD = rdiv(1., SR - SL);
   // f_k = (SR FL_k - SL FR_k + SL SR dq_k) / D
   double SLb = 0., SRb = 0., Db = 0., Nb[8];
 #pragma unroll
@@ -488,16 +507,43 @@ __host__ __device__ inline void hlle_vjp(const double* wL, const double* wR, dou
 }
 
 // ------------------------------------------------------------- HLLD flux
+// hlld_star with the quotients above
+__host__ __device__ AMR_INLINE void hlld_star_fast(const double* w, double S, double SM, double pts, double e,
+                                                   double pt, double* ws, double& es) {
+  const RDen dS = rden(S - SM);
+  ws[0] = quot(w[0] * (S - w[1]), dS);
+  ws[1] = SM;
+  ws[4] = 0.;
+  ws[5] = w[5];
+  const double dn = w[0] * (S - w[1]) * (S - SM) - (w[5] * w[5]);
+  if (dn != 0) {
+    const RDen dd = rden(dn);
+    const double sv = quot(SM - w[1], dd);
+    ws[2] = w[2] - w[5] * w[6] * sv;
+    ws[3] = w[3] - w[5] * w[7] * sv;
+    const double sb = quot(w[0] * ((S - w[1]) * (S - w[1])) - (w[5] * w[5]), dd);
+    ws[6] = w[6] * sb;
+    ws[7] = w[7] * sb;
+  } else {
+    ws[2] = w[2];
+    ws[3] = w[3];
+    ws[6] = 0.;
+    ws[7] = 0.;
+  }
+  es = quot((S - w[1]) * e - pt * w[1] + pts * SM + w[5] * (vdotb(w) - vdotb(ws)), dS);
+}
+
 // star state (hlld_star) reverse: (wsb, esb) -> adjoints of the side's w, S,
 // SM, pts, e and pt (accumulated); ws/es are the forward's outputs
-__host__ __device__ inline void hlld_star_bwd(const double* w, double S, double SM, double pts, double e, double pt,
+__host__ __device__ AMR_INLINE void hlld_star_bwd(const double* w, double S, double SM, double pts, double e, double pt,
                                               const double* ws, double es, double* wsb, double esb, double* wb,
                                               double& Sb, double& SMb, double& ptsb, double& eb, double& ptb) {
   const double a = S - w[1], b = S - SM;
   double ab = 0., bb = 0.;
   // es = (a e - pt w1 + pts SM + w5 (vdotb(w) - vdotb(ws))) / b
-  const double Nb = esb / b;
-  bb -= esb * es / b;
+  const RDen db = rden(b);
+  const double Nb = quot(esb, db);
+  bb -= quot(esb * es, db);
   ab += Nb * e;
   eb += Nb * a;
   ptb -= Nb * w[1];
@@ -518,17 +564,18 @@ __host__ __device__ inline void hlld_star_bwd(const double* w, double S, double 
   wsb[6] += vs * ws[2];
   wsb[3] += vs * ws[7];
   wsb[7] += vs * ws[3];
-  const double den = w[0] * (S - w[1]) * (S - SM) - (w[5] * w[5]);
-  if (den != 0) {
-    const double sv = (SM - w[1]) / den;
-    const double sb = (w[0] * ((S - w[1]) * (S - w[1])) - (w[5] * w[5])) / den;
+  const double dn = w[0] * (S - w[1]) * (S - SM) - (w[5] * w[5]);
+  if (dn != 0) {
+    const RDen dd = rden(dn);
+    const double sv = quot(SM - w[1], dd);
+    const double sb = quot(w[0] * ((S - w[1]) * (S - w[1])) - (w[5] * w[5]), dd);
     double denb = 0., svb = 0., sbb = 0.;
     wb[7] += wsb[7] * sb;
     sbb += wsb[7] * w[7];
     wb[6] += wsb[6] * sb;
     sbb += wsb[6] * w[6];
-    const double Nsb = sbb / den;
-    denb -= sbb * sb / den;
+    const double Nsb = quot(sbb, dd);
+    denb -= quot(sbb * sb, dd);
     wb[0] += Nsb * (a * a);
     ab += Nsb * w[0] * 2. * a;
     wb[5] -= Nsb * 2. * w[5];
@@ -540,9 +587,10 @@ __host__ __device__ inline void hlld_star_bwd(const double* w, double S, double 
     wb[5] -= wsb[2] * w[6] * sv;
     wb[6] -= wsb[2] * w[5] * sv;
     svb -= wsb[2] * w[5] * w[6];
-    SMb += svb / den;
-    wb[1] -= svb / den;
-    denb -= svb * sv / den;
+    const double Nsv = quot(svb, dd);
+    SMb += Nsv;
+    wb[1] -= Nsv;
+    denb -= quot(svb * sv, dd);
     wb[0] += denb * a * b;
     ab += denb * w[0] * b;
     bb += denb * w[0] * a;
@@ -554,16 +602,16 @@ __host__ __device__ inline void hlld_star_bwd(const double* w, double S, double 
   wb[5] += wsb[5];
   SMb += wsb[1];
   // ws0 = w0 a / b
-  wb[0] += wsb[0] * a / b;
-  ab += wsb[0] * w[0] / b;
-  bb -= wsb[0] * ws[0] / b;
+  wb[0] += quot(wsb[0] * a, db);
+  ab += quot(wsb[0] * w[0], db);
+  bb -= quot(wsb[0] * ws[0], db);
   Sb += ab + bb;
   wb[1] -= ab;
   SMb -= bb;
 }
 
 // star_cons reverse: ub -> (wb, eb) of the star state
-__host__ __device__ inline void star_cons_bwd(const double* w, const double* ub, double* wb, double& eb) {
+__host__ __device__ AMR_INLINE void star_cons_bwd(const double* w, const double* ub, double* wb, double& eb) {
   wb[0] += ub[0] + ub[1] * w[1] + ub[2] * w[2] + ub[3] * w[3];
   wb[1] += ub[1] * w[0];
   wb[2] += ub[2] * w[0];
@@ -575,7 +623,7 @@ __host__ __device__ inline void star_cons_bwd(const double* w, const double* ub,
 }
 
 // star_cons reverse with ub = sc Nb
-__host__ __device__ inline void star_cons_bwd_s(const double* w, const double* Nb, double sc, double* wb,
+__host__ __device__ AMR_INLINE void star_cons_bwd_s(const double* w, const double* Nb, double sc, double* wb,
                                                 double& eb) {
   double ub[8];
 #pragma unroll
@@ -584,7 +632,7 @@ __host__ __device__ inline void star_cons_bwd_s(const double* w, const double* N
 }
 
 // component k of star_cons(w, e)
-__host__ __device__ inline double star_cons_k(const double* w, double e, int k) {
+__host__ __device__ AMR_INLINE double star_cons_k(const double* w, double e, int k) {
   switch (k) {
     case 0: return w[0];
     case 1: return w[0] * w[1];
@@ -606,13 +654,13 @@ struct HlldSides {
   double eL, HL, ptL, eR, HR, ptR;
   FastT fL, fR;
 };
-__host__ __device__ inline void hlld_sides(const double* wL, const double* wR, double g, HlldSides& s) {
+__host__ __device__ AMR_INLINE void hlld_sides(const double* wL, const double* wR, double g, HlldSides& s) {
   side_fwd(wL, g, s.fL, s.eL, s.HL);
   side_fwd(wR, g, s.fR, s.eR, s.HR);
   s.ptL = wL[4] + 0.5 * (wL[5] * wL[5] + wL[6] * wL[6] + wL[7] * wL[7]);
   s.ptR = wR[4] + 0.5 * (wR[5] * wR[5] + wR[6] * wR[6] + wR[7] * wR[7]);
 }
-__host__ __device__ inline void hlld_tail_bwd(const double* wL_, const double* wR_, double g, double SL, double SR,
+__host__ __device__ AMR_INLINE void hlld_tail_bwd(const double* wL_, const double* wR_, double g, double SL, double SR,
                                               double SM, double pts, double den, bool left, const double* fb,
                                               double sq, double SLb, double SRb, double SMb, double ptsb, double eLb,
                                               double eRb, double ptLb, double ptRb, double* wLb, double* wRb) {
@@ -629,8 +677,9 @@ __host__ __device__ inline void hlld_tail_bwd(const double* wL_, const double* w
   const double dR = SR - vR, dL = SL - vL;
   double dRb = 0., dLb = 0., denb = 0., vLb = 0., vRb = 0., wL0b = 0., wR0b = 0.;
   {
-    const double Ns = SMb / den, Np = ptsb / den;
-    denb -= SMb * SM / den + ptsb * pts / den;
+    const RDen dn = rden(den);
+    const double Ns = quot(SMb, dn), Np = quot(ptsb, dn);
+    denb -= quot(SMb * SM, dn) + quot(ptsb * pts, dn);
     dRb += Ns * wR[0] * vR;
     wR0b += Ns * dR * vR;
     vRb += Ns * dR * wR[0];
@@ -685,7 +734,7 @@ __host__ __device__ inline void hlld_tail_bwd(const double* wL_, const double* w
 // (1, 6) reverse one side's flux, regions 2 and 5 one star state, regions 3
 // and 4 both star states and the double-star state.  Star conserved vectors
 // are formed per component where they are used.
-__host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, double g, const double* fb, double* wLb,
+__host__ __device__ AMR_INLINE void hlld_vjp(const double* wL, const double* wR, double g, const double* fb, double* wLb,
                                          double* wRb, double* f = nullptr) {
   HlldSides s;
   hlld_sides(wL, wR, g, s);
@@ -694,13 +743,15 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
   const double SL = std_min(vL, vR) - cmax;
   const double SR = std_max(vL, vR) + cmax;
   const double den = (SR - vR) * wR[0] - (SL - vL) * wL[0];
-  const double SM = ((SR - vR) * wR[0] * vR - (SL - vL) * wL[0] * vL - s.ptR + s.ptL) / den;
-  const double pts = ((SR - vR) * wR[0] * s.ptL - (SL - vL) * wL[0] * s.ptR +
-                      wL[0] * wR[0] * (SR - vR) * (SL - vL) * (vR - vL)) / den;
+  const RDen dm = rden(den);
+  const double SM = quot((SR - vR) * wR[0] * vR - (SL - vL) * wL[0] * vL - s.ptR + s.ptL, dm);
+  const double pts = quot((SR - vR) * wR[0] * s.ptL - (SL - vL) * wL[0] * s.ptR +
+                              wL[0] * wR[0] * (SR - vR) * (SL - vL) * (vR - vL),
+                          dm);
   // star densities (hlld_star's ws[0]) and the Alfven speeds they give
-  const double rl = sqrt(wL[0] * (SL - wL[1]) / (SL - SM)), rr = sqrt(wR[0] * (SR - wR[1]) / (SR - SM));
-  const double SLs = SM - fabs(wL[5]) / rl;
-  const double SRs = SM + fabs(wR[5]) / rr;
+  const double rl = rroot(rdiv(wL[0] * (SL - wL[1]), SL - SM)), rr = rroot(rdiv(wR[0] * (SR - wR[1]), SR - SM));
+  const double SLs = SM - rdiv(fabs(wL[5]), rl);
+  const double SRs = SM + rdiv(fabs(wR[5]), rr);
   int region = 0;
   if (SL > 0) region = 1;
   else if (SL <= 0. && SLs >= 0.) region = 2;
@@ -733,7 +784,7 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
   if (region == 2 || region == 5) {
     // f = F + S (q* - q) of the active side
     double ws[8], es;
-    hlld_star(w, S, SM, pts, ee, left ? s.ptL : s.ptR, ws, es);
+    hlld_star_fast(w, S, SM, pts, ee, left ? s.ptL : s.ptR, ws, es);
     double Sb = 0.;
     for (int k = 0; k < 8; k++) {
       double q, F;
@@ -757,19 +808,20 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
   }
   // regions 3 and 4: both star states and the double-star state
   double wLs[8], wRs[8], eLs, eRs;
-  hlld_star(wL, SL, SM, pts, s.eL, s.ptL, wLs, eLs);
-  hlld_star(wR, SR, SM, pts, s.eR, s.ptR, wRs, eRs);
-  const double rlr = sqrt(wLs[0] * wRs[0]);
+  hlld_star_fast(wL, SL, SM, pts, s.eL, s.ptL, wLs, eLs);
+  hlld_star_fast(wR, SR, SM, pts, s.eR, s.ptR, wRs, eRs);
+  const double rlr = rroot(wLs[0] * wRs[0]);
   const double sg = sign0(wL[5]), sgR = sign0(wR[5]);
+  const RDen dlr = rden(rl + rr);
   double wss[8];
   wss[0] = wLs[0];
   wss[1] = SM;
-  wss[2] = (rl * wLs[2] + rr * wRs[2] + (wRs[6] - wLs[6]) * sg) / (rl + rr);
-  wss[3] = (rl * wLs[3] + rr * wRs[3] + (wRs[7] - wLs[7]) * sg) / (rl + rr);
+  wss[2] = quot(rl * wLs[2] + rr * wRs[2] + (wRs[6] - wLs[6]) * sg, dlr);
+  wss[3] = quot(rl * wLs[3] + rr * wRs[3] + (wRs[7] - wLs[7]) * sg, dlr);
   wss[4] = 0.;
   wss[5] = wLs[5];
-  wss[6] = (rl * wRs[6] + rr * wLs[6] + rlr * (wRs[2] - wLs[2]) * sg) / (rl + rr);
-  wss[7] = (rl * wRs[7] + rr * wLs[7] + rlr * (wRs[3] - wLs[3]) * sg) / (rl + rr);
+  wss[6] = quot(rl * wRs[6] + rr * wLs[6] + rlr * (wRs[2] - wLs[2]) * sg, dlr);
+  wss[7] = quot(rl * wRs[7] + rr * wLs[7] + rlr * (wRs[3] - wLs[3]) * sg, dlr);
   const double dss = vdotb(wss);
   const double eLss = eLs - rl * (vdotb(wLs) - dss) * sg;
   const double eRss = eRs + rr * (vdotb(wRs) - dss) * sgR;
@@ -803,10 +855,10 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
   }
   // S_L* = SM - |BxL| / rl, S_R* = SM + |BxR| / rr
   SMb += SLsb + SRsb;
-  wLb[5] -= SLsb * sign0(wL[5]) / rl;
-  rlb += SLsb * fabs(wL[5]) / (rl * rl);
-  wRb[5] += SRsb * sign0(wR[5]) / rr;
-  rrb -= SRsb * fabs(wR[5]) / (rr * rr);
+  wLb[5] -= rdiv(SLsb * sign0(wL[5]), rl);
+  rlb += rdiv(SLsb * fabs(wL[5]), rl * rl);
+  wRb[5] += rdiv(SRsb * sign0(wR[5]), rr);
+  rrb -= rdiv(SRsb * fabs(wR[5]), rr * rr);
   // e_L** = e_L* - rl (vdotb(wLs) - dss) sg; e_R** = e_R* + rr (vdotb(wRs) - dss) sgR
   double dssb = 0., vLsb = 0., vRsb = 0.;
   eLsb += eLssb;
@@ -837,14 +889,14 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
   wssb[3] += dssb * wss[7];
   wssb[7] += dssb * wss[3];
   // w**
-  const double D = rl + rr;
+  const RDen dD = rden(rl + rr);
   double Db = 0.;
   wLsb[0] += wssb[0];
   SMb += wssb[1];
   wLsb[5] += wssb[5];
   {
-    const double N = wssb[2] / D;
-    Db -= wssb[2] * wss[2] / D;
+    const double N = quot(wssb[2], dD);
+    Db -= quot(wssb[2] * wss[2], dD);
     rlb += N * wLs[2];
     wLsb[2] += N * rl;
     rrb += N * wRs[2];
@@ -853,8 +905,8 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
     wLsb[6] -= N * sg;
   }
   {
-    const double N = wssb[3] / D;
-    Db -= wssb[3] * wss[3] / D;
+    const double N = quot(wssb[3], dD);
+    Db -= quot(wssb[3] * wss[3], dD);
     rlb += N * wLs[3];
     wLsb[3] += N * rl;
     rrb += N * wRs[3];
@@ -863,8 +915,8 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
     wLsb[7] -= N * sg;
   }
   {
-    const double N = wssb[6] / D;
-    Db -= wssb[6] * wss[6] / D;
+    const double N = quot(wssb[6], dD);
+    Db -= quot(wssb[6] * wss[6], dD);
     rlb += N * wRs[6];
     wRsb[6] += N * rl;
     rrb += N * wLs[6];
@@ -874,8 +926,8 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
     wLsb[2] -= N * rlr * sg;
   }
   {
-    const double N = wssb[7] / D;
-    Db -= wssb[7] * wss[7] / D;
+    const double N = quot(wssb[7], dD);
+    Db -= quot(wssb[7] * wss[7], dD);
     rlb += N * wRs[7];
     wRsb[7] += N * rl;
     rrb += N * wLs[7];
@@ -887,10 +939,10 @@ __host__ __device__ inline void hlld_vjp(const double* wL, const double* wR, dou
   rlb += Db;
   rrb += Db;
   // rl = sqrt(rhoL*), rr = sqrt(rhoR*), rlr = sqrt(rhoL* rhoR*)
-  if (rl > 0.) wLsb[0] += rlb * 0.5 / rl;
-  if (rr > 0.) wRsb[0] += rrb * 0.5 / rr;
+  if (rl > 0.) wLsb[0] += rdiv(rlb * 0.5, rl);
+  if (rr > 0.) wRsb[0] += rdiv(rrb * 0.5, rr);
   if (rlr > 0.) {
-    const double pb = rlrb * 0.5 / rlr;
+    const double pb = rdiv(rlrb * 0.5, rlr);
     wLsb[0] += pb * wRs[0];
     wRsb[0] += pb * wLs[0];
   }

@@ -45,13 +45,8 @@ __device__ inline int spec_solver(int inst_solver) {
 // +0.
 enum { kTileNan = 1, kTileWide = 2, kTileSpatial = 4 };
 
-template <int NT, int NG>
-__device__ AMR_INLINE void stage_prim_cell(const double* __restrict__ Qin, double g, int lim, int step, const LeafItem& L,
-                                       DevError* err, int c, double* sWc, int VS, int* flags) {
-  constexpr int N2 = NT * NT, LO = NG - 1, HI = NT - 1 - NG;
-  double u[8], w[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) u[k] = Qin[k * N2 + c];
+// primitives w of the conserved state u; returns the flags it sets
+__device__ AMR_INLINE int tile_prim(const double* u, double g, double* w) {
   ExpSpan us, rs, ws;
   rs.add(u[0]);
 #pragma unroll
@@ -59,17 +54,27 @@ __device__ AMR_INLINE void stage_prim_cell(const double* __restrict__ Qin, doubl
   cons_to_prim<true>(u, g, w);
   if (!(us.within(-860, 400) && rs.within(-100, 100))) cons_to_prim<false>(u, g, w);
 #pragma unroll
-  for (int k = 0; k < 8; k++) {
-    ws.add(w[k]);
-    sWc[k * VS] = w[k];
-  }
+  for (int k = 0; k < 8; k++) ws.add(w[k]);
+  return (ws.within(kPrimLo, kPrimHi) ? 0 : kTileWide) |
+         ((__double_as_longlong(w[3]) | __double_as_longlong(w[7])) ? kTileSpatial : 0);
+}
+
+template <int NT, int NG>
+__device__ AMR_INLINE void stage_prim_cell(const double* __restrict__ Qin, double g, int lim, int step, const LeafItem& L,
+                                       DevError* err, int c, double* sWc, int VS, int* flags) {
+  constexpr int N2 = NT * NT, LO = NG - 1, HI = NT - 1 - NG;
+  double u[8], w[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) u[k] = Qin[k * N2 + c];
+  const int tile = tile_prim(u, g, w);
+#pragma unroll
+  for (int k = 0; k < 8; k++) sWc[k * VS] = w[k];
   const int i = c % NT, j = c / NT;
   if (w[4] <= 0 && i > LO && i < HI + 1 && j > LO && j < HI + 1)
     report(err, L.inst, error_key(step, L.nb, 0, i, j, 0, L.nb, kErrPressure));
   if (step == 2 && (isnan(w[1]) || isnan(w[2]) || isnan(w[3])))
     report(err, L.inst, error_key(step, L.nb, 0, i, j, 1, L.nb, kErrNanVel));
-  if (!ws.within(kPrimLo, kPrimHi)) atomicOr(flags, kTileWide);
-  if (__double_as_longlong(w[3]) | __double_as_longlong(w[7])) atomicOr(flags, kTileSpatial);
+  if (tile) atomicOr(flags, tile);
   if (lim < kLimWENO3) {
     bool bad = false;
 #pragma unroll
@@ -149,36 +154,44 @@ __device__ AMR_INLINE void face_edges_of(int lim, const double* W, int VS, int s
   }
 }
 
-// Flux fl of the x face (ydir = 0: between cells (i, j) and (i + 1, j)) or
-// y face (between (i, j) and (i, j + 1)) from the primitives in sWb (cell
-// (i, j) of variable k at sWb[k * VS + j * NT + i]) and the face B, with the
-// solver-failure and NaN-flux checks of MUSCL2D.cpp:62-115.  tile: the tile's
-// flags.
-template <int NT, int SPEC>
-__device__ AMR_INLINE void stage_face(const double* sWb, int VS, const double* __restrict__ B, int lim, int solver,
-                                  double g, double dxl, int tile, int i, int j, int ydir, int step,
-                                  const LeafItem& L, DevError* err, double* fl) {
-  constexpr int N2 = NT * NT;
-  const int s = ydir ? NT : 1;  // stride along the face normal
-  const int c = j * NT + i;     // left cell; right cell is c + s
-  const double bn = B[ydir * N2 + c + s];
+// Flux fl, in the tile's frame, of the face above the left cell W along x
+// (ydir = 0) or y from the tile's primitives (component stride VS, cell stride
+// s along the normal) and the face's normal field bn.  tile: the tile's flags.
+template <int SPEC>
+__device__ AMR_INLINE int tile_face_flux(const double* W, int VS, int s, int lim, int solver, double g, double dxl,
+                                         double bn, int tile, int ydir, double* fl) {
   const bool planar = !(tile & kTileSpatial);
   int st = 0;
   bool ok = false;
   if (!(tile & kTileWide)) {
     double wl[8], wr[8];
     wl[5] = wr[5] = bn;
-    face_edges_of<SPEC, true>(lim, sWb + c, VS, s, ydir, dxl, planar, wl, wr);
+    face_edges_of<SPEC, true>(lim, W, VS, s, ydir, dxl, planar, wl, wr);
     ok = fast_flux(solver, wl, wr, g, fl, &st);
   }
   if (!ok) {
     asm volatile("" ::: "memory");  // the tile is read again, not kept in registers across the fast path
     double wl[8], wr[8];
     wl[5] = wr[5] = bn;
-    face_edges_of<SPEC, false>(lim, sWb + c, VS, s, ydir, dxl, planar, wl, wr);
+    face_edges_of<SPEC, false>(lim, W, VS, s, ydir, dxl, planar, wl, wr);
     st = normal_flux(solver, wl, wr, g, fl);
   }
   if (ydir) swap_xy(fl);
+  return st;
+}
+
+// Flux fl of the x face (ydir = 0: between cells (i, j) and (i + 1, j)) or
+// y face (between (i, j) and (i, j + 1)) from the primitives in sWb (cell
+// (i, j) of variable k at sWb[k * VS + j * NT + i]) and the face B, with the
+// solver-failure and NaN-flux checks of MUSCL2D.cpp:62-115.
+template <int NT, int SPEC>
+__device__ AMR_INLINE void stage_face(const double* sWb, int VS, const double* __restrict__ B, int lim, int solver,
+                                      double g, double dxl, int tile, int i, int j, int ydir, int step,
+                                      const LeafItem& L, DevError* err, double* fl) {
+  constexpr int N2 = NT * NT;
+  const int s = ydir ? NT : 1;  // stride along the face normal
+  const int c = j * NT + i;     // left cell; right cell is c + s
+  const int st = tile_face_flux<SPEC>(sWb + c, VS, s, lim, solver, g, dxl, B[ydir * N2 + c + s], tile, ydir, fl);
   // per (i, j) the x face (solver, NaN), then the y face
   if (st) report(err, L.inst, error_key(step, L.nb, 2, i, j, ydir ? 3 : 0, L.nb, kErrHLLC));
   bool nan = false;

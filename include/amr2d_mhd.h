@@ -314,7 +314,7 @@ int amr_adj_step_vjp(amr_adj *adj, const double *U, const double *Bx, const doub
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc.  Same step, same results as amr_adj_step on a context created
  * with (n, dx, gamma, flux).  Its work memory is a static device array the
- * library holds on every GPU it runs on until the process ends (25.7 MB), so
+ * library holds on every GPU it runs on until the process ends (25.2 MB), so
  * n is limited to 4..256 (AMR_ERR_CONFIG beyond).  Every call on one GPU
  * shares that array: calls that overlap on one GPU (different streams or
  * host threads) race; calls ordered on one stream do not. */

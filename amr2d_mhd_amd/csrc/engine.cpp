@@ -3576,14 +3576,27 @@ int amr_riemann_batch(int solver, int dir, double gamma, int n, const double* wL
   AMR_CATCH
 }
 
+static int recon_batch(int NT, int nghosts, const char* limiter, double dx, int nt, const double* W, double* out,
+                       bool fill, void* stream) {
+  const int lim = limiter ? lim_code(limiter) : -1;
+  if (lim < 0 || NT < 2 * nghosts + 4) return AMR_ERR_CONFIG;
+  launch_recon_batch(NT, nghosts, lim, dx, nt, W, out, fill, (hipStream_t)stream);
+  HIPCHK(hipGetLastError());
+  return AMR_OK;
+}
+
 int amr_recon_batch(int NT, int nghosts, const char* limiter, double dx, int nt, const double* W, double* out,
                     void* stream) {
   AMR_TRY
-  const int lim = limiter ? lim_code(limiter) : -1;
-  if (lim < 0 || NT < 2 * nghosts + 4) return AMR_ERR_CONFIG;
-  launch_recon_batch(NT, nghosts, lim, dx, nt, W, out, (hipStream_t)stream);
-  HIPCHK(hipGetLastError());
-  return AMR_OK;
+  return recon_batch(NT, nghosts, limiter, dx, nt, W, out, false, stream);
+  AMR_CATCH
+}
+
+// amr_recon_batch into memory the caller has not cleared (the Python binding)
+int amr_recon_batch_fill(int NT, int nghosts, const char* limiter, double dx, int nt, const double* W, double* out,
+                         void* stream) {
+  AMR_TRY
+  return recon_batch(NT, nghosts, limiter, dx, nt, W, out, true, stream);
   AMR_CATCH
 }
 

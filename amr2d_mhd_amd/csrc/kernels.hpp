@@ -181,6 +181,8 @@ int launch_step(int NT, int ng, int spec, int lanes_idx, int grid, const StepArg
 // pointwise / tile-level parity entry points
 void launch_riemann_batch(int solver, int dir, double gamma, int n, const double* wL, const double* wR, double* flux,
                           int32_t* status, hipStream_t s);
-void launch_recon_batch(int NT, int ng, int lim, double dx, int nt, const double* W, double* out, hipStream_t s);
+// fill: entries outside the reference's computed range are written as zeros
+void launch_recon_batch(int NT, int ng, int lim, double dx, int nt, const double* W, double* out, bool fill,
+                        hipStream_t s);
 
 }  // namespace amr

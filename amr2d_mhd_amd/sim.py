@@ -300,9 +300,9 @@ def recon_batch(W, limiter, nghosts, dx=1.0):
 
     W = W.contiguous()
     nt, NT = W.shape[0], W.shape[-1]
-    out = torch.zeros((nt, 4, 8, NT, NT), dtype=torch.float64, device=W.device)
+    out = torch.empty((nt, 4, 8, NT, NT), dtype=torch.float64, device=W.device)
     stream = torch.cuda.current_stream(W.device).cuda_stream
-    rc = lib().amr_recon_batch(NT, nghosts, limiter.encode(), float(dx), nt, W.data_ptr(), out.data_ptr(), stream)
+    rc = lib().amr_recon_batch_fill(NT, nghosts, limiter.encode(), float(dx), nt, W.data_ptr(), out.data_ptr(), stream)
     if rc != 0:
         raise AmrError(rc)
     return out

@@ -106,3 +106,42 @@ def test_stage_exponents(lim, ng, variant, planar):
             same = _same_bits(np.ascontiguousarray(a), np.ascontiguousarray(b))
             assert same.all(), f"{lim} below 2^-{lo}: {f} differs in {int((~same).sum())} values"
     sim.close()
+
+
+@pytest.mark.parametrize("lim,ng", [("1st", 2), ("noSL", 2), ("minmod", 1), ("VanLeer", 2), ("Superbee", 2),
+                                    ("MC", 2), ("Koren", 2), ("Cada3rd", 2), ("WENO3", 2), ("WENO5", 3), ("WENO5", 4)])
+@pytest.mark.parametrize("NT", [12, 17, 20, 28, 30])
+def test_recon_batch_exponents_and_sizes(lim, ng, NT):
+    """Tiles in LDS (up to 28 cells a side) and beyond: values in and out of
+    the range against the oracle; entries outside the computed range are zeros
+    from the binding and untouched by the C entry point."""
+    torch = pytest.importorskip("torch")
+    import amr2d_mhd_amd as A
+    from amr2d_mhd_amd._lib import lib
+
+    if NT < 2 * ng + 4:
+        pytest.skip("smaller than the ghost depth allows")
+    rng = np.random.default_rng(3 + NT)
+    nt = 4
+    W = rng.uniform(0.2, 2.0, (nt, 8, NT, NT))
+    for t, lo in ((1, 700), (2, 830), (3, 1070)):
+        W[t] *= np.exp2(-rng.integers(0, lo, W[t].shape).astype(np.float64)) * (rng.random(W[t].shape) < 0.9)
+    dW = torch.from_numpy(W).cuda()
+    torch.full((nt, 4, 8, NT, NT), 7.0, dtype=torch.float64, device="cuda")  # what an allocation may hold
+    out = A.recon_batch(dW, lim, ng, dx=1.0 / 30).cpu().numpy()
+    raw = torch.full((nt, 4, 8, NT, NT), 7.0, dtype=torch.float64, device="cuda")
+    rc = lib().amr_recon_batch(NT, ng, lim.encode(), 1.0 / 30, nt, dW.data_ptr(), raw.data_ptr(),
+                               torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    raw = raw.cpu().numpy()
+    weno = lim.startswith("WENO")
+    lo, hi = (ng - 1, NT - ng) if weno else (0, NT - 2)
+    inside = np.zeros(out.shape, bool)
+    inside[:, :, :, lo:hi + 1, lo:hi + 1] = True
+    inside[:, 0:2, 5] = inside[:, 2:4, 6] = False
+    for t in range(nt):
+        (xl, xr, yl, yr), _ = O.recon_tile(W[t], lim, ng, dx=1.0 / 30)
+        same = _same_bits(out[t], np.stack([xl, xr, yl, yr]))[inside[t]]
+        assert same.all(), f"{lim}: tile {t} differs in {int((~same).sum())} entries"
+    assert _same_bits(raw, out)[inside].all()
+    assert (out[~inside].view(np.int64) == 0).all() and (raw[~inside] == 7.0).all()

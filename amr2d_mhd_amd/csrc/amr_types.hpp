@@ -100,6 +100,24 @@ struct FillOp {
   uint16_t pad;
 };
 
+// The fill program by destination: for each ring element of a slot (ring_index)
+// the op that fills it, packed as version (24 bits) | kind (2) | source cell
+// (10) | source slot or FillGen index (28).  The entry counts while its version
+// is the current one: programs overwrite the table without clearing it.
+constexpr int ring_cells(int NT, int ng) { return NT * NT - (NT - 2 * ng) * (NT - 2 * ng); }
+// position of cell (i, j) among the ring cells in row order, -1 in the interior
+inline __host__ __device__ int ring_index(int NT, int ng, int i, int j) {
+  const int w = NT - 2 * ng;
+  if (j < ng) return j * NT + i;
+  if (j >= NT - ng) return ng * NT + w * 2 * ng + (j - (NT - ng)) * NT + i;
+  if (i < ng) return ng * NT + (j - ng) * 2 * ng + i;
+  return i >= NT - ng ? ng * NT + (j - ng) * 2 * ng + i - w : -1;
+}
+constexpr uint32_t kRingVersions = 1u << 24;
+inline __host__ __device__ uint64_t ring_entry(uint32_t version, int op, int cell, int32_t src) {
+  return ((uint64_t)version << 40) | ((uint64_t)op << 38) | ((uint64_t)cell << 28) | (uint64_t)(uint32_t)src;
+}
+
 // explicit operands of a restriction, in the order of FillOp's 2x2 cells
 struct FillGen {
   int64_t ref[4];

@@ -456,6 +456,10 @@ struct amr_ctx {
   int steps_same_topo = 0;
   // compiled fill programs kept per instance besides the current one (LRU)
   int prog_cache_max = 4;
+  // fill programs by destination and scratch of the fused CT launches, which
+  // serve the current trees when ct_fused
+  RingTable ring;
+  bool ct_fused = false;
   // a step launched by step_begin and not yet completed by step_end
   bool in_flight = false;
   uint64_t prog_clock = 0;
@@ -2073,6 +2077,28 @@ int upload_tree(amr_ctx* c, int q) {
   return 0;
 }
 
+// Whether the blocks a fill of I reads and writes are all leaves: the finer
+// neighbours of a leaf are (a tree whose levels step by one), so that every
+// source block forms its CT values in the same launch.
+bool leaf_neighbours(const Instance& I) {
+  static const int son[4] = {1, 0, 2, 0}, stride[4] = {2, 2, 1, 1};
+  for (int nb = 0; nb < I.lastActive; nb++) {
+    if (!I.leafs[nb]) continue;
+    for (int s = 0; s < 4; s++) {
+      const int n = I.lp[nb][4 + s];
+      if (n == -1 || I.leafs[n]) continue;
+      if (I.lp[n][0] < I.lp[nb][0]) return false;
+      const int f = I.lp[n][2] + son[s];
+      if (!I.leafs[f] || !I.leafs[f + stride[s]]) return false;
+    }
+  }
+  return true;
+}
+
+size_t ring_bytes(const amr_ctx* c) {
+  return sizeof(uint64_t) * (size_t)c->cap_slots * ring_cells(c->NT, c->ng);
+}
+
 int rebuild_topology(amr_ctx* c) {
   HostTimed ht(c, PF_HOST_TOPO);
   HIPCHK(hipStreamSynchronize(c->stream));  // previous uploads consumed
@@ -2246,6 +2272,16 @@ int rebuild_topology(amr_ctx* c) {
   c->d_tail_prefix = (int32_t*)(c->d_topo + off_tpre);
   c->d_rgi = (RegridInst*)(c->d_topo + off_rgi);
   c->d_leaves = (LeafItem*)(c->d_topo + off_leaf);
+  // the programs by destination, for the fused CT launches
+  c->ct_fused = true;
+  for (const Instance& I : c->inst) c->ct_fused &= I.done || leaf_neighbours(I);
+  if (c->ct_fused) {
+    if (++c->ring.version == kRingVersions) {
+      HIPCHK(hipMemsetAsync(c->ring.entries, 0, ring_bytes(c), c->stream));
+      c->ring.version = 1;
+    }
+    launch_ring_table(c->NT, c->ng, c->d_inst_ops, c->d_prefix, ni, c->nchunks, c->ring, c->stream);
+  }
   c->topo_dirty = false;
   c->steps_same_topo = 0;
   direct_geometry(c);
@@ -2306,6 +2342,13 @@ void run_stage(amr_ctx* c, int step) {
 
 // CT2D.cpp:11-124
 void run_ct(amr_ctx* c, int step) {
+  // (a captured step's kernels may not hold the table's version: it outlives it)
+  if (c->ct_fused && !c->launch_counts) {
+    Timed tm(c, PF_CT);
+    launch_ct(c->NT, c->ng, c->F, c->d_leaves, c->grid_leaves, c->d_ip, step, c->rk, c->d_inst_gen, c->ring, c->d_err,
+              c->stream);
+    return;
+  }
   {
     Timed tm(c, PF_CT);
     launch_emf(c->NT, c->F, c->d_leaves, c->grid_leaves, c->d_ip, step, c->rk, c->d_err, c->stream, c->launch_counts);
@@ -2926,6 +2969,14 @@ int amr_create(int n_inst, const amr_sim_config* cfgs, int64_t slot_capacity, am
       return AMR_ERR_HIP;
     }
   }
+  if (hipMalloc((void**)&c->ring.entries, ring_bytes(c)) != hipSuccess ||
+      hipMemset(c->ring.entries, 0, ring_bytes(c)) != hipSuccess ||
+      hipMalloc((void**)&c->ring.emf, sizeof(double) * N2 * c->cap_slots) != hipSuccess ||
+      hipMalloc((void**)&c->ring.old, sizeof(double) * 2 * N2 * c->cap_slots) != hipSuccess ||
+      hipMalloc((void**)&c->ring.rdx, sizeof(double) * c->cap_slots) != hipSuccess) {
+    amr_destroy(c);
+    return AMR_ERR_HIP;
+  }
   // error records, then the step kernel's barrier-failure flag
   c->rec_err_bytes = (sizeof(DevError) * n_inst + sizeof(int32_t) + 255) & ~size_t(255);
   // [error records | regrid records | op log | per-leaf CFL bounds and indicators]
@@ -2994,6 +3045,10 @@ int amr_destroy(amr_ctx* c) {
   if (c->own_stream) hipStreamSynchronize(c->own_stream);
   for (int f = 0; f < kNumFields; f++)
     if (c->F.f[f]) hipFree(c->F.f[f]);
+  hipFree(c->ring.entries);
+  hipFree(c->ring.emf);
+  hipFree(c->ring.old);
+  hipFree(c->ring.rdx);
   hipFree(c->d_topo);
   if (c->h_topo) hipHostFree(c->h_topo);
   for (auto& I : c->inst) {

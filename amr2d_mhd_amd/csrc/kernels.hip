@@ -14,6 +14,16 @@ __global__ __launch_bounds__(kThreads) void fill_kernel(FillProgram P, FillSet s
   fill_chunk(P, set, NT, blockIdx.x, threadIdx.x, true);
 }
 
+// the program's ops by destination
+__global__ __launch_bounds__(kFillChunk) void ring_table_kernel(FillProgram P, int NT, int ng, uint64_t* ring,
+                                                                uint32_t version) {
+  const int w = blockIdx.x, q = find_segment(P, w);
+  const FillOp op = P.ops[q][(w - P.cprefix[q]) * kFillChunk + threadIdx.x];
+  if (op.op == kFillNop) return;
+  const int r = ring_index(NT, ng, op.dst_cell % NT, op.dst_cell / NT);
+  if (r >= 0) ring[(size_t)op.dst_gs * ring_cells(NT, ng) + r] = ring_entry(version, op.op, op.src_cell, op.src);
+}
+
 // ------------------------------------------------------------------ regrid
 // refine.cpp:17-36: minmod-limited quarter-slope prolongation of one value
 __device__ inline double prolong(const double* Q, int NT, int i, int j, int sx, int sy) {
@@ -188,7 +198,7 @@ __global__ __launch_bounds__(kFaceLanes) __attribute__((amdgpu_waves_per_eu(3)))
   for (int k = 0; k < 8; k++) flux[8 * q + k] = f[k];
 }
 
-// edge states of whole tiles: out = [tile][4: xL xR yL yR][8][NT][NT]
+// edge states of whole tiles, any tile size and ghost depth: out = [tile][4: xL xR yL yR][8][NT][NT]
 // (celledges.cpp ranges for MUSCL, WENO2D_primvar.cpp ranges for WENO)
 __global__ void recon_batch_kernel(int NT, int ng, int lim, double dxl, const double* W, double* out) {
   const int N2 = NT * NT;
@@ -349,6 +359,28 @@ void launch_bsync(int NT, const FieldPtrs& F, const LeafItem* leaves, int nleaf,
   if (nleaf <= 0) return;
   dim3 grid((NT * NT + kThreads - 1) / kThreads, nleaf);
   AMR_DISPATCH_TILE(NT, (NT == 24 ? 4 : 2), (bsync_kernel<T><<<grid, kThreads, 0, s>>>(F, leaves, last, counts)));
+}
+
+// kernel arguments of the fused CT launches
+static CtArgs ct_args(const FieldPtrs& F, const LeafItem* leaves, const InstParams* ip, int step, int rk,
+                      const FillGen* const* inst_gen, const RingTable& ring, DevError* err) {
+  return CtArgs{F,    leaves,   ip,       inst_gen, ring.entries, ring.version, step,
+                rk,   ring.emf, ring.old, ring.rdx, err};
+}
+
+void launch_ct(int NT, int ng, const FieldPtrs& F, const LeafItem* leaves, int nleaf, const InstParams* ip, int step,
+               int rk, const FillGen* const* inst_gen, const RingTable& ring, DevError* err, hipStream_t s) {
+  if (nleaf <= 0) return;
+  const CtArgs A = ct_args(F, leaves, ip, step, rk, inst_gen, ring, err);
+  AMR_DISPATCH_TILE(NT, ng, (ct_emf_kernel<T, G><<<nleaf, kCtLanes<T>, 0, s>>>(A)));
+  AMR_DISPATCH_TILE(NT, ng, (ct_faces_kernel<T, G><<<nleaf, kCtLanes<T>, 0, s>>>(A)));
+}
+
+void launch_ring_table(int NT, int ng, const FillOp* const* inst_ops, const int32_t* cprefix, int ninst, int nchunks,
+                       const RingTable& ring, hipStream_t s) {
+  if (nchunks <= 0) return;
+  const FillProgram P{inst_ops, nullptr, cprefix, ninst};
+  ring_table_kernel<<<nchunks, kFillChunk, 0, s>>>(P, NT, ng, ring.entries, ring.version);
 }
 
 void launch_fill(int NT, const FillOp* const* inst_ops, const FillGen* const* inst_gen, const int32_t* cprefix,

@@ -94,6 +94,22 @@ void launch_bsync(int NT, const FieldPtrs& F, const LeafItem* leaves, int nleaf,
 // ghost fill of up to four fields through a program made of per-instance
 // segments of whole kFillChunk-op chunks (device pointer tables
 // inst_ops/inst_gen, cprefix[ninst+1] of chunk counts), one workgroup per chunk
+// The fill programs by destination (amr_types.hpp) and the scratch fields of the
+// fused CT launches; version: the entries that count
+struct RingTable {
+  uint64_t* entries = nullptr;  // [slot][ring_cells]
+  double* emf = nullptr;        // [slot][N2]
+  double* old = nullptr;        // [slot][2][N2]
+  double* rdx = nullptr;        // [slot]
+  uint32_t version = 0;
+};
+// enters the programs of the running instances into the table
+void launch_ring_table(int NT, int ng, const FillOp* const* inst_ops, const int32_t* cprefix, int ninst, int nchunks,
+                       const RingTable& ring, hipStream_t s);
+// CT2D.cpp:11-124 with its ghost fills for trees whose programs touch leaves
+// only: two launches
+void launch_ct(int NT, int ng, const FieldPtrs& F, const LeafItem* leaves, int nleaf, const InstParams* ip, int step,
+               int rk, const FillGen* const* inst_gen, const RingTable& ring, DevError* err, hipStream_t s);
 void launch_fill(int NT, const FillOp* const* inst_ops, const FillGen* const* inst_gen, const int32_t* cprefix,
                  int ninst, int nchunks, const FillSet& set, hipStream_t s, const int32_t* counts = nullptr);
 // per-leaf CFL bound min(dx,dy)/lambda and refinement indicator, as pairs

@@ -18,35 +18,22 @@ __device__ inline void ct2_pc(const double* q, int N2, int c, double g, double& 
   C = sqrt((g * p + (q5 * q5 + q6 * q6 + q7 * q7)) / q0);
 }
 
-// CT2D.cpp:15-75: corner EMF from the face fluxes for i,j in [1,NT-1].
-// CTtype 1: the mean of the four face values.  CTtype 2 ("upwind"): the
-// y-flux and x-flux pairs weighted 1 - psi and psi, psi = dPx / (dPx + dPy)
-// where the pressure jump around the corner exceeds half the smallest
-// pressure (sw1) and the flow is compressive beyond a tenth of the smallest
-// fast speed (sw2), else psi = 0.5; the velocity divergence keeps the
-// reference's terms as written (two y-velocity quotients divide q2 by
-// itself, CT2D.cpp:45).  q is the stage state (Us, or U on the last stage).
+// CT2D.cpp:28-75: the CTtype 2 ("upwind") weight at the corner of cell c:
+// psi = dPx / (dPx + dPy) where the pressure jump around the corner exceeds half
+// the smallest pressure (sw1) and the flow is compressive beyond a tenth of the
+// smallest fast speed (sw2), else 0.5; the velocity divergence keeps the
+// reference's terms as written (two y-velocity quotients divide q2 by itself,
+// CT2D.cpp:45).  q is the stage state (Us, or U on the last stage).
 template <int NT>
-__device__ inline void emf_cell(const FieldPtrs& F, const LeafItem L, const InstParams* __restrict__ ip, int last,
-                                DevError* err, int step, int c) {
+__device__ inline double ct2_weight(const double* q, int c, double g) {
   constexpr int N2 = NT * NT;
-  const int i = c % NT, j = c / NT;
-  if (i < 1 || j < 1) return;
-  const double* gg5 = F.f[kGG] + (size_t)L.gs * 8 * N2 + 5 * N2;
-  const double* ff6 = F.f[kFF] + (size_t)L.gs * 8 * N2 + 6 * N2;
-  const InstParams& P = ip[L.inst];
-  if (P.ct_type != 2) {
-    F.f[kEMF][(size_t)L.gs * N2 + c] = 0.25 * ((gg5[c - 1] + gg5[c]) - (ff6[c - NT] + ff6[c]));
-    return;
-  }
-  const double* q = F.f[last ? kU : kUs] + (size_t)L.gs * 8 * N2;
   // cells (i, j), (i, j-1), (i-1, j), (i-1, j-1) of the reference's [i][j]
   const int c00 = c, c0m = c - NT, cm0 = c - 1, cmm = c - 1 - NT;
   double p00, p0m, pm0, pmm, C00, C0m, Cm0, Cmm;
-  ct2_pc(q, N2, c00, P.gamma, p00, C00);
-  ct2_pc(q, N2, c0m, P.gamma, p0m, C0m);
-  ct2_pc(q, N2, cm0, P.gamma, pm0, Cm0);
-  ct2_pc(q, N2, cmm, P.gamma, pmm, Cmm);
+  ct2_pc(q, N2, c00, g, p00, C00);
+  ct2_pc(q, N2, c0m, g, p0m, C0m);
+  ct2_pc(q, N2, cm0, g, pm0, Cm0);
+  ct2_pc(q, N2, cmm, g, pmm, Cmm);
   const double beta = 0.5, delta = 0.1;
   const double dPx = 0.5 * fabs(p00 + p0m - pm0 - pmm);
   const double dPy = 0.5 * fabs(p00 + pm0 - p0m - pmm);
@@ -65,6 +52,26 @@ __device__ inline void emf_cell(const FieldPtrs& F, const LeafItem L, const Inst
   const bool sw2 = (-delta * tC) > divV;
   double psi = 0.5;
   if (sw1 && sw2) psi = dPx / (dPx + dPy);
+  return psi;
+}
+
+// CT2D.cpp:15-75: corner EMF from the face fluxes for i,j in [1,NT-1].
+// CTtype 1: the mean of the four face values.  CTtype 2: the y-flux and x-flux
+// pairs weighted 1 - psi and psi.
+template <int NT>
+__device__ inline void emf_cell(const FieldPtrs& F, const LeafItem L, const InstParams* __restrict__ ip, int last,
+                                DevError* err, int step, int c) {
+  constexpr int N2 = NT * NT;
+  const int i = c % NT, j = c / NT;
+  if (i < 1 || j < 1) return;
+  const double* gg5 = F.f[kGG] + (size_t)L.gs * 8 * N2 + 5 * N2;
+  const double* ff6 = F.f[kFF] + (size_t)L.gs * 8 * N2 + 6 * N2;
+  const InstParams& P = ip[L.inst];
+  if (P.ct_type != 2) {
+    F.f[kEMF][(size_t)L.gs * N2 + c] = 0.25 * ((gg5[c - 1] + gg5[c]) - (ff6[c - NT] + ff6[c]));
+    return;
+  }
+  const double psi = ct2_weight<NT>(F.f[last ? kU : kUs] + (size_t)L.gs * 8 * N2, c, P.gamma);
   if (psi < 0 || psi > 1) report(err, L.inst, error_key(step, kSeqCt | L.nb, 0, i, j, 0, L.nb, kErrCtPsi));
   F.f[kEMF][(size_t)L.gs * N2 + c] = 0.5 * (1. - psi) * (gg5[c - 1] + gg5[c]) - 0.5 * psi * (ff6[c - NT] + ff6[c]);
 }
@@ -118,20 +125,24 @@ __global__ __launch_bounds__(kThreads) void bupdate_kernel(FieldPtrs F, const Le
   if (c < NT * NT) bupdate_cell<NT>(F, leaves[blockIdx.y], ip, step, rk, c);
 }
 
-// CT2D.cpp:95-123: cell-centred B from the updated faces + energy correction
+// CT2D.cpp:95-123: cell-centred B from the updated faces Bn + energy correction
 template <int NT>
-__device__ inline void bsync_cell(const FieldPtrs& F, const LeafItem L, int last, int c) {
+__device__ inline void sync_cell(const double* Bn, double* q, int c, double q4, double q5, double q6) {
   constexpr int N2 = NT * NT;
   const int i = c % NT, j = c / NT;
-  const double* Bn = F.f[last ? kBi : kBis] + (size_t)L.gs * 2 * N2;
-  double* q = F.f[last ? kU : kUs] + (size_t)L.gs * 8 * N2;
   const int ip = i < NT - 1 ? i + 1 : i, jp = j < NT - 1 ? j + 1 : j;
   const double bx = 0.5 * (Bn[j * NT + ip] + Bn[j * NT + ip - 1]);
   const double by = 0.5 * (Bn[N2 + jp * NT + i] + Bn[N2 + (jp - 1) * NT + i]);
-  const double q5 = q[5 * N2 + c], q6 = q[6 * N2 + c];
-  q[4 * N2 + c] = q[4 * N2 + c] + 0.5 * ((bx * bx + by * by) - ((q5 * q5) + (q6 * q6)));
+  q[4 * N2 + c] = q4 + 0.5 * ((bx * bx + by * by) - ((q5 * q5) + (q6 * q6)));
   q[5 * N2 + c] = bx;
   q[6 * N2 + c] = by;
+}
+
+template <int NT>
+__device__ inline void bsync_cell(const FieldPtrs& F, const LeafItem L, int last, int c) {
+  constexpr int N2 = NT * NT;
+  double* q = F.f[last ? kU : kUs] + (size_t)L.gs * 8 * N2;
+  sync_cell<NT>(F.f[last ? kBi : kBis] + (size_t)L.gs * 2 * N2, q, c, q[4 * N2 + c], q[5 * N2 + c], q[6 * N2 + c]);
 }
 
 template <int NT>
@@ -353,6 +364,168 @@ __global__ __launch_bounds__(kThreads) void fill_kernel_nv(FillProgram P, FillSe
     set.copy_dst[i] = set.copy_src[i];
   if (counts && (int)blockIdx.x >= counts[kCountChunks]) return;
   fill_chunk_nv<NV0, NV1, NV2, K0, K1, K2>(P, set, NT, blockIdx.x, threadIdx.x, true);
+}
+
+// --------------------------------------------- constrained transport, fused
+// CT2D.cpp:11-124 as two launches where every block a program reads or writes
+// is a leaf (the others run emf, fill, bupdate, fill and bsync as launches of
+// their own): ct_emf_kernel forms the corner EMF and its ghost fill,
+// ct_faces_kernel the face update, its ghost fill and the cell sync.  A fill
+// applied to a value that its source block forms in the same phase is that
+// formula evaluated at the source cell, so a ghost element needs nothing
+// another workgroup writes: one workgroup a leaf, its ring's ops from the
+// table by destination.  What is read at other blocks is not written in the
+// same launch: the EMF goes to a scratch copy (`emf`) from which the second
+// kernel reads, and the faces a stage updates in place (all but the first
+// stage's) are read from a copy the first kernel made (`old`).
+// The five launches took 14.9 us at 16 blocks, 17.8 at 180 and 22.3 at 430, each
+// at the floor of launch and latency; the two take 7.5, 9.6 and 12.2.  They are
+// bound by the chain of dependent loads (leaf, table entry, operands): a loop
+// over the cells with 256 lanes, or a load of the source's level before its
+// cell size, took 18.9 us at 180 blocks.
+struct CtArgs {
+  FieldPtrs F;
+  const LeafItem* leaves;
+  const InstParams* ip;
+  const FillGen* const* gen;
+  const uint64_t* ring;  // [slot][ring_cells]
+  uint32_t version;
+  int step, rk;
+  double* emf;           // [slot][N2]
+  double* old;           // [slot][2][N2]: the updated faces before the stage
+  double* rdx;           // [slot] 1 / dx of the leaf, by ct_emf_kernel for ct_faces_kernel
+  DevError* err;
+};
+
+// one lane a cell: a workgroup's loads are one round of memory latency each
+// (leaf, ring entry, operands)
+template <int NT>
+constexpr int kCtLanes = (NT * NT + 63) / 64 * 64;
+
+template <int NT, int NG>
+__global__ __launch_bounds__(kCtLanes<NT>) void ct_emf_kernel(CtArgs A) {
+  constexpr int N2 = NT * NT, R = ring_cells(NT, NG);
+  const LeafItem L = A.leaves[blockIdx.x];
+  const InstParams& P = A.ip[L.inst];
+  const int last = A.step == A.rk, c = threadIdx.x;
+  if (c == 0) A.rdx[L.gs] = 1. / P.dx[L.lev];
+  if (c >= N2) return;
+  const int r = ring_index(NT, NG, c % NT, c / NT);
+  const uint64_t e = r < 0 ? 0 : A.ring[(size_t)L.gs * R + r];
+  if (A.step > 1) {
+    const double* B = A.F.f[last ? kBi : kBis] + (size_t)L.gs * 2 * N2;
+    double* o = A.old + (size_t)L.gs * 2 * N2;
+    const double b0 = B[c], b1 = B[N2 + c];
+    o[c] = b0;
+    o[N2 + c] = b1;
+  }
+  // the element whose pre-fill value this one takes (injection for restrictions)
+  int64_t gs = L.gs;
+  int a = c;
+  if ((e >> 40) == A.version) {
+    gs = (int64_t)(e & 0xfffffff);
+    a = (int)((e >> 28) & 0x3ff);
+    if (((e >> 38) & 3) == kFillGeneral) {
+      const int64_t ref = A.gen[L.inst][gs].ref[0];
+      gs = ref >> 16;
+      a = (int)(ref & 0xffff);
+    }
+  }
+  double v;
+  if (a % NT < 1 || a < NT) {
+    v = A.F.f[kEMF][(size_t)gs * N2 + a];  // row and column 0 keep what they hold
+  } else {
+    const double* gg5 = A.F.f[kGG] + (size_t)gs * 8 * N2 + 5 * N2;
+    const double* ff6 = A.F.f[kFF] + (size_t)gs * 8 * N2 + 6 * N2;
+    const double g0 = gg5[a - 1], g1 = gg5[a], f0 = ff6[a - NT], f1 = ff6[a];
+    if (P.ct_type != 2) {
+      v = 0.25 * ((g0 + g1) - (f0 + f1));
+    } else {
+      // (the range check of the weight, CT2D.cpp:60, where a block keeps its own
+      // value: a quotient a / (a + b) of magnitudes cannot leave [0, 1])
+      const double psi = ct2_weight<NT>(A.F.f[last ? kU : kUs] + (size_t)gs * 8 * N2, a, P.gamma);
+      if ((psi < 0 || psi > 1) && gs == L.gs && a == c)
+        report(A.err, L.inst, error_key(A.step, kSeqCt | L.nb, 0, c % NT, c / NT, 0, L.nb, kErrCtPsi));
+      v = 0.5 * (1. - psi) * (g0 + g1) - 0.5 * psi * (f0 + f1);
+    }
+  }
+  A.emf[(size_t)L.gs * N2 + c] = v;
+}
+
+// both components of the updated faces at cell c of slot gs
+template <int NT>
+__device__ AMR_INLINE void face_values(const CtArgs& A, double dt, int64_t gs, int c, double* v) {
+  constexpr int N2 = NT * NT;
+  const double* E = A.emf + (size_t)gs * N2;
+  const size_t t2 = (size_t)gs * 2 * N2;
+  const double* Bi = A.F.f[kBi] + t2;
+  const double* old = A.old + t2;  // of the array the stage updates in place
+  const bool last = A.step == A.rk;
+  const double* B = A.step == 1 ? Bi : last ? A.F.f[kBis] + t2 : old;
+  const double* B0 = A.step == 1 ? Bi : last ? old : Bi;  // the step's starting faces
+  const int i = c % NT, j = c / NT;
+  const double e0 = E[c], ej = E[j < NT - 1 ? c + NT : c], ei = E[i < NT - 1 ? c + 1 : c];
+  const double bx = B[c], by = B[N2 + c], b0x = B0[c], b0y = B0[N2 + c];
+  const double rdx = A.rdx[gs];
+  // face_rk: its Bn (RK2's second stage) is the starting value too
+  v[0] = face_rk(A.rk, A.step, bx, b0x, b0x, dt, rdx * (ej - e0));
+  v[1] = face_rk(A.rk, A.step, by, b0y, b0y, dt, -rdx * (ei - e0));
+}
+
+template <int NT, int NG>
+__global__ __launch_bounds__(kCtLanes<NT>) void ct_faces_kernel(CtArgs A) {
+  constexpr int N2 = NT * NT, R = ring_cells(NT, NG);
+  __shared__ double sB[2 * N2];
+  const LeafItem L = A.leaves[blockIdx.x];
+  const double dt = A.ip[L.inst].dt;
+  const int last = A.step == A.rk, c = threadIdx.x;
+  double* q = A.F.f[last ? kU : kUs] + (size_t)L.gs * 8 * N2;
+  double q4 = 0., q5 = 0., q6 = 0.;
+  if (c < N2) {
+    const int r = ring_index(NT, NG, c % NT, c / NT);
+    const uint64_t e = r < 0 ? 0 : A.ring[(size_t)L.gs * R + r];
+    q4 = q[4 * N2 + c];
+    q5 = q[5 * N2 + c];
+    q6 = q[6 * N2 + c];
+    A.F.f[kEMF][(size_t)L.gs * N2 + c] = A.emf[(size_t)L.gs * N2 + c];
+    // the cell itself, the copied one, or the three of a face pair's restriction
+    // (along j for component 0, along i for component 1: restrict_combine)
+    int64_t g0 = L.gs, gx = 0, gy = 0;
+    int a0 = c, ax = 0, ay = 0;
+    bool pair = false;
+    if ((e >> 40) == A.version) {
+      const int op = (int)((e >> 38) & 3);
+      g0 = gx = gy = (int64_t)(e & 0xfffffff);
+      a0 = (int)((e >> 28) & 0x3ff);
+      pair = op != kFillCopy;
+      ax = a0 + NT;
+      ay = a0 + 1;
+      if (op == kFillGeneral) {
+        const FillGen& G = A.gen[L.inst][g0];
+        const int64_t r0 = G.ref[0], rx = G.ref[1], ry = G.ref[2];
+        g0 = r0 >> 16;
+        a0 = (int)(r0 & 0xffff);
+        gx = rx >> 16;
+        ax = (int)(rx & 0xffff);
+        gy = ry >> 16;
+        ay = (int)(ry & 0xffff);
+      }
+    }
+    double v[2];
+    face_values<NT>(A, dt, g0, a0, v);
+    if (pair) {
+      double x[2], y[2];
+      face_values<NT>(A, dt, gx, ax, x);
+      face_values<NT>(A, dt, gy, ay, y);
+      v[0] = restrict_combine(kFillFace, 0, v[0], x[0], 0., 0.);
+      v[1] = restrict_combine(kFillFace, 1, v[1], 0., y[1], 0.);
+    }
+    double* Bn = A.F.f[last ? kBi : kBis] + (size_t)L.gs * 2 * N2;
+    sB[c] = Bn[c] = v[0];
+    sB[N2 + c] = Bn[N2 + c] = v[1];
+  }
+  __syncthreads();
+  if (c < N2) sync_cell<NT>(sB, q, c, q4, q5, q6);
 }
 
 // ------------------------------------------------------ CFL and criteria

@@ -2359,13 +2359,6 @@ void run_stage(amr_ctx* c, int step) {
 
 // CT2D.cpp:11-124
 void run_ct(amr_ctx* c, int step) {
-  // (a captured step's kernels may not hold the table's version: it outlives it)
-  if (c->ct_fused && !c->launch_counts) {
-    Timed tm(c, PF_CT);
-    launch_ct(c->NT, c->ng, c->F, c->d_leaves, c->grid_leaves, c->d_ip, step, c->rk, c->d_inst_gen, c->ring, c->d_err,
-              c->stream);
-    return;
-  }
   {
     Timed tm(c, PF_CT);
     launch_emf(c->NT, c->F, c->d_leaves, c->grid_leaves, c->d_ip, step, c->rk, c->d_err, c->stream, c->launch_counts);
@@ -2380,6 +2373,22 @@ void run_ct(amr_ctx* c, int step) {
     Timed tm(c, PF_CT);
     launch_bsync(c->NT, c->F, c->d_leaves, c->grid_leaves, step == c->rk, c->stream, c->launch_counts);
   }
+}
+
+// the flux fills and the CT of a step's stage
+void run_flux_ct(amr_ctx* c, int step) {
+  // (a captured step's kernels may not hold the table's version: it outlives it)
+  if (c->ct_fused && !c->launch_counts) {
+    Timed tm(c, PF_CT);
+    const int ni = (int)c->inst.size();
+    launch_ct(c->NT, c->ng, c->F, c->d_leaves, c->nleaf, c->d_ip, step, c->rk,
+              {c->d_inst_ops, c->d_inst_gen, c->d_prefix, ni, c->nchunks},
+              {c->d_tail_ops, c->d_inst_gen, c->d_tail_prefix, ni, c->ntail_chunks}, c->ring, c->d_err, c->stream);
+    return;
+  }
+  if (step == 1) run_fill(c, make_set(c, {{kBi, kFillFace}, {kFF, kFillFace}, {kGG, kFillFace}}));
+  else run_fill(c, make_set(c, {{kFF, kFillFace}, {kGG, kFillFace}}));
+  run_ct(c, step);
 }
 
 // waits for the stream (the error records already queued for download) and
@@ -2726,17 +2735,14 @@ int enqueue_step(amr_ctx* c) {
     }
   }
   run_stage(c, 1);
-  run_fill(c, make_set(c, {{kBi, kFillFace}, {kFF, kFillFace}, {kGG, kFillFace}}));
-  run_ct(c, 1);
+  run_flux_ct(c, 1);
   run_fill(c, make_set(c, {{kUs, kFillCell}}));
   run_stage(c, 2);
-  run_fill(c, make_set(c, {{kFF, kFillFace}, {kGG, kFillFace}}));
-  run_ct(c, 2);
+  run_flux_ct(c, 2);
   if (c->rk == 3) {
     run_fill(c, make_set(c, {{kUs, kFillCell}}));
     run_stage(c, 3);
-    run_fill(c, make_set(c, {{kFF, kFillFace}, {kGG, kFillFace}}));
-    run_ct(c, 3);
+    run_flux_ct(c, 3);
   }
   run_fill(c, make_set(c, {{kU, kFillCell}}));
   launch_cfl_regrid(c, nullptr, c->grid_leaves);

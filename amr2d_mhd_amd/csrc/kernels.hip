@@ -361,19 +361,19 @@ void launch_bsync(int NT, const FieldPtrs& F, const LeafItem* leaves, int nleaf,
   AMR_DISPATCH_TILE(NT, (NT == 24 ? 4 : 2), (bsync_kernel<T><<<grid, kThreads, 0, s>>>(F, leaves, last, counts)));
 }
 
-// kernel arguments of the fused CT launches
-static CtArgs ct_args(const FieldPtrs& F, const LeafItem* leaves, const InstParams* ip, int step, int rk,
-                      const FillGen* const* inst_gen, const RingTable& ring, DevError* err) {
-  return CtArgs{F,    leaves,   ip,       inst_gen, ring.entries, ring.version, step,
-                rk,   ring.emf, ring.old, ring.rdx, err};
-}
-
 void launch_ct(int NT, int ng, const FieldPtrs& F, const LeafItem* leaves, int nleaf, const InstParams* ip, int step,
-               int rk, const FillGen* const* inst_gen, const RingTable& ring, DevError* err, hipStream_t s) {
+               int rk, const FillTables& all, const FillTables& tail, const RingTable& ring, DevError* err,
+               hipStream_t s) {
   if (nleaf <= 0) return;
-  const CtArgs A = ct_args(F, leaves, ip, step, rk, inst_gen, ring, err);
-  AMR_DISPATCH_TILE(NT, ng, (ct_emf_kernel<T, G><<<nleaf, kCtLanes<T>, 0, s>>>(A)));
-  AMR_DISPATCH_TILE(NT, ng, (ct_faces_kernel<T, G><<<nleaf, kCtLanes<T>, 0, s>>>(A)));
+  auto program = [](const FillTables& T) { return FillProgram{T.ops, T.gen, T.cprefix, T.ninst}; };
+  CtArgs A{F,        leaves,   ip,       all.gen, ring.entries, ring.version,  step,         rk,
+           ring.emf, ring.old, ring.rdx, err,     nleaf,        program(tail), program(all), 0, 0};
+  A.ntail = step == 1 ? tail.nchunks : 0;  // of Bi
+  AMR_DISPATCH_TILE(NT, ng, (ct_emf_kernel<T, G><<<nleaf + ct_tail_wgs<T>(A.ntail), kCtLanes<T>, 0, s>>>(A)));
+  A.ntail = tail.nchunks;
+  A.nall = all.nchunks;
+  AMR_DISPATCH_TILE(NT, ng, (ct_faces_kernel<T, G><<<nleaf + 2 * (ct_tail_wgs<T>(A.ntail) + ct_flux_wgs<T>(A.nall)),
+                                                     kCtLanes<T>, 0, s>>>(A)));
 }
 
 void launch_ring_table(int NT, int ng, const FillOp* const* inst_ops, const int32_t* cprefix, int ninst, int nchunks,

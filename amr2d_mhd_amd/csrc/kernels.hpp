@@ -106,10 +106,21 @@ struct RingTable {
 // enters the programs of the running instances into the table
 void launch_ring_table(int NT, int ng, const FillOp* const* inst_ops, const int32_t* cprefix, int ninst, int nchunks,
                        const RingTable& ring, hipStream_t s);
-// CT2D.cpp:11-124 with its ghost fills for trees whose programs touch leaves
-// only: two launches
+// a fill program's device tables (launch_fill)
+struct FillTables {
+  const FillOp* const* ops;
+  const FillGen* const* gen;
+  const int32_t* cprefix;
+  int ninst, nchunks;
+};
+// the ghost fills of the fluxes and, in the first stage, of Bi, then
+// CT2D.cpp:11-124 with its own, for trees whose programs (all: whole, tail: their
+// linked tails) touch leaves only: two launches.  Bi comes filled from the step's
+// first fill; of the fluxes of the stages before the last only what a later
+// kernel reads is filled in memory (ct_fill_fluxes).
 void launch_ct(int NT, int ng, const FieldPtrs& F, const LeafItem* leaves, int nleaf, const InstParams* ip, int step,
-               int rk, const FillGen* const* inst_gen, const RingTable& ring, DevError* err, hipStream_t s);
+               int rk, const FillTables& all, const FillTables& tail, const RingTable& ring, DevError* err,
+               hipStream_t s);
 void launch_fill(int NT, const FillOp* const* inst_ops, const FillGen* const* inst_gen, const int32_t* cprefix,
                  int ninst, int nchunks, const FillSet& set, hipStream_t s, const int32_t* counts = nullptr);
 // per-leaf CFL bound min(dx,dy)/lambda and refinement indicator, as pairs

@@ -367,22 +367,29 @@ __global__ __launch_bounds__(kThreads) void fill_kernel_nv(FillProgram P, FillSe
 }
 
 // --------------------------------------------- constrained transport, fused
-// CT2D.cpp:11-124 as two launches where every block a program reads or writes
-// is a leaf (the others run emf, fill, bupdate, fill and bsync as launches of
-// their own): ct_emf_kernel forms the corner EMF and its ghost fill,
-// ct_faces_kernel the face update, its ghost fill and the cell sync.  A fill
-// applied to a value that its source block forms in the same phase is that
-// formula evaluated at the source cell, so a ghost element needs nothing
-// another workgroup writes: one workgroup a leaf, its ring's ops from the
-// table by destination.  What is read at other blocks is not written in the
-// same launch: the EMF goes to a scratch copy (`emf`) from which the second
-// kernel reads, and the faces a stage updates in place (all but the first
-// stage's) are read from a copy the first kernel made (`old`).
-// The five launches took 14.9 us at 16 blocks, 17.8 at 180 and 22.3 at 430, each
-// at the floor of launch and latency; the two take 7.5, 9.6 and 12.2.  They are
-// bound by the chain of dependent loads (leaf, table entry, operands): a loop
-// over the cells with 256 lanes, or a load of the source's level before its
-// cell size, took 18.9 us at 180 blocks.
+// The flux fills of a stage and CT2D.cpp:11-124 as two launches where every block
+// a program reads or writes is a leaf (the others run fill, emf, fill, bupdate,
+// fill and bsync as launches of their own): ct_emf_kernel forms the corner EMF
+// and its ghost fill, ct_faces_kernel the face update, its ghost fill and the
+// cell sync.  A fill applied to a value that its source block forms in the same
+// phase is that formula evaluated at the source cell, so a ghost element needs
+// nothing another workgroup writes: one workgroup a leaf, its ring's ops from the
+// table by destination, and the filled fluxes looked up the same way.  What is
+// read at other blocks is not written in the same launch: the EMF goes to a
+// scratch copy (`emf`) from which the second kernel reads, the faces a stage
+// updates in place (all but the first stage's) are read from a copy the first
+// kernel made (`old`), and workgroups past the leaves' fill in memory what the
+// other kernel reads: Bi with ct_emf_kernel (the first stage's second fill of
+// it: its linked tails), the fluxes with ct_faces_kernel.
+//
+// A stage's fill and CT as six launches, each at the floor of launch and latency,
+// then as these two: 19.4 -> 9.0 us at 16 blocks, 26.1 -> 12.8 at 180, 34.8 ->
+// 19.4 at 430 on average over the two stages.  The leaves' part is bound by the
+// chain of dependent loads (leaf, table entries, operands): a loop over the cells
+// with 256 lanes, or a load of the source's level before its cell size, took 9 us
+// more at 180 blocks.  The last stage's flux fill is bound by the cache lines of
+// the ghost columns (two of 16 elements of each used): 9.4 us of the kernel at
+// 180 blocks against 6.2 in the first stage; with both fields in a lane 12.1.
 struct CtArgs {
   FieldPtrs F;
   const LeafItem* leaves;
@@ -395,16 +402,110 @@ struct CtArgs {
   double* old;           // [slot][2][N2]: the updated faces before the stage
   double* rdx;           // [slot] 1 / dx of the leaf, by ct_emf_kernel for ct_faces_kernel
   DevError* err;
+  int nleaf;
+  FillProgram tail, all;   // the programs' linked tails, and the whole programs
+  int ntail, nall;         // chunks that the launch's workgroups past the leaves run
 };
 
 // one lane a cell: a workgroup's loads are one round of memory latency each
-// (leaf, ring entry, operands)
+// (leaf, ring entry, operands); at least one fill chunk a workgroup
 template <int NT>
-constexpr int kCtLanes = (NT * NT + 63) / 64 * 64;
+constexpr int kCtLanes = (NT * NT + 63) / 64 * 64 < kFillChunk ? kFillChunk : (NT * NT + 63) / 64 * 64;
+template <int NT>
+constexpr int kCtChunks = kCtLanes<NT> / kFillChunk;  // fill chunks an extra workgroup runs
+
+// workgroups of a field's n chunks of linked tails (kept whole) and of unlinked ops
+template <int NT>
+__host__ __device__ constexpr int ct_tail_wgs(int n) { return (n + kCtChunks<NT> - 1) / kCtChunks<NT>; }
+template <int NT>
+__host__ __device__ constexpr int ct_flux_wgs(int n) { return (n * kFillChunk + kCtLanes<NT> - 1) / kCtLanes<NT>; }
+
+// workgroup wg of a field's linked tails
+template <int NT, int NV>
+__device__ inline void ct_fill_tails(const CtArgs& A, double* field, int wg) {
+  const int sub = threadIdx.x / kFillChunk, w = wg * kCtChunks<NT> + sub;
+  FillSet set{};
+  set.base[0] = field;
+  fill_chunk_nv<NV, 0, 0, kFillFace, 0, 0>(A.tail, set, NT, w, threadIdx.x % kFillChunk,
+                                           sub < kCtChunks<NT> && w < A.ntail);
+}
+
+// Workgroup wg of a flux field's unlinked ops, which read nothing that a fill
+// writes, so that any lane may run any of them.  All of them in the last
+// stage; before it memory has to hold only (besides what the linked tails read)
+// the face x = LO of a row (ff) and y = LO of a column (gg), which the next
+// stage's residual of the ghost cells beside them reads: an eighth of the ring in
+// one of the two fields.  The rest is written by the last stage.
+template <int NT, int NG>
+__device__ inline void ct_fill_fluxes(const CtArgs& A, double* field, bool isx, int wg) {
+  constexpr int N2 = NT * NT, LO = NG - 1;
+  const int e = wg * kCtLanes<NT> + threadIdx.x, w = e / kFillChunk;
+  if (w >= A.nall) return;
+  const int q = find_segment(A.all, w), k = w - A.all.cprefix[q];
+  if (k >= A.all.cprefix[q + 1] - A.all.cprefix[q] - (A.tail.cprefix[q + 1] - A.tail.cprefix[q])) return;
+  const FillOp op = A.all.ops[q][k * kFillChunk + e % kFillChunk];
+  if (op.op == kFillNop || (A.step != A.rk && (isx ? op.dst_cell % NT : op.dst_cell / NT) != LO)) return;
+  int64_t e0 = src_ref(op.src, op.src_cell), ei = e0, ej = e0;
+  if (op.op == kFillRestrict) {
+    ei = e0 + 1;
+    ej = e0 + NT;
+  } else if (op.op == kFillGeneral) {
+    const FillGen& g = A.all.gen[q][op.src];
+    e0 = g.ref[0];
+    ej = g.ref[1];
+    ei = g.ref[2];
+  }
+  const bool copy = op.op == kFillCopy;
+  double* o = field + (size_t)op.dst_gs * 8 * N2 + op.dst_cell;
+  const double* p0 = field + (size_t)(e0 >> 16) * 8 * N2 + (e0 & 0xffff);
+  const double* pi = field + (size_t)(ei >> 16) * 8 * N2 + (ei & 0xffff);
+  const double* pj = field + (size_t)(ej >> 16) * 8 * N2 + (ej & 0xffff);
+  double v[8], r[8];  // (a copy's second operand is its first)
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    v[c] = p0[c * N2];
+    r[c] = (c ? pi : pj)[c * N2];
+  }
+#pragma unroll
+  for (int c = 0; c < 8; c++) o[c * N2] = copy ? v[c] : restrict_kind<kFillFace>(c, v[c], r[c], r[c], 0.);
+}
+
+// where element x of slot gs takes its filled value from: offsets into a field of
+// eight components, of one element or of the two of a face pair
+struct FaceRef {
+  size_t o0, o1;
+  bool pair;
+};
+template <int NT, int NG>
+__device__ AMR_INLINE FaceRef face_ref(const CtArgs& A, const FillGen* gen, int64_t gs, int x) {
+  constexpr int N2 = NT * NT, R = ring_cells(NT, NG);
+  const int r = ring_index(NT, NG, x % NT, x / NT);
+  const uint64_t e = r < 0 ? 0 : A.ring[(size_t)gs * R + r];
+  size_t o0 = (size_t)gs * 8 * N2 + x, o1 = o0;
+  bool pair = false;
+  if ((e >> 40) == A.version) {
+    const int op = (int)((e >> 38) & 3);
+    o0 = (size_t)(e & 0xfffffff) * 8 * N2 + ((e >> 28) & 0x3ff);
+    pair = op != kFillCopy;
+    o1 = pair ? o0 + 1 : o0;
+    if (op == kFillGeneral) {
+      const FillGen& G = gen[e & 0xfffffff];
+      const int64_t r0 = G.ref[0], r1 = G.ref[2];
+      o0 = (size_t)(r0 >> 16) * 8 * N2 + (r0 & 0xffff);
+      o1 = (size_t)(r1 >> 16) * 8 * N2 + (r1 & 0xffff);
+    }
+  }
+  return {o0, o1, pair};
+}
+// the filled value of a component other than the first
+__device__ AMR_INLINE double face_filled(const FaceRef& r, double v0, double v1) {
+  return r.pair ? restrict_combine(kFillFace, 1, v0, 0., v1, 0.) : v0;
+}
 
 template <int NT, int NG>
 __global__ __launch_bounds__(kCtLanes<NT>) void ct_emf_kernel(CtArgs A) {
   constexpr int N2 = NT * NT, R = ring_cells(NT, NG);
+  if ((int)blockIdx.x >= A.nleaf) return ct_fill_tails<NT, 2>(A, A.F.f[kBi], blockIdx.x - A.nleaf);
   const LeafItem L = A.leaves[blockIdx.x];
   const InstParams& P = A.ip[L.inst];
   const int last = A.step == A.rk, c = threadIdx.x;
@@ -435,9 +536,15 @@ __global__ __launch_bounds__(kCtLanes<NT>) void ct_emf_kernel(CtArgs A) {
   if (a % NT < 1 || a < NT) {
     v = A.F.f[kEMF][(size_t)gs * N2 + a];  // row and column 0 keep what they hold
   } else {
-    const double* gg5 = A.F.f[kGG] + (size_t)gs * 8 * N2 + 5 * N2;
-    const double* ff6 = A.F.f[kFF] + (size_t)gs * 8 * N2 + 6 * N2;
-    const double g0 = gg5[a - 1], g1 = gg5[a], f0 = ff6[a - NT], f1 = ff6[a];
+    const double* gg5 = A.F.f[kGG] + 5 * N2;
+    const double* ff6 = A.F.f[kFF] + 6 * N2;
+    const FillGen* gen = A.gen[L.inst];
+    const FaceRef rm = face_ref<NT, NG>(A, gen, gs, a - 1), r0 = face_ref<NT, NG>(A, gen, gs, a),
+                  rj = face_ref<NT, NG>(A, gen, gs, a - NT);
+    const double gm0 = gg5[rm.o0], gm1 = gg5[rm.o1], g00 = gg5[r0.o0], g01 = gg5[r0.o1], fj0 = ff6[rj.o0],
+                 fj1 = ff6[rj.o1], f00 = ff6[r0.o0], f01 = ff6[r0.o1];
+    const double g0 = face_filled(rm, gm0, gm1), g1 = face_filled(r0, g00, g01), f0 = face_filled(rj, fj0, fj1),
+                 f1 = face_filled(r0, f00, f01);
     if (P.ct_type != 2) {
       v = 0.25 * ((g0 + g1) - (f0 + f1));
     } else {
@@ -473,9 +580,16 @@ __device__ AMR_INLINE void face_values(const CtArgs& A, double dt, int64_t gs, i
 }
 
 template <int NT, int NG>
-__global__ __launch_bounds__(kCtLanes<NT>) void ct_faces_kernel(CtArgs A) {
+__global__ __launch_bounds__(kCtLanes<NT>) __attribute__((amdgpu_waves_per_eu(7))) void ct_faces_kernel(CtArgs A) {
   constexpr int N2 = NT * NT, R = ring_cells(NT, NG);
   __shared__ double sB[2 * N2];
+  if ((int)blockIdx.x >= A.nleaf) {
+    const int w = blockIdx.x - A.nleaf, n = ct_tail_wgs<NT>(A.ntail);
+    double* field = A.F.f[w & 1 ? kGG : kFF];
+    if (w / 2 < n) ct_fill_tails<NT, 8>(A, field, w / 2);
+    else ct_fill_fluxes<NT, NG>(A, field, !(w & 1), w / 2 - n);
+    return;
+  }
   const LeafItem L = A.leaves[blockIdx.x];
   const double dt = A.ip[L.inst].dt;
   const int last = A.step == A.rk, c = threadIdx.x;

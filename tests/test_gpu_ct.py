@@ -1,12 +1,13 @@
 """Constrained transport with its ghost fills (CT2D.cpp:11-124, boundaryec.cpp,
-boundaryfc.cpp) against the oracle, bitwise, on trees whose levels step by one
-(two launches a stage) and on a tree with a jump of two levels, whose fills
-read blocks that are no leaves (five launches)."""
+boundaryfc.cpp) against the oracle, bitwise: the phase by itself (a launch a
+kernel and a fill), and within steps, on trees whose levels step by one (two
+launches a stage with the flux fills) and on a tree with a jump of two levels,
+whose fills read blocks that are no leaves (the separate launches)."""
 import numpy as np
 import pytest
 
 import oracle as O
-from gpu_util import compare_states, gpu_state, oracle_state
+from gpu_util import FIELD_MAP, compare_states, gpu_state, oracle_state
 
 pytestmark = pytest.mark.gpu
 
@@ -45,15 +46,18 @@ def _merge_next_to_finer(st):
     raise AssertionError("no such father")
 
 
-@pytest.mark.parametrize("jump", [False, True], ids=["one level", "two levels"])
-@pytest.mark.parametrize("cfg", [
+CONFIGS = pytest.mark.parametrize("cfg", [
     dict(ic="rotor", limiter="MC", flux="HLLD", cfl=0.5, nx=16, nghosts=2, maxlevs=5),
     dict(ic="rotor", limiter="MC", flux="HLLC", cfl=0.5, nx=8, nghosts=2, maxlevs=4, ct_type=2),
     dict(ic="rotor", limiter="WENO5", flux="HLLD", cfl=0.4, nx=16, nghosts=4, maxlevs=4, rk_stages=3),
     dict(ic="rotor", limiter="MC", flux="HLLD", cfl=0.4, nx=16, nghosts=2, maxlevs=4, periodic=True, rk_stages=3,
          ct_type=2),
 ], ids=["RK2", "8 cells, type 2", "4 ghosts, RK3", "periodic, RK3, type 2"])
-def test_ct_bitwise(cfg, jump):
+
+
+def _pair(cfg, jump, scale):
+    """GPU and oracle in the same state: six steps of the run, with `jump` on the
+    changed tree, every field scaled cell by cell within 1 +- `scale`."""
     import amr2d_mhd_amd as A
 
     dom = O.Domain(**cfg)
@@ -64,20 +68,42 @@ def test_ct_bitwise(cfg, jump):
     assert _two_level_jumps(st["lp"], st["leafs"]) == 0
     if jump:
         st = _merge_next_to_finer(st)
-    # fluxes and stage states of every slot, the smooth run's scaled cell by cell
     rng = np.random.default_rng(7)
     for f in ("ff", "gg", "Us", "Bis", "Bi", "U"):
-        st[f] = st[f] * rng.uniform(0.98, 1.02, st[f].shape)
+        st[f] = st[f] * rng.uniform(1 - scale, 1 + scale, st[f].shape)
     sim = A.Simulation(cfg)
     sim.init()
     sim.load_state(st)
     dom.set_tree(st["lp"], st["icoord"], st["leafs"])
-    for name, f in (("U", O.U), ("Us", O.US), ("Bi", O.BI), ("Bis", O.BIS), ("ff", O.FF), ("gg", O.GG), ("EMF", O.EMF)):
+    for name, f in FIELD_MAP.items():
         dom.set_field(f, st[name])
+    inf = dom.info()
+    sim.set_time(inf["t"], inf["dt"], inf["dt_next"], inf["count"])
+    return sim, dom
+
+
+@pytest.mark.parametrize("jump", [False, True], ids=["one level", "two levels"])
+@CONFIGS
+def test_ct_bitwise(cfg, jump):
+    sim, dom = _pair(cfg, jump, 0.02)
     dom.locate_bounds()
     for step in range(1, cfg.get("rk_stages", 2) + 1):
         sim.ct(step)
         assert dom.ct(step) == 0
         d = compare_states(gpu_state(sim), oracle_state(dom))
         assert not d, f"after stage {step}: " + "; ".join(d[:4])
+    sim.close()
+
+
+@pytest.mark.parametrize("jump", [False, True], ids=["one level", "two levels"])
+@CONFIGS
+def test_steps_bitwise(cfg, jump):
+    """The first step fills from unfilled ghosts, the second (without a change of
+    the tree) runs its first fill on the programs' tails."""
+    sim, dom = _pair(cfg, jump, 1e-4)
+    for step in range(2):
+        assert dom.step() == 0
+        sim.step()
+        d = compare_states(gpu_state(sim), oracle_state(dom))
+        assert not d, f"after step {step}: " + "; ".join(d[:4])
     sim.close()

@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstdio>
 #include <chrono>
+#include <climits>
 #include <cstdlib>
 #include <new>
 #include <cstring>
@@ -30,6 +31,7 @@
 #include "../../include/amr2d_mhd.h"
 #include "abi_guard.hpp"
 #include "amr_types.hpp"
+#include "fill_pull.hpp"
 #include "flop_count.hpp"
 #include "kernels.hpp"
 #include "physics.hpp"
@@ -461,6 +463,9 @@ struct amr_ctx {
   // serve the current trees when ct_fused
   RingTable ring;
   bool ct_fused = false;
+  int32_t* h_pull = nullptr;  // staging and scratch of the compiles on the device
+  int32_t* d_pull = nullptr;
+  int64_t cap_pull_h = 0, cap_pull = 0;
   char* slot_mem = nullptr;  // the allocation of all per-slot arrays (F, ring)
   // a step launched by step_begin and not yet completed by step_end
   bool in_flight = false;
@@ -2116,6 +2121,124 @@ int for_slot_runs(const Instance& I, int n, const F& f) {
   return 0;
 }
 
+// From how many ring elements in all the programs of changed trees are compiled
+// on the device: 20x20 tiles, 52 leaves (7488 elements) take 55 us on the device
+// and 41 on the host, 100 leaves 57 and 108, 196 leaves 57 and 139
+constexpr int64_t kPullElements = 8192;
+
+// Compiles the programs of those `dirty` instances whose device trees are current
+// and of the form the look-up by destination takes; takes out of `dirty` those
+// that are done (the others the host compiles).
+int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
+  if (!c->regrid_device || dirty.empty()) return 0;
+  const int R = ring_cells(c->NT, c->ng);
+  std::vector<int> todo;
+  int64_t total = 0;
+  for (int q : dirty) {
+    const Instance& I = c->inst[q];
+    if (I.dev_tree_dirty || !pull_form(PullTree{I.lp[0].data(), I.leafs.data()}, I.lastActive)) continue;
+    todo.push_back(q);
+    total += (int64_t)(c->leaf_inst_begin[q + 1] - c->leaf_inst_begin[q]) * R;
+  }
+  if (todo.empty() || total < kPullElements || total > INT32_MAX / 4) return 0;
+  auto chunks = [](int n) { return (n + kFillChunk - 1) / kFillChunk * kFillChunk; };
+  // staging: [instances | leaves, ranks, slots of each], then on the device only
+  // the counters and the scratch
+  const int n = (int)todo.size();
+  const size_t head = std::max((sizeof(PullInst) * n + 3) / 4, (size_t)n * kPullMeta);  // (the counters come back here)
+  size_t words = head, scratch = 0;
+  for (int q : todo) {
+    const Instance& I = c->inst[q];
+    const int nleaf = c->leaf_inst_begin[q + 1] - c->leaf_inst_begin[q];
+    words += nleaf + 2 * I.lastActive;
+    scratch += (size_t)chunks(nleaf * R) * 6;
+  }
+  words = (words + 63) / 64 * 64;
+  if (words > (size_t)c->cap_pull_h) {
+    if (c->h_pull) hipHostFree(c->h_pull);
+    c->h_pull = nullptr;
+    c->cap_pull_h = 0;
+    const size_t cap = words + words / 2;
+    HIPCHK(hipHostMalloc((void**)&c->h_pull, sizeof(int32_t) * cap));
+    c->cap_pull_h = (int64_t)cap;
+  }
+  const size_t need = words + (size_t)n * kPullMeta + scratch;
+  if (need > (size_t)c->cap_pull) {
+    hipFree(c->d_pull);
+    c->d_pull = nullptr;
+    c->cap_pull = 0;
+    HIPCHK(hipMalloc((void**)&c->d_pull, sizeof(int32_t) * (need + need / 2)));
+    c->cap_pull = (int64_t)(need + need / 2);
+  }
+  PullInst* P = (PullInst*)c->h_pull;
+  size_t at = head;  // of the staging words
+  int32_t* meta = c->d_pull + words;
+  int32_t* free_at = meta + (size_t)n * kPullMeta;
+  int max_main = 0, max_ops = 0;
+  for (int t = 0; t < n; t++) {
+    Instance& I = c->inst[todo[t]];
+    const int l0 = c->leaf_inst_begin[todo[t]], nleaf = c->leaf_inst_begin[todo[t] + 1] - l0;
+    PullInst p{};
+    const size_t off = (size_t)c->tree_off[todo[t]];
+    p.lp = c->dtree.lp + 8 * off;
+    p.leafs = c->dtree.leafs + off;
+    p.nleaf = nleaf;
+    p.main = chunks(nleaf * R);
+    p.cap_tail = chunks(p.main / 2 + 8 * kFillChunk);
+    p.cap_gen = p.main / 4 + 1024;
+    p.cap_edges = p.main;
+    if (int e = ensure(I.d_ops, I.cap_ops, p.main + p.cap_tail)) return e;
+    if (int e = ensure(I.d_gen, I.cap_gen, p.cap_gen)) return e;
+    p.ops = I.d_ops;
+    p.gen = I.d_gen;
+    p.meta = meta + (size_t)t * kPullMeta;
+    int32_t* leaf = c->h_pull + at;
+    int32_t* rank = leaf + nleaf;
+    int32_t* gs = rank + I.lastActive;
+    p.leaf = c->d_pull + at;
+    p.rank = p.leaf + nleaf;
+    p.gs = p.rank + I.lastActive;
+    at += nleaf + 2 * (size_t)I.lastActive;
+    std::fill(rank, rank + I.lastActive, -1);
+    for (int l = 0; l < nleaf; l++) {
+      leaf[l] = c->h_leaves[l0 + l].nb;
+      rank[leaf[l]] = l;
+    }
+    std::copy(I.gs.begin(), I.gs.begin() + I.lastActive, gs);
+    p.uf = free_at;
+    p.size = p.uf + p.main;
+    p.linked = p.size + p.main;
+    p.root = p.linked + p.main;
+    p.edges = p.root + p.main;
+    free_at = p.edges + 2 * (size_t)p.main;
+    max_main = std::max(max_main, p.main);
+    max_ops = std::max(max_ops, p.main + p.cap_tail);
+    P[t] = p;
+  }
+  HIPCHK(hipMemcpyAsync(c->d_pull, c->h_pull, sizeof(int32_t) * words, hipMemcpyHostToDevice, c->stream));
+  launch_pull(c->NT, c->ng, (const PullInst*)c->d_pull, n, max_main, max_ops, c->stream);
+  HIPCHK(hipGetLastError());
+  // (the staging's start: the instances are on the device by then)
+  HIPCHK(hipMemcpyAsync(c->h_pull, meta, sizeof(int32_t) * kPullMeta * n, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
+  std::vector<char> done(c->inst.size(), 0);
+  for (int t = 0; t < n; t++) {
+    const int32_t* m = c->h_pull + (size_t)t * kPullMeta;
+    if (m[kPullFlags] & ~kPullSelf) continue;
+    Instance& I = c->inst[todo[t]];
+    const int main = chunks((c->leaf_inst_begin[todo[t] + 1] - c->leaf_inst_begin[todo[t]]) * R);
+    I.nops = main + m[kPullTail];
+    I.ngen = m[kPullGen];
+    for (int k = 0; k < 3; k++) I.op_kinds[k] = m[kPullKinds + k];
+    I.op_kinds[3] = I.nops - I.op_kinds[0] - I.op_kinds[1] - I.op_kinds[2];
+    I.tail_chunk0 = (m[kPullFlags] & kPullSelf) ? 0 : main / kFillChunk;
+    I.prog_dirty = false;
+    done[todo[t]] = 1;
+  }
+  dirty.erase(std::remove_if(dirty.begin(), dirty.end(), [&](int q) { return done[q]; }), dirty.end());
+  return 0;
+}
+
 int rebuild_topology(amr_ctx* c) {
   HostTimed ht(c, PF_HOST_TOPO);
   HIPCHK(hipStreamSynchronize(c->stream));  // previous uploads consumed
@@ -2146,6 +2269,8 @@ int rebuild_topology(amr_ctx* c) {
     dirty.swap(todo);
   }
   const auto t_compile = std::chrono::steady_clock::now();
+  const int ncompile = (int)dirty.size();
+  if (int e = compile_on_device(c, dirty)) return e;  // the rest, below, on the host
   const int hw = (int)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
   int nthreads = (int)std::min<size_t>(dirty.size(), hw);
   if (nthreads < 1) nthreads = 1;
@@ -2171,10 +2296,10 @@ int rebuild_topology(amr_ctx* c) {
     work(0);
     for (auto& x : th) x.join();
   }
-  if (!dirty.empty() && (c->prof_mask & (1u << PF_HOST_COMPILE))) {
+  if (ncompile && (c->prof_mask & (1u << PF_HOST_COMPILE))) {
     c->prof[PF_HOST_COMPILE].ms +=
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_compile).count();
-    c->prof[PF_HOST_COMPILE].launches += (int64_t)dirty.size();
+    c->prof[PF_HOST_COMPILE].launches += ncompile;
   }
   bool failed = false;
   for (size_t q = 0; q < dirty.size(); q++)
@@ -3070,6 +3195,8 @@ int amr_destroy(amr_ctx* c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   if (c->own_stream) hipStreamSynchronize(c->own_stream);
   hipFree(c->slot_mem);
+  hipFree(c->d_pull);
+  if (c->h_pull) hipHostFree(c->h_pull);
   hipFree(c->d_topo);
   if (c->h_topo) hipHostFree(c->h_topo);
   for (auto& I : c->inst) {
@@ -4043,6 +4170,69 @@ int amr_debug_compile_ranges(int NT, int ng, int n, const int32_t* lp, const int
   if (gen) std::memcpy(gen, I.gen.data(), sizeof(FillGen) * std::min<size_t>(I.gen.size(), (size_t)gcap));
   if (ngen) *ngen = (int)I.gen.size();
   return m;
+  AMR_CATCH
+}
+
+// The fill by destination (fill_pull.hpp) of the given tree against the compiled
+// program: every ring element's kind and operands, and which ops read an element
+// that another op writes (the program's linked tail).  Returns the number of
+// elements that differ, -1 if the tree is not of that form, -2 if it does not
+// compile (nested restrictions, which pull_op reports too); counts: ops per kind.
+int amr_debug_pull_fill(int NT, int ng, int n, const int32_t* lp, const int32_t* icoord, const int32_t* leafs,
+                        int64_t* counts) {
+  AMR_TRY
+  Instance I;
+  I.lastActive = n;
+  grow_tree(I, n);
+  for (int nb = 0; nb < n; nb++) {
+    for (int s = 0; s < 8; s++) I.lp[nb][s] = lp[8 * nb + s];
+    I.icoord[nb] = {icoord[2 * nb], icoord[2 * nb + 1]};
+    I.leafs[nb] = (uint8_t)leafs[nb];
+    I.gs.push_back(nb);
+  }
+  const PullTree T{I.lp[0].data(), I.leafs.data()};
+  if (!pull_form(T, n)) return -1;
+  build_schedule(I);
+  FillScratch S;
+  if (compile_instance(I, NT, ng, S)) return -2;
+  const int N2 = NT * NT;
+  std::vector<int> at((size_t)n * N2, -1);
+  const int m = (int)I.ops.size();
+  for (int e = 0; e < m; e++)
+    if (I.ops.data()[e].op != kFillNop) at[(size_t)I.ops.data()[e].dst_gs * N2 + I.ops.data()[e].dst_cell] = e;
+  const int off[4] = {0, NT, 1, NT + 1};
+  int differ = 0;
+  bool self_read = false;
+  std::vector<char> linked((size_t)n * N2, 0);
+  for (int b = 0; b < n; b++)
+    for (int c = 0; c < N2; c++) {
+      const int i = c % NT, j = c / NT, e = at[(size_t)b * N2 + c];
+      const bool ring = ring_index(NT, ng, i, j) >= 0;
+      if (!I.leafs[b] || !ring) {
+        differ += e >= 0;
+        continue;
+      }
+      const PullOp o = pull_op(T, NT, ng, b, i, j);
+      const FillOp op = e < 0 ? FillOp{0, 0, kFillNop, 0, 0, 0} : I.ops.data()[e];
+      bool same = o.op == op.op && !o.nested;
+      counts[o.op]++;
+      for (int q = 0; same && q < o.nref; q++) {
+        const int64_t ref = src_ref(o.nb[q], o.j[q] * NT + o.i[q]);
+        same = ref == (op.op == kFillGeneral ? I.gen[op.src].ref[q]
+                                             : src_ref(op.src, op.src_cell + (op.op == kFillCopy ? 0 : off[q])));
+        if (pull_filled(T, NT, ng, o.nb[q], o.i[q], o.j[q])) {
+          const size_t r = (size_t)o.nb[q] * N2 + o.j[q] * NT + o.i[q];
+          if (r == (size_t)b * N2 + c) self_read = true;
+          else linked[r] = linked[(size_t)b * N2 + c] = 1;
+        }
+      }
+      differ += !same;
+    }
+  if (self_read != (I.tail_chunk0 == 0 && m > 0)) return differ + 1;
+  if (!self_read)
+    for (size_t t = 0; t < at.size(); t++)
+      differ += at[t] >= 0 && (bool)linked[t] != (at[t] / kFillChunk >= I.tail_chunk0);
+  return differ;
   AMR_CATCH
 }
 

@@ -44,7 +44,7 @@ struct Grid {
 
 // -------------------------------------------------------------- forward
 // A stage is two launches.  k_fwd_faces: primitives and face fluxes of a tile
-// of T x T cells, whose lower x and y faces it owns -- the primitives of the
+// of kFx x kFy cells, whose lower x and y faces it owns -- the primitives of the
 // tile and of the three more columns and rows its faces read go through LDS,
 // with the AMR stage's reconstruction, solver and range flags (stage.hpp).
 // k_fwd_update: everything that follows the fluxes, a lane a cell: the stage
@@ -52,22 +52,27 @@ struct Grid {
 // its field averages read (formed twice rather than stored and read back), and
 // the cell sync.  (Primitives, fluxes, update, EMF, faces and sync as a launch
 // each took 70 us a stage at 512 x 512, HLLD, and six launch gaps.)
-// T = 8 (128 lanes, the x faces on the first wavefront, the y faces on the
-// second) up to kSmallN cells a side, where 16 x 16 tiles leave CUs idle;
-// T = 16 (256 lanes, x then y faces) beyond.
-template <int T, int SOLVER>
-__global__ __launch_bounds__(T == 16 ? 256 : 128) __attribute__((amdgpu_waves_per_eu(3))) void k_fwd_faces(
+// Tiles of 16 x 8 with a lane a face, the x faces on the first two wavefronts, the
+// y faces on the others: bound by the flux arithmetic of the three wavefronts a
+// SIMD its registers allow and by how evenly the last of them fill the card.  A
+// step at 150, 300 and 512 cells a side, HLLD: 24.0, 42.0 and 80.5 us; 8 x 8 tiles of
+// 128 lanes 27.7, 43.7 and 87.3, 16 x 16 tiles of 256 lanes (x then y faces) 30.3,
+// 48.2 and 87.2, 32 x 4 tiles 24.2, 41.8 and 78.4 but 31.7 against 20.8 at 100.
+constexpr int kFx = 16, kFy = 8, kFaceLanes = 2 * kFx * kFy;
+
+template <int SOLVER>
+__global__ __launch_bounds__(kFaceLanes) __attribute__((amdgpu_waves_per_eu(3))) void k_fwd_faces(
     Grid G, const double* __restrict__ Q, const double* __restrict__ Bx, const double* __restrict__ By,
     double* __restrict__ W, double* __restrict__ Fx, double* __restrict__ Fy) {
-  constexpr int P = T + 3, VS = P * P, TPB = T == 16 ? 256 : 128;
+  constexpr int P = kFx + 3, VS = P * (kFy + 3);
   __shared__ double sW[8 * VS];
   __shared__ int sFlags;
-  const int tid = threadIdx.x, i0 = blockIdx.x * T, j0 = blockIdx.y * T;
+  const int tid = threadIdx.x, i0 = blockIdx.x * kFx, j0 = blockIdx.y * kFy;
   if (tid == 0) sFlags = 0;
   __syncthreads();
-  for (int c = tid; c < VS; c += TPB) {
+  for (int c = tid; c < VS; c += kFaceLanes) {
     const int ti = c % P, tj = c / P;  // cell (i0 + ti - 2, j0 + tj - 2)
-    const bool ci = ti >= 2 && ti < 2 + T, cj = tj >= 2 && tj < 2 + T;
+    const bool ci = ti >= 2 && ti < 2 + kFx, cj = tj >= 2 && tj < 2 + kFy;
     if (!ci && !cj) continue;  // no face reads the corners
     const size_t e = (size_t)wrap_any(j0 + tj - 2, G.n) * G.n + wrap_any(i0 + ti - 2, G.n);
     double u[8], w[8];
@@ -84,19 +89,16 @@ __global__ __launch_bounds__(T == 16 ? 256 : 128) __attribute__((amdgpu_waves_pe
   }
   __syncthreads();
   const int tile = sFlags;
-  for (int q = tid; q < 2 * T * T; q += TPB) {
-    const int dir = q >= T * T, r = q - dir * T * T;
-    const int ci = r % T, cj = r / T;
-    if (i0 + ci >= G.n || j0 + cj >= G.n) continue;
-    const size_t f = (size_t)(j0 + cj) * G.n + i0 + ci;
-    const double* Wl = sW + (cj + 2 - dir) * P + ci + 1 + dir;  // the cell below the face
-    double fl[8];
-    tile_face_flux<kStageHLLDMuscl>(Wl, VS, dir ? P : 1, kLimMinmod, SOLVER, G.g, 1., dir ? By[f] : Bx[f], tile, dir,
-                                    fl);
-    double* F = dir ? Fy : Fx;
+  const int dir = tid >= kFx * kFy, r = tid - dir * kFx * kFy;
+  const int ci = r % kFx, cj = r / kFx;
+  if (i0 + ci >= G.n || j0 + cj >= G.n) return;
+  const size_t f = (size_t)(j0 + cj) * G.n + i0 + ci;
+  const double* Wl = sW + (cj + 2 - dir) * P + ci + 1 + dir;  // the cell below the face
+  double fl[8];
+  tile_face_flux<kStageHLLDMuscl>(Wl, VS, dir ? P : 1, kLimMinmod, SOLVER, G.g, 1., dir ? By[f] : Bx[f], tile, dir, fl);
+  double* F = dir ? Fy : Fx;
 #pragma unroll
-    for (int k = 0; k < 8; k++) F[k * G.n2 + f] = fl[k];
-  }
+  for (int k = 0; k < 8; k++) F[k * G.n2 + f] = fl[k];
 }
 
 constexpr int kUx = 64, kUy = 4;  // cells of one workgroup of the per-cell kernels
@@ -523,18 +525,11 @@ namespace {
     }                                                                                          \
   } while (0)
 
-constexpr int kSmallN = 256;  // 8 x 8 tiles up to this many cells a side (k_fwd_faces)
-
 template <int SOLVER>
 void launch_faces(amr_adj* a, const double* Q, const double* Bx, const double* By, double* W, hipStream_t s) {
   const unsigned n = (unsigned)a->G.n;
-  if (a->G.n <= kSmallN) {
-    const dim3 grid((n + 7) / 8, (n + 7) / 8);
-    k_fwd_faces<8, SOLVER><<<grid, 128, 0, s>>>(a->G, Q, Bx, By, W, a->Fx, a->Fy);
-  } else {
-    const dim3 grid((n + 15) / 16, (n + 15) / 16);
-    k_fwd_faces<16, SOLVER><<<grid, 256, 0, s>>>(a->G, Q, Bx, By, W, a->Fx, a->Fy);
-  }
+  const dim3 grid((n + kFx - 1) / kFx, (n + kFy - 1) / kFy);
+  k_fwd_faces<SOLVER><<<grid, kFaceLanes, 0, s>>>(a->G, Q, Bx, By, W, a->Fx, a->Fy);
 }
 
 dim3 cell_grid(const Grid& G) { return dim3((unsigned)((G.n + kUx - 1) / kUx), (unsigned)((G.n + kUy - 1) / kUy)); }

@@ -413,19 +413,28 @@ __global__ __launch_bounds__(kT) void k_gather_prim_vjp(Grid G, const double* __
 }
 
 // Fused face reverse + stencil sum + cons->prim reverse over a tile of
-// TW x TH cells, one workgroup of TT lanes: the x faces the tile's cells
-// read (TH rows of TW + 3) are reversed one per lane and leave their
-// stencil contributions in LDS; after a barrier every cell sums its four;
-// the y faces (TH + 3 rows of TW) follow in the same LDS; then the cell
-// adds (dW/dQ)^T Wb to Qb.  Faces next to the tile edge are reversed by both
-// tiles that read them; the normal-B adjoint of a face is added only by the
-// tile that owns the face.  Deterministic: fixed summation order, no
-// atomics.
-template <int TW, int TH, int TT, int SOLVER, int STAGE>
-__global__ __launch_bounds__(TT) void k_stage_vjp(Grid G, const double* __restrict__ W,
+// 16 x 13 cells, one workgroup: the x faces the tile's cells read (13 rows of 19)
+// and the y faces (16 rows of 16) are reversed one per lane and leave their stencil
+// contributions in LDS, from which, after a barrier, every cell sums its eight and
+// adds (dW/dQ)^T Wb to Qb.  Faces next to the tile edge are reversed by both tiles
+// that read them; the normal-B adjoint of a face is added only by the tile that
+// owns the face.  Deterministic: fixed summation order, no atomics.
+// Bound by the solver reverse's arithmetic at the two wavefronts a SIMD its 250
+// registers allow.  Grids of no more tiles than CUs, which would be left half
+// idle, take 512 lanes with the y faces beside the x faces (k_stage_vjp_both);
+// others 256 lanes, the y faces after the x faces in the same LDS, two workgroups
+// a CU (k_stage_vjp).  The reverse of a step, HLLD, as 512 lanes and as 256: 54.6
+// and 63.5 us at 208 tiles (200 cells a side), 86.9 and 84.7 at 285, 220 and 203
+// at 1280 (512 a side).
+constexpr int kVjpFaces = 256, kVjpW = 16, kVjpH = 13;
+constexpr int kVjpBothTiles = 256;  // CUs
+
+template <int SOLVER, int STAGE>
+__global__ __launch_bounds__(kVjpFaces) void k_stage_vjp(Grid G, const double* __restrict__ W,
                                                   const double* __restrict__ Bx, const double* __restrict__ By, RevIn R,
                                                   double* __restrict__ Bnbx, double* __restrict__ Bnby,
                                                   double* __restrict__ Ub, double* __restrict__ Qb) {
+  constexpr int TW = kVjpW, TH = kVjpH, TT = kVjpFaces;
   static_assert(TH * (TW + 3) <= TT && (TH + 3) * TW <= TT, "one face per lane and direction");
   __shared__ double S[8][4][TT];  // [variable][stencil position][face of the tile]
   // x-face sums of the tile's cells, kept in LDS across the y-face reverse
@@ -491,11 +500,53 @@ __global__ __launch_bounds__(TT) void k_stage_vjp(Grid G, const double* __restri
   }
 }
 
-template <int TW, int TH, int TT, int SOLVER, int STAGE>
-void launch_stage_vjp(const Grid& G, const double* W, const double* Bx, const double* By, const RevIn& R, double* Bnbx,
-                      double* Bnby, double* Ub, double* Qb, hipStream_t s) {
-  const dim3 grid((unsigned)((G.n + TW - 1) / TW), (unsigned)((G.n + TH - 1) / TH));
-  k_stage_vjp<TW, TH, TT, SOLVER, STAGE><<<grid, TT, 0, s>>>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb);
+// the same with the y faces beside the x faces
+template <int SOLVER, int STAGE>
+__global__ __launch_bounds__(2 * kVjpFaces) void k_stage_vjp_both(
+    Grid G, const double* __restrict__ W, const double* __restrict__ Bx, const double* __restrict__ By, RevIn R,
+    double* __restrict__ Bnbx, double* __restrict__ Bnby, double* __restrict__ Ub, double* __restrict__ Qb) {
+  constexpr int TW = kVjpW, TH = kVjpH, TT = kVjpFaces;
+  __shared__ double Sx[8][4][TT], Sy[8][4][TT];  // as k_stage_vjp's S, of the x faces and of the y faces
+  const int tid = threadIdx.x, lane = tid % TT;
+  const int i0 = blockIdx.x * TW, j0 = blockIdx.y * TH;
+  double wlb[8], wrb[8];
+  size_t cell[4];
+  if (tid < TT) {
+    const int r = lane / (TW + 3), q = lane % (TW + 3);
+    const int fj = j0 + r, fi = wrap_any(i0 - 1 + q, G.n);
+    if (r < TH && fj < G.n) {
+      face_reverse<0, SOLVER>(G, fi, fj, W, Bx, R, wlb, wrb, cell);
+      if (q >= 1 && q <= TW && i0 - 1 + q < G.n) Bnbx[(size_t)fj * G.n + fi] += wlb[5] + wrb[5];
+      stencil_reverse<0>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
+        for (int s = 0; s < 4; s++) Sx[k][s][lane] = vb[s];
+      });
+    }
+  } else {
+    const int r = lane / TW, q = lane % TW;
+    const int fj = wrap_any(j0 - 1 + r, G.n), fi = i0 + q;
+    if (r < TH + 3 && fi < G.n) {
+      face_reverse<1, SOLVER>(G, fi, fj, W, By, R, wlb, wrb, cell);
+      if (r >= 1 && r <= TH && j0 - 1 + r < G.n) Bnby[(size_t)fj * G.n + fi] += wlb[6] + wrb[6];
+      stencil_reverse<1>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
+        for (int s = 0; s < 4; s++) Sy[k][s][lane] = vb[s];
+      });
+    }
+  }
+  __syncthreads();
+  const int ci = tid % TW, cj = tid / TW, i = i0 + ci, j = j0 + cj;
+  if (tid >= TW * TH || i >= G.n || j >= G.n) return;
+  const size_t c = (size_t)j * G.n + i;
+  double w[8], ub[8], wb[8];
+  for (int k = 0; k < 8; k++) {
+    double a = 0.;
+    for (int s = 0; s < 4; s++) a += Sx[k][s][cj * (TW + 3) + ci + 3 - s];
+    for (int s = 0; s < 4; s++) a += Sy[k][s][(cj + 3 - s) * TW + ci];
+    wb[k] = a;
+    w[k] = W[k * G.n2 + c];
+    ub[k] = 0.;
+  }
+  prim_vjp_w(w, G.g, wb, ub);
+  pass_state<STAGE>(G, R, c, ub, Ub, Qb);
 }
 
 unsigned blocks(size_t n) { return (unsigned)((n + kT - 1) / kT); }
@@ -505,8 +556,8 @@ unsigned blocks(size_t n) { return (unsigned)((n + kT - 1) / kT); }
 struct amr_adj {
   Grid G;
   int solver = kFluxHLLE;  // kFluxHLLE or kFluxHLLD
-  int fused = 1;  // face reverse + gather in one tiled kernel: 1 16x13 tiles of 256 lanes, 2 32x13 tiles of
-                  // 512 lanes; 0: per-face kernels and a gather
+  int fused = 1;  // face reverse + gather in one tiled kernel: 1 by the number of tiles, 2 the y faces after the
+                  // x faces; 0: per-face kernels and a gather
   // forward scratch
   double *Fx, *Fy, *Us, *Uo, *Bxo, *Byo, *tape;
   // adjoint work
@@ -563,10 +614,11 @@ template <int SOLVER, int STAGE>
 void face_and_gather(amr_adj* a, const double* W, const double* Bx, const double* By, const RevIn& R, double* Bnbx,
                      double* Bnby, double* Ub, double* Qb, hipStream_t s) {
   const Grid& G = a->G;
-  if (a->fused == 1) {
-    launch_stage_vjp<16, 13, 256, SOLVER, STAGE>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb, s);
-  } else if (a->fused == 2) {
-    launch_stage_vjp<32, 13, 512, SOLVER, STAGE>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb, s);
+  if (a->fused) {
+    const dim3 grid((unsigned)((G.n + kVjpW - 1) / kVjpW), (unsigned)((G.n + kVjpH - 1) / kVjpH));
+    if (a->fused == 1 && grid.x * grid.y <= kVjpBothTiles)
+      k_stage_vjp_both<SOLVER, STAGE><<<grid, 2 * kVjpFaces, 0, s>>>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb);
+    else k_stage_vjp<SOLVER, STAGE><<<grid, kVjpFaces, 0, s>>>(G, W, Bx, By, R, Bnbx, Bnby, Ub, Qb);
   } else {
     const unsigned b1 = blocks(G.n2);
     k_flux_vjp<0, SOLVER><<<b1, kT, 0, s>>>(G, W, Bx, R, a->Sx, Bnbx);
@@ -738,9 +790,9 @@ int amr_adj_step_vjp(amr_adj* a, const double* U, const double* Bx, const double
   AMR_CATCH
 }
 
-// test hook: 1 = fused tiled face reverse on 16x13 tiles (default), 2 = on
-// 32x13 tiles, 0 = per-face kernels and a separate gather (same derivative,
-// different summation order)
+// test hook: 1 = fused tiled face reverse, its form by the number of tiles
+// (default), 2 = the y faces after the x faces, 0 = per-face kernels and a
+// separate gather (same derivative, different summation order)
 int amr_debug_adj_set_fused(amr_adj* a, int mode) {
   AMR_TRY
   if (!a || mode < 0 || mode > 2) return AMR_ERR_CONFIG;

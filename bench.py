@@ -12,9 +12,8 @@ cost.  One line of JSON carries all three:
                 reduction and regrid.  The run starts from the initial
                 condition; W untimed steps, then exactly K timed steps
                 (defaults: the whole run, 4763 steps).  A zone-update is one
-                interior leaf cell advanced by one step.  The stage-kernel
-                tuner's decisions come from an untimed run, so no trial launch
-                falls in the timed window;
+                interior leaf cell advanced by one step.  An untimed run
+                of the same workload goes before;
   whole_run     (when the window is not the whole run) every step of the run;
   batched_vs_plain  256 seeded rotors of depth 3-6 advanced together against
                 the same instances run one after another (same zone-updates);
@@ -380,9 +379,8 @@ def stage_op_count(at=(1000, 2500, 4000)):
 
 
 def rotor_tuning():
-    """Stage-kernel tuner decisions of the whole rotor run, from an untimed
-    run (the timed runs import them, so no trial launch falls in a timed
-    region)."""
+    """Stage-kernel variants of the whole rotor run per leaf-count bucket, from an
+    untimed run (the timed runs import them)."""
     import amr2d_mhd_amd as A
 
     sim = A.Simulation(ROTOR)
@@ -419,7 +417,6 @@ def rotor_run(warmup, steps, tuning):
     torch.cuda.synchronize()
     nleaf0 = sim.info()["nleaf"]
     fill0 = sim.fill_stats() if FILL_STATS else None
-    tuner0 = sim.stage_tuning()
     sim.profile(("stage",), stride=EVENT_STRIDE)
     t0 = time.perf_counter()
     n, zu = sim.run(steps)
@@ -428,13 +425,11 @@ def rotor_run(warmup, steps, tuning):
     prof = sim.profile_read()
     info = sim.info()
     fill1 = sim.fill_stats() if FILL_STATS else None
-    # a trial launch changes its bucket's per-variant timings
-    trial_buckets = sorted(b for b, v in sim.stage_tuning().items() if tuner0.get(b) != v)
     sim.close()
     stage_ms, stage_n = prof["stage"]
     return dict(steps=n, zone_updates=zu, seconds=secs, value=zu / secs, ms_per_step=secs / n * 1e3,
                 t_reached=info["t"], leaves_at_start=nleaf0, leaves_at_end=info["nleaf"],
-                stage_ms=stage_ms, stage_launches=stage_n, trial_buckets=trial_buckets,
+                stage_ms=stage_ms, stage_launches=stage_n,
                 fill_program=dict(window_start=fill0, window_end=fill1) if FILL_STATS else None)
 
 
@@ -536,8 +531,7 @@ def main():
                    "regrid": ("on the device (markref, critneighup/down, updatelpup/down per instance; the host "
                               "reads back the op list)") if REGRID_DEVICE else "on the host (per-leaf indicators downloaded)",
                    **({"fill_program": win["fill_program"]} if win["fill_program"] else {}),
-                   "stage_tuner": "decisions imported from an untimed run; leaf-count buckets that ran "
-                                  f"trial launches inside the timed window: {win['trial_buckets']}"},
+                   "stage_tuner": "variants by leaf count, imported from an untimed run"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": STAGE_TRAFFIC_BYTES_PER_ZONE * zones_per_launch,

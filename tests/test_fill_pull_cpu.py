@@ -18,7 +18,7 @@ def _check(NT, ng, lp, ic, lf):
 
 
 @pytest.mark.parametrize("cfg,tiles,steps", [
-    (dict(ic="BWx", limiter="MC", flux="RUSA", cfl=0.4, maxlevs=4), [(20, 2), (12, 2), (24, 4)], 150),
+    (dict(ic="BWx", limiter="MC", flux="RUSA", cfl=0.4, maxlevs=4), [(20, 2), (12, 2), (24, 4)], 300),
     (dict(ic="rotor", limiter="MC", flux="HLLD", cfl=0.5, maxlevs=5), [(20, 2), (24, 4)], 80),
     (dict(ic="rotor", limiter="MC", flux="HLLD", cfl=0.4, maxlevs=4, periodic=True), [(20, 2), (12, 2), (24, 4)], 60),
     (dict(ic="OT", limiter="MC", flux="HLLD", cfl=0.4, maxlevs=5, periodic=True), [(24, 4)], 20),

@@ -383,6 +383,12 @@ void launch_ring_table(int NT, int ng, const FillOp* const* inst_ops, const int3
   ring_table_kernel<<<nchunks, kFillChunk, 0, s>>>(P, NT, ng, ring.entries, ring.version);
 }
 
+// Up to this many chunks the fills of U (and Bi) take two components a workgroup
+// (fill_parts_kernel): a workgroup a chunk leaves CUs idle and its loads in one
+// queue.  Both ways: tails of 9 chunks 5.9 -> 4.0 us, U at 120 chunks 6.0 -> 5.3, at
+// 256 to 319 9.9 -> 9.1, at 320 to 399 10.2 and 10.2, at 400 to 511 11.1 and 11.4.
+constexpr int kFillPartsChunks = 320;
+
 void launch_fill(int NT, const FillOp* const* inst_ops, const FillGen* const* inst_gen, const int32_t* cprefix,
                  int ninst, int nchunks, const FillSet& set, hipStream_t s, const int32_t* counts) {
   static_assert(kFillChunk == kThreads, "one workgroup per fill chunk");
@@ -391,7 +397,11 @@ void launch_fill(int NT, const FillOp* const* inst_ops, const FillGen* const* in
   const int a = set.nv[0], b = set.n > 1 ? set.nv[1] : 0, c = set.n > 2 ? set.nv[2] : 0;
   const int ka = set.kind[0], kb = set.n > 1 ? set.kind[1] : -1, kc = set.n > 2 ? set.kind[2] : -1;
   constexpr int C = kFillCell, F = kFillFace, E = kFillEdge;
-  if (set.n == 1 && a == 8 && ka == C) fill_kernel_nv<8, 0, 0, C, 0, 0><<<nchunks, kThreads, 0, s>>>(P, set, NT, counts);
+  if (nchunks <= kFillPartsChunks && set.n == 1 && a == 8 && ka == C)
+    fill_parts_kernel<0><<<dim3(nchunks, 4), kThreads, 0, s>>>(P, set, NT, counts);
+  else if (nchunks <= kFillPartsChunks && set.n == 2 && a == 8 && b == 2 && ka == C && kb == F)
+    fill_parts_kernel<2><<<dim3(nchunks, 5), kThreads, 0, s>>>(P, set, NT, counts);
+  else if (set.n == 1 && a == 8 && ka == C) fill_kernel_nv<8, 0, 0, C, 0, 0><<<nchunks, kThreads, 0, s>>>(P, set, NT, counts);
   else if (set.n == 1 && a == 2 && ka == F)
     fill_kernel_nv<2, 0, 0, F, 0, 0><<<nchunks, kThreads, 0, s>>>(P, set, NT, counts);
   else if (set.n == 1 && a == 1 && ka == E)

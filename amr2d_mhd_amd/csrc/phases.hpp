@@ -357,6 +357,60 @@ __device__ inline void fill_chunk_nv(const FillProgram& P, const FillSet& set, i
 // field sets of the step (engine.cpp) with their combine kinds: {U, Bi},
 // {Bi, ff, gg}, {ff, gg}, one cell field, one face field, EMF; any other set
 // takes the per-field path
+// {U} or {U, Bi} (NB = 2) with a chunk's components over four workgroups, two each,
+// and Bi's in a fifth (blockIdx.y)
+template <int NB>
+__global__ __launch_bounds__(kThreads) void fill_parts_kernel(FillProgram P, FillSet set, int NT,
+                                                              const int32_t* __restrict__ counts) {
+  if (blockIdx.y == 0)
+    for (int i = blockIdx.x * kThreads + threadIdx.x; i < set.copy_words; i += gridDim.x * kThreads)
+      set.copy_dst[i] = set.copy_src[i];
+  if (counts && (int)blockIdx.x >= counts[kCountChunks]) return;
+  const int w = blockIdx.x, q = find_segment(P, w);
+  const FillOp op = P.ops[q][(w - P.cprefix[q]) * kFillChunk + threadIdx.x];
+  const int N2 = NT * NT;
+  int64_t e[4] = {src_ref(op.src, op.src_cell), 0, 0, 0};
+  if (op.op == kFillRestrict) {
+    e[1] = e[0] + NT;
+    e[2] = e[0] + 1;
+    e[3] = e[0] + 1 + NT;
+  } else if (op.op == kFillGeneral) {
+    const FillGen& g = P.gen[q][op.src];
+#pragma unroll
+    for (int t = 0; t < 4; t++) e[t] = g.ref[t];
+  }
+  auto run = [&](int nv, int k0, double* base, auto combine) {
+    constexpr int N = 2;
+    double v[N];
+    if (op.op != kFillNop) {
+      const double* p0 = base + ((size_t)(e[0] >> 16) * nv + k0) * N2 + (e[0] & 0xffff);
+      if (op.op == kFillCopy) {
+#pragma unroll
+        for (int k = 0; k < N; k++) v[k] = p0[(size_t)k * N2];
+      } else {
+        const double* p1 = base + ((size_t)(e[1] >> 16) * nv + k0) * N2 + (e[1] & 0xffff);
+        const double* p2 = base + ((size_t)(e[2] >> 16) * nv + k0) * N2 + (e[2] & 0xffff);
+        const double* p3 = base + ((size_t)(e[3] >> 16) * nv + k0) * N2 + (e[3] & 0xffff);
+#pragma unroll
+        for (int k = 0; k < N; k++)
+          v[k] = combine(k, p0[(size_t)k * N2], p1[(size_t)k * N2], p2[(size_t)k * N2], p3[(size_t)k * N2]);
+      }
+    }
+    __syncthreads();  // every read of the chunk precedes every write
+    if (op.op != kFillNop) {
+      double* o = base + ((size_t)op.dst_gs * nv + k0) * N2 + op.dst_cell;
+#pragma unroll
+      for (int k = 0; k < N; k++) o[(size_t)k * N2] = v[k];
+    }
+  };
+  if (NB && blockIdx.y == 4)
+    run(2, 0, set.base[1],
+        [](int k, double a, double b, double c, double d) { return restrict_kind<kFillFace>(k, a, b, c, d); });
+  else
+    run(8, blockIdx.y * 2, set.base[0],
+        [](int k, double a, double b, double c, double d) { return restrict_kind<kFillCell>(k, a, b, c, d); });
+}
+
 template <int NV0, int NV1, int NV2, int K0, int K1, int K2>
 __global__ __launch_bounds__(kThreads) void fill_kernel_nv(FillProgram P, FillSet set, int NT,
                                                            const int32_t* __restrict__ counts) {

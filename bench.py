@@ -51,19 +51,18 @@ ROTOR_STEPS = 4763  # steps of the full rotor run to t = 0.295 without FMA contr
 # Us and U (128 B) and face B (16 B), writes U (64 B) -> mean 176 B
 STAGE_BYTES_PER_ZONE = 176.0
 # HBM bytes per leaf zone one stage launch actually moves, from rocprofv3 FETCH_SIZE
-# (x2.0, copy-calibrated) + WRITE_SIZE (x1.0) over the 9526 stage launches of the
-# whole run, with the variants the tuner picks: profiles/stage_traffic_rotor_lv5.md
-# (311.5 read + 286.5 written)
-STAGE_TRAFFIC_BYTES_PER_ZONE = 598.0
+# (x2.0, copy-calibrated) + WRITE_SIZE (x1.0) over the stage launches of the
+# whole run: profiles/stage_traffic_rotor_lv5.md (341.0 read + 271.8 written)
+STAGE_TRAFFIC_BYTES_PER_ZONE = 612.8
 HBM_PEAK_GBS = 8000.0
 # FP64 FLOPs one stage launch executes per leaf zone: rocprofv3 counters
 # (SQ_INSTS_VALU_FLOPS_FP64 + SQ_INSTS_VALU_FLOPS_FP64_TRANS) x 64 lanes per
 # dispatch / (256 x leaves), median over the stage dispatches of this workload
-# (profiles/fp64_flops_rotor_lv5_adjoint_512.md, 768-lane variant specialised
-# to HLLD/MUSCL); FP64 division and sqrt count with their full instruction
+# (profiles/fp64_flops_rotor_lv5_adjoint_512.md, the kernels specialised to
+# HLLD/MUSCL: 2709 with 768 lanes a leaf, 2699 with 256); FP64 division and sqrt count with their full instruction
 # sequences, a wave counts every branch any of its lanes takes, and the whole
 # 20x20 tile is computed
-STAGE_FP64_FLOPS_PER_ZONE = 3956.0
+STAGE_FP64_FLOPS_PER_ZONE = 2705.0
 FP64_PEAK_TFLOPS = 78.6
 
 

@@ -2,10 +2,11 @@
 that path (engine.cpp, kPullElements), in lockstep with the oracle, bitwise, on
 every tile form, at mirror and periodic boundaries, and several instances of
 different trees in one context."""
+import numpy as np
 import pytest
 
 import oracle as O
-from gpu_util import compare_states, gpu_state, oracle_state
+from gpu_util import FIELD_MAP, compare_states, gpu_state, oracle_state
 
 pytestmark = pytest.mark.gpu
 
@@ -48,4 +49,37 @@ def test_runs_bitwise(steps, cfgs):
                 diff = compare_states(gpu_state(sim, q), oracle_state(d))
                 assert not diff, f"instance {q} after step {step}: " + "; ".join(diff[:4])
     assert changed > 1
+    sim.close()
+
+
+@pytest.mark.parametrize("cfg,steps", [
+    (dict(ic="BWx", limiter="MC", flux="HLLE", cfl=0.4, nx=16, nghosts=2, maxlevs=2), 1),
+    (dict(ic="rotor", limiter="MC", flux="HLLD", cfl=0.5, nx=8, nghosts=2, maxlevs=6), 6),
+    (dict(ic="OT", limiter="MC", flux="HLLD", cfl=0.4, nx=16, nghosts=2, maxlevs=5, periodic=True), 4),
+    (dict(ic="OT", limiter="WENO5", flux="HLLD", cfl=0.4, nx=16, nghosts=4, maxlevs=4, periodic=True), 2),
+], ids=["16 leaves", "12x12", "over 320 chunks", "24x24"])
+def test_cell_fill_bitwise(cfg, steps):
+    """The fill of U by itself, random values in every element: programs below and
+    above the chunk count to which a chunk's components go to several workgroups,
+    restrictions, copies and linked (stale-read) ops."""
+    import amr2d_mhd_amd as A
+
+    dom = O.Domain(**cfg)
+    assert dom.init() == 0
+    for _ in range(steps):
+        assert dom.step() == 0
+    st = oracle_state(dom)
+    rng = np.random.default_rng(3)
+    st["U"] = rng.standard_normal(st["U"].shape)
+    sim = A.Simulation(cfg)
+    sim.init()
+    sim.load_state(st)
+    for name, f in FIELD_MAP.items():
+        dom.set_field(f, st[name])
+    dom.locate_bounds()
+    for _ in range(2):
+        sim.fill("U", "cell")
+        assert dom.fill(O.U, O.FILL_CC) == 0
+        d = compare_states(gpu_state(sim), oracle_state(dom), ("U",))
+        assert not d, "; ".join(d[:4])
     sim.close()

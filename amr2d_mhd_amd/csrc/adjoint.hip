@@ -188,16 +188,21 @@ Tape tape_at(double* base, size_t n2) {
 
 // edge states of one face: x faces (dir 0) take Bx as the normal component,
 // y faces (dir 1) By, and are returned in the rotated frame (swap_xy)
-__device__ inline void face_states(const Grid& G, const double* W, const double* Bn, int dir, int i, int j,
-                                   double* wl, double* wr, size_t* cell) {
+template <bool FAST>
+__device__ AMR_INLINE void face_states(Rev<FAST>& A, const Grid& G, const double* W, const double* Bn, int dir, int i,
+                                       int j, double* wl, double* wr, size_t* cell) {
+#pragma unroll
   for (int s = 0; s < 4; s++) {
     const int o = s - 2;
     cell[s] = dir == 0 ? (size_t)j * G.n + wrap(i + o, G.n) : (size_t)wrap(j + o, G.n) * G.n + i;
   }
+#pragma unroll
   for (int k = 0; k < 8; k++) {
     double v[4];
+    if (k == 5 + dir) continue;
+#pragma unroll
     for (int s = 0; s < 4; s++) v[s] = W[k * G.n2 + cell[s]];
-    recon_minmod(v, wl[k], wr[k]);
+    recon_minmod(A, v, wl[k], wr[k]);
   }
   const double b = Bn[(size_t)j * G.n + i];
   if (dir == 0) {
@@ -284,13 +289,20 @@ __device__ inline double presync(const Grid& G, const RevIn& R, int k, size_t c)
 
 // adjoints of the fluxes through the lower face of cell (i, j) in direction
 // DIR: from the update's residual and from the EMF (components 6 of x, 5 of y)
-template <int DIR>
-__device__ AMR_INLINE void flux_adjoint(const Grid& G, const RevIn& R, int i, int j, double* fb) {
+template <int DIR, bool FAST>
+__device__ AMR_INLINE void flux_adjoint(Rev<FAST>& A, const Grid& G, const RevIn& R, int i, int j, double* fb) {
   const size_t f = (size_t)j * G.n + i;
   const size_t l = DIR == 0 ? (size_t)j * G.n + wrap(i - 1, G.n) : (size_t)wrap(j - 1, G.n) * G.n + i;
-  const RDen dx = rden(G.dx);
+  A.note_den(G.dx);
+  const Den<FAST> dx = A.den(G.dx);
 #pragma unroll
-  for (int k = 0; k < 8; k++) fb[k] = quot(R.s * presync(G, R, k, l) - R.s * presync(G, R, k, f), dx);
+  for (int k = 0; k < 8; k++) fb[k] = R.s * presync(G, R, k, l) - R.s * presync(G, R, k, f);
+#pragma unroll
+  for (int k = 0; k < 8; k += 2) {
+    A.note(fb[k], fb[k + 1]);
+    fb[k] = A.over(fb[k], dx);
+    fb[k + 1] = A.over(fb[k + 1], dx);
+  }
   if (DIR == 0) fb[6] -= 0.25 * (R.Eb[f] + R.Eb[(size_t)wrap(j + 1, G.n) * G.n + i]);
   else fb[5] += 0.25 * (R.Eb[f] + R.Eb[(size_t)j * G.n + wrap(i + 1, G.n)]);
 }
@@ -311,26 +323,54 @@ __device__ inline void pass_state(const Grid& G, const RevIn& R, size_t c, const
   }
 }
 
-// per-face reverse of reconstruction + HLLE for the faces of one direction
-// (blockIdx.y): stencil contributions S[s][k] (s = cells i-2 .. i+1 along the
-// face normal) and the normal-B adjoint (accumulated into Bnb)
-// reverse of reconstruction + HLLE at one face (i, j) of direction DIR: the
-// adjoints (wlb, wrb) of its two edge states in the grid frame, the stencil
-// cells (i-2 .. i+1 along the normal) and the normal-B adjoint
-template <int DIR, int SOLVER>
-__device__ inline void face_reverse(const Grid& G, int i, int j, const double* __restrict__ W,
-                                    const double* __restrict__ Bn, const RevIn& R, double* wlb, double* wrb,
-                                    size_t* cell) {
+// Reverse of reconstruction + flux at one face (i, j) of direction DIR: the
+// adjoints (wlb, wrb) of its two edge states in the grid frame.  Returns whether
+// they hold (Rev).
+template <int DIR, int SOLVER, bool FAST>
+__device__ AMR_INLINE bool face_reverse_as(const Grid& G, int i, int j, const double* __restrict__ W,
+                                           const double* __restrict__ Bn, const RevIn& R, double* wlb, double* wrb) {
+  Rev<FAST> A;
   double wl[8], wr[8], fb[8];
-  face_states(G, W, Bn, DIR, i, j, wl, wr, cell);
-  flux_adjoint<DIR>(G, R, i, j, fb);
+  size_t cell[4];
+  face_states(A, G, W, Bn, DIR, i, j, wl, wr, cell);
+  flux_adjoint<DIR>(A, G, R, i, j, fb);
   for (int k = 0; k < 8; k++) wlb[k] = wrb[k] = 0.;
   if (DIR) swap_xy(fb);  // adjoint of the output swap
-  if (SOLVER == kFluxHLLD) hlld_vjp(wl, wr, G.g, fb, wlb, wrb);
-  else hlle_vjp(wl, wr, G.g, fb, wlb, wrb);
+  if (SOLVER == kFluxHLLD) hlld_vjp(A, wl, wr, G.g, fb, wlb, wrb);
+  else hlle_vjp(A, wl, wr, G.g, fb, wlb, wrb);
   if (DIR) {
     swap_xy(wlb);  // adjoint of the input swap
     swap_xy(wrb);
+  }
+  return A.ok();
+}
+
+// the same with plain quotients, into out[q * stride], q = 0 .. 15 (wlb, then wrb);
+// out of line, for its registers (inlined, the kernels below spilled 335 of them)
+template <int DIR, int SOLVER>
+__device__ __attribute__((noinline)) void face_reverse_plain(Grid G, int i, int j, const double* W, const double* Bn,
+                                                             RevIn R, double* out, size_t stride) {
+  double wlb[8], wrb[8];
+  face_reverse_as<DIR, SOLVER, false>(G, i, j, W, Bn, R, wlb, wrb);
+  for (int k = 0; k < 8; k++) {
+    out[k * stride] = wlb[k];
+    out[(8 + k) * stride] = wrb[k];
+  }
+}
+
+// the same with the FAST quotients where they are exact; also the stencil cells
+// (i-2 .. i+1 along the normal).  mem, stride: as face_reverse_plain's out, this
+// lane's own memory
+template <int DIR, int SOLVER>
+__device__ AMR_INLINE void face_reverse(const Grid& G, int i, int j, const double* __restrict__ W,
+                                        const double* __restrict__ Bn, const RevIn& R, double* mem, size_t stride,
+                                        double* wlb, double* wrb, size_t* cell) {
+  if (!face_reverse_as<DIR, SOLVER, true>(G, i, j, W, Bn, R, wlb, wrb)) {
+    face_reverse_plain<DIR, SOLVER>(G, i, j, W, Bn, R, mem, stride);
+    for (int k = 0; k < 8; k++) {
+      wlb[k] = mem[k * stride];
+      wrb[k] = mem[(8 + k) * stride];
+    }
   }
   // Recompute the stencil cells from opaque copies of (i, j) rather than
   // keep the four 64-bit offsets alive across the solver reverse.
@@ -357,7 +397,13 @@ __device__ inline void stencil_reverse(const Grid& G, const double* __restrict__
     if (k != nc) {
       double v[4];
       for (int s = 0; s < 4; s++) v[s] = Wr[k * G.n2 + cell[s]];
-      recon_minmod_vjp(v, wlb[k], wrb[k], vb);
+      Rev<true> A;
+      recon_minmod_vjp(A, v, wlb[k], wrb[k], vb);
+      if (!A.ok()) {
+        Rev<false> plain;
+        for (int s = 0; s < 4; s++) vb[s] = 0.;
+        recon_minmod_vjp(plain, v, wlb[k], wrb[k], vb);
+      }
     }
     out(k, vb);
   }
@@ -370,7 +416,7 @@ __device__ inline void flux_vjp_face(const Grid& G, size_t f, const double* __re
   const int i = (int)(f % G.n), j = (int)(f / G.n);
   double wlb[8], wrb[8];
   size_t cell[4];
-  face_reverse<DIR, SOLVER>(G, i, j, W, Bn, R, wlb, wrb, cell);
+  face_reverse<DIR, SOLVER>(G, i, j, W, Bn, R, S + f, G.n2, wlb, wrb, cell);
   constexpr int nc = DIR ? 6 : 5;
   Bnb[f] += wlb[nc] + wrb[nc];
   stencil_reverse<DIR>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
@@ -408,7 +454,8 @@ __global__ __launch_bounds__(kT) void k_gather_prim_vjp(Grid G, const double* __
     w[k] = W[k * G.n2 + c];
     ub[k] = 0.;
   }
-  prim_vjp_w(w, G.g, wb, ub);
+  Rev<false> plain;
+  prim_vjp_w(plain, w, G.g, wb, ub);
   pass_state<STAGE>(G, R, c, ub, Ub, Qb);
 }
 
@@ -453,7 +500,7 @@ __global__ __launch_bounds__(kVjpFaces) void k_stage_vjp(Grid G, const double* _
     if (fj < G.n) {
       double wlb[8], wrb[8];
       size_t cell[4];
-      face_reverse<0, SOLVER>(G, fi, fj, W, Bx, R, wlb, wrb, cell);
+      face_reverse<0, SOLVER>(G, fi, fj, W, Bx, R, &S[0][0][tid], TT, wlb, wrb, cell);
       if (q >= 1 && q <= TW && i0 - 1 + q < G.n) Bnbx[(size_t)fj * G.n + fi] += wlb[5] + wrb[5];
       stencil_reverse<0>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
         for (int s = 0; s < 4; s++) S[k][s][tid] = vb[s];
@@ -477,7 +524,7 @@ __global__ __launch_bounds__(kVjpFaces) void k_stage_vjp(Grid G, const double* _
     if (fi < G.n) {
       double wlb[8], wrb[8];
       size_t cell[4];
-      face_reverse<1, SOLVER>(G, fi, fj, W, By, R, wlb, wrb, cell);
+      face_reverse<1, SOLVER>(G, fi, fj, W, By, R, &S[0][0][tid], TT, wlb, wrb, cell);
       if (r >= 1 && r <= TH && j0 - 1 + r < G.n) Bnby[(size_t)fj * G.n + fi] += wlb[6] + wrb[6];
       stencil_reverse<1>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
         for (int s = 0; s < 4; s++) S[k][s][tid] = vb[s];
@@ -495,7 +542,8 @@ __global__ __launch_bounds__(kVjpFaces) void k_stage_vjp(Grid G, const double* _
       w[k] = W[k * G.n2 + c];
       ub[k] = 0.;
     }
-    prim_vjp_w(w, G.g, wb, ub);
+    Rev<false> plain;
+    prim_vjp_w(plain, w, G.g, wb, ub);
     pass_state<STAGE>(G, R, c, ub, Ub, Qb);
   }
 }
@@ -515,7 +563,7 @@ __global__ __launch_bounds__(2 * kVjpFaces) void k_stage_vjp_both(
     const int r = lane / (TW + 3), q = lane % (TW + 3);
     const int fj = j0 + r, fi = wrap_any(i0 - 1 + q, G.n);
     if (r < TH && fj < G.n) {
-      face_reverse<0, SOLVER>(G, fi, fj, W, Bx, R, wlb, wrb, cell);
+      face_reverse<0, SOLVER>(G, fi, fj, W, Bx, R, &Sx[0][0][lane], TT, wlb, wrb, cell);
       if (q >= 1 && q <= TW && i0 - 1 + q < G.n) Bnbx[(size_t)fj * G.n + fi] += wlb[5] + wrb[5];
       stencil_reverse<0>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
         for (int s = 0; s < 4; s++) Sx[k][s][lane] = vb[s];
@@ -525,7 +573,7 @@ __global__ __launch_bounds__(2 * kVjpFaces) void k_stage_vjp_both(
     const int r = lane / TW, q = lane % TW;
     const int fj = wrap_any(j0 - 1 + r, G.n), fi = i0 + q;
     if (r < TH + 3 && fi < G.n) {
-      face_reverse<1, SOLVER>(G, fi, fj, W, By, R, wlb, wrb, cell);
+      face_reverse<1, SOLVER>(G, fi, fj, W, By, R, &Sy[0][0][lane], TT, wlb, wrb, cell);
       if (r >= 1 && r <= TH && j0 - 1 + r < G.n) Bnby[(size_t)fj * G.n + fi] += wlb[6] + wrb[6];
       stencil_reverse<1>(G, W, cell, wlb, wrb, [&](int k, const double* vb) {
         for (int s = 0; s < 4; s++) Sy[k][s][lane] = vb[s];
@@ -545,7 +593,8 @@ __global__ __launch_bounds__(2 * kVjpFaces) void k_stage_vjp_both(
     w[k] = W[k * G.n2 + c];
     ub[k] = 0.;
   }
-  prim_vjp_w(w, G.g, wb, ub);
+  Rev<false> plain;
+  prim_vjp_w(plain, w, G.g, wb, ub);
   pass_state<STAGE>(G, R, c, ub, Ub, Qb);
 }
 
@@ -804,7 +853,8 @@ int amr_debug_adj_set_fused(amr_adj* a, int mode) {
 // host entry points of the pointwise reverse pieces (CPU tests)
 void amr_debug_hlle_vjp(const double* wL, const double* wR, double gamma, const double* fb, double* wLb, double* wRb) {
   for (int k = 0; k < 8; k++) wLb[k] = wRb[k] = 0.;
-  hlle_vjp(wL, wR, gamma, fb, wLb, wRb);
+  Rev<false> A;
+  hlle_vjp(A, wL, wR, gamma, fb, wLb, wRb);
 }
 
 void amr_debug_hlle(const double* wL, const double* wR, double gamma, double* f) { flux_hlle(wL, wR, gamma, f); }
@@ -813,7 +863,8 @@ void amr_debug_hlle(const double* wL, const double* wR, double gamma, double* f)
 void amr_debug_hlld_vjp(const double* wL, const double* wR, double gamma, const double* fb, double* wLb, double* wRb,
                         double* f) {
   for (int k = 0; k < 8; k++) wLb[k] = wRb[k] = 0.;
-  hlld_vjp(wL, wR, gamma, fb, wLb, wRb, f);
+  Rev<false> A;
+  hlld_vjp(A, wL, wR, gamma, fb, wLb, wRb, f);
 }
 
 void amr_debug_hlld(const double* wL, const double* wR, double gamma, double* f) {
@@ -827,10 +878,11 @@ void amr_debug_hlld(const double* wL, const double* wR, double gamma, double* f)
 void amr_debug_side_roe(const double* wL, const double* wR, double gamma, double* out, double* ref) {
   FastT fL, fR;
   double eL, HL, eR, HR, lmin, lmax;
-  side_fwd(wL, gamma, fL, eL, HL);
-  side_fwd(wR, gamma, fR, eR, HR);
+  Rev<false> A;
+  side_fwd(A, wL, gamma, fL, eL, HL);
+  side_fwd(A, wR, gamma, fR, eR, HR);
   RoeT rt;
-  roe_fwd(wL, wR, gamma, HL, HR, rt, lmin, lmax);
+  roe_fwd(A, wL, wR, gamma, HL, HR, rt, lmin, lmax);
   const double o[] = {fL.cf, eL, HL, fR.cf, eR, HR, lmin, lmax};
   Side L, R;
   side_state(wL, gamma, L);
@@ -846,14 +898,16 @@ void amr_debug_side_roe(const double* wL, const double* wR, double gamma, double
 
 void amr_debug_recon_minmod_vjp(const double* v, double wlb, double wrb, double* vb, double* wlr) {
   for (int s = 0; s < 4; s++) vb[s] = 0.;
-  recon_minmod_vjp(v, wlb, wrb, vb);
-  recon_minmod(v, wlr[0], wlr[1]);
+  Rev<false> A;
+  recon_minmod_vjp(A, v, wlb, wrb, vb);
+  recon_minmod(A, v, wlr[0], wlr[1]);
 }
 
 void amr_debug_prim_vjp(const double* u, double gamma, const double* wb, double* ub, double* w) {
   for (int k = 0; k < 8; k++) ub[k] = 0.;
-  prim_vjp(u, gamma, wb, ub);
-  prim_of(u, gamma, w);
+  Rev<false> A;
+  prim_vjp(A, u, gamma, wb, ub);
+  prim_of(A, u, gamma, w);
 }
 
 }  // extern "C"

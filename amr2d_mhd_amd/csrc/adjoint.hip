@@ -17,8 +17,10 @@
 // fluxes follow the faces; E[j][i] sits at the corner (i-1/2, j-1/2).
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 
 #include "../../include/amr2d_mhd.h"
@@ -111,12 +113,14 @@ struct FwdFaces {
 };
 
 // STAGE 1: out = U - dt res, Bn = B0 - dt r; 2: out = 0.5 (U + Us - dt res),
-// Bn = 0.5 (Bs + B0 - dt r).  pre: the cell B before the sync.
+// Bn = 0.5 (Bs + B0 - dt r).  pre: the cell B before the sync.  out may be U (a lane
+// reads its cell before it writes it); the faces written may not be faces read,
+// which neighbours read too.
 template <int STAGE>
-__global__ __launch_bounds__(kUx* kUy) void k_fwd_update(Grid G, const double* __restrict__ U,
-                                                         const double* __restrict__ Us, const double* __restrict__ Fx,
-                                                         const double* __restrict__ Fy, FwdFaces B, double dt,
-                                                         double* __restrict__ out, double* __restrict__ pre) {
+__global__ __launch_bounds__(kUx* kUy) void k_fwd_update(Grid G, const double* U, const double* __restrict__ Us,
+                                                         const double* __restrict__ Fx, const double* __restrict__ Fy,
+                                                         FwdFaces B, double dt, double* out,
+                                                         double* __restrict__ pre) {
   const int i = blockIdx.x * kUx + threadIdx.x % kUx, j = blockIdx.y * kUy + threadIdx.x / kUx;
   if (i >= G.n || j >= G.n) return;
   const int n = G.n, ip = wrap(i + 1, n), im = wrap(i - 1, n), jp = wrap(j + 1, n), jm = wrap(j - 1, n);
@@ -600,6 +604,23 @@ __global__ __launch_bounds__(2 * kVjpFaces) void k_stage_vjp_both(
 
 unsigned blocks(size_t n) { return (unsigned)((n + kT - 1) / kT); }
 
+// In-place calls: a kernel, not a copy of the runtime's, as a caller may capture it
+__global__ __launch_bounds__(kT) void k_copy(const double* __restrict__ from, double* __restrict__ to, size_t n) {
+  const size_t e = (size_t)blockIdx.x * kT + threadIdx.x;
+  if (e < n) to[e] = from[e];
+}
+
+struct Span {
+  const double* p;
+  size_t n;
+};
+bool overlap(std::initializer_list<Span> a, std::initializer_list<Span> b) {
+  for (const Span& x : a)
+    for (const Span& y : b)
+      if ((uintptr_t)x.p < (uintptr_t)(y.p + y.n) && (uintptr_t)y.p < (uintptr_t)(x.p + x.n)) return true;
+  return false;
+}
+
 }  // namespace
 
 struct amr_adj {
@@ -645,8 +666,16 @@ int forward_of(amr_adj* a, const double* U, const double* Bx, const double* By, 
                                               FwdFaces{Bx, By, nullptr, nullptr, T.Bxs, T.Bys, nullptr, nullptr}, dt,
                                               a->Us, T.pre1);
   launch_faces<SOLVER>(a, a->Us, T.Bxs, T.Bys, T.W2, s);
-  k_fwd_update<2><<<cells, kUx * kUy, 0, s>>>(G, U, a->Us, a->Fx, a->Fy,
-                                              FwdFaces{Bx, By, T.Bxs, T.Bys, Bxo, Byo, T.Bxo, T.Byo}, dt, Uo, T.pre2);
+  // in place the faces go to the tape alone, and out of it when all are formed
+  const size_t n2 = G.n2;
+  const bool in_place = overlap({{Bxo, n2}, {Byo, n2}}, {{U, 8 * n2}, {Bx, n2}, {By, n2}});
+  const FwdFaces faces = in_place ? FwdFaces{Bx, By, T.Bxs, T.Bys, T.Bxo, T.Byo, nullptr, nullptr}
+                                  : FwdFaces{Bx, By, T.Bxs, T.Bys, Bxo, Byo, T.Bxo, T.Byo};
+  k_fwd_update<2><<<cells, kUx * kUy, 0, s>>>(G, U, a->Us, a->Fx, a->Fy, faces, dt, Uo, T.pre2);
+  if (in_place) {
+    k_copy<<<blocks(n2), kT, 0, s>>>(T.Bxo, Bxo, n2);
+    k_copy<<<blocks(n2), kT, 0, s>>>(T.Byo, Byo, n2);
+  }
   ADJ_CHK(hipGetLastError());
   return 0;
 }
@@ -694,6 +723,17 @@ int reverse_of(amr_adj* a, const Tape& T, const double* Bx, const double* By, do
 
 int reverse(amr_adj* a, const Tape& T, const double* Bx, const double* By, double dt, const double* Uob,
             const double* Bxob, const double* Byob, double* Ub, double* Bxb, double* Byb, hipStream_t s) {
+  // in place from a copy of the cotangents, in buffers that only amr_adj_step_vjp's
+  // forward uses, before: the kernels read neighbours' while they write their own
+  const size_t n2 = a->G.n2;
+  if (overlap({{Ub, 8 * n2}, {Bxb, n2}, {Byb, n2}}, {{Uob, 8 * n2}, {Bxob, n2}, {Byob, n2}})) {
+    k_copy<<<blocks(8 * n2), kT, 0, s>>>(Uob, a->Uo, 8 * n2);
+    k_copy<<<blocks(n2), kT, 0, s>>>(Bxob, a->Bxo, n2);
+    k_copy<<<blocks(n2), kT, 0, s>>>(Byob, a->Byo, n2);
+    Uob = a->Uo;
+    Bxob = a->Bxo;
+    Byob = a->Byo;
+  }
   return a->solver == kFluxHLLD ? reverse_of<kFluxHLLD>(a, T, Bx, By, dt, Uob, Bxob, Byob, Ub, Bxb, Byb, s)
                                 : reverse_of<kFluxHLLE>(a, T, Bx, By, dt, Uob, Bxob, Byob, Ub, Bxb, Byb, s);
 }

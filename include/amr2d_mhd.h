@@ -292,8 +292,11 @@ int amr_profile_sample(amr_ctx *ctx, int stride);
  * discrete adjoint (U_b, Bx_b, By_b) = J^T (Uo_b, Bxo_b, Byo_b) (branch-wise at
  * limiter and wave-speed switches), without recomputing the step.
  * amr_adj_step_vjp recomputes the step from its input into the context's own
- * tape, then runs the reverse sweep.  Outputs must not alias inputs; calls on
- * one context are stream-ordered and share its work buffers. */
+ * tape, then runs the reverse sweep.  A step's outputs may be its inputs, and a
+ * reverse's its cotangents (in place: the same results, with two or three copies);
+ * otherwise outputs must not overlap inputs, nor ever the tape or the faces a
+ * reverse reads.  Calls on one context are stream-ordered and share its work
+ * buffers. */
 typedef struct amr_adj amr_adj;
 int amr_adj_create(int n, double dx, double gamma, const char *flux, amr_adj **out);
 int amr_adj_destroy(amr_adj *adj);
@@ -312,8 +315,8 @@ int amr_adj_step_vjp(amr_adj *adj, const double *U, const double *Bx, const doub
 /* amr_adj_step without a context and without allocating: no counterpart in
  * the reference.  For callers that cannot allocate device memory -- code
  * under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc.  Same step, same results as amr_adj_step on a context created
- * with (n, dx, gamma, flux).  Its work memory is a static device array the
+ * hipMalloc.  Same step, same results and same rule for overlapping arguments as
+ * amr_adj_step on a context created with (n, dx, gamma, flux).  Its work memory is a static device array the
  * library holds on every GPU it runs on until the process ends (25.2 MB), so
  * n is limited to 4..256 (AMR_ERR_CONFIG beyond).  Every call on one GPU
  * shares that array: calls that overlap on one GPU (different streams or

@@ -466,6 +466,11 @@ struct amr_ctx {
   int32_t* h_pull = nullptr;  // staging and scratch of the compiles on the device
   int32_t* d_pull = nullptr;
   int64_t cap_pull_h = 0, cap_pull = 0;
+  // programs compiled on the device, on the host, and of those after the device
+  // had tried; tests may lower the device's room {FillGen, pairs, linked ops, ops
+  // of a group}
+  int64_t compiled[3] = {0, 0, 0};
+  std::array<int32_t, 4> pull_room = {INT32_MAX, INT32_MAX, INT32_MAX, kFillChunk};
   char* slot_mem = nullptr;  // the allocation of all per-slot arrays (F, ring)
   // a step launched by step_begin and not yet completed by step_end
   bool in_flight = false;
@@ -2184,9 +2189,10 @@ int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
     p.leafs = c->dtree.leafs + off;
     p.nleaf = nleaf;
     p.main = chunks(nleaf * R);
-    p.cap_tail = chunks(p.main / 2 + 8 * kFillChunk);
-    p.cap_gen = p.main / 4 + 1024;
-    p.cap_edges = p.main;
+    p.cap_tail = std::min(chunks(p.main / 2 + 8 * kFillChunk), c->pull_room[2]);
+    p.cap_gen = std::min(p.main / 4 + 1024, c->pull_room[0]);
+    p.cap_edges = std::min(p.main, c->pull_room[1]);
+    p.max_group = c->pull_room[3];
     if (int e = ensure(I.d_ops, I.cap_ops, p.main + p.cap_tail)) return e;
     if (int e = ensure(I.d_gen, I.cap_gen, p.cap_gen)) return e;
     p.ops = I.d_ops;
@@ -2224,7 +2230,10 @@ int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
   std::vector<char> done(c->inst.size(), 0);
   for (int t = 0; t < n; t++) {
     const int32_t* m = c->h_pull + (size_t)t * kPullMeta;
-    if (m[kPullFlags] & ~kPullSelf) continue;
+    if (m[kPullFlags] & ~kPullSelf) {
+      c->compiled[2]++;
+      continue;
+    }
     Instance& I = c->inst[todo[t]];
     const int main = chunks((c->leaf_inst_begin[todo[t] + 1] - c->leaf_inst_begin[todo[t]]) * R);
     I.nops = main + m[kPullTail];
@@ -2235,7 +2244,9 @@ int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
     I.prog_dirty = false;
     done[todo[t]] = 1;
   }
+  const size_t before = dirty.size();
   dirty.erase(std::remove_if(dirty.begin(), dirty.end(), [&](int q) { return done[q]; }), dirty.end());
+  c->compiled[0] += (int64_t)(before - dirty.size());
   return 0;
 }
 
@@ -2270,7 +2281,8 @@ int rebuild_topology(amr_ctx* c) {
   }
   const auto t_compile = std::chrono::steady_clock::now();
   const int ncompile = (int)dirty.size();
-  if (int e = compile_on_device(c, dirty)) return e;  // the rest, below, on the host
+  if (int e = compile_on_device(c, dirty)) return e;
+  c->compiled[1] += (int64_t)dirty.size();  // the rest, below, on the host
   const int hw = (int)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
   int nthreads = (int)std::min<size_t>(dirty.size(), hw);
   if (nthreads < 1) nthreads = 1;
@@ -4233,6 +4245,25 @@ int amr_debug_pull_fill(int NT, int ng, int n, const int32_t* lp, const int32_t*
     for (size_t t = 0; t < at.size(); t++)
       differ += at[t] >= 0 && (bool)linked[t] != (at[t] / kFillChunk >= I.tail_chunk0);
   return differ;
+  AMR_CATCH
+}
+
+// Fill programs the context has compiled on the device, on the host, and of those
+// after the device had tried and found no room.
+int amr_debug_compiled(amr_ctx* c, int64_t* out) {
+  AMR_TRY
+  if (!c || !out) return AMR_ERR_CONFIG;
+  for (int k = 0; k < 3; k++) out[k] = c->compiled[k];
+  return AMR_OK;
+  AMR_CATCH
+}
+
+// Lowers the device compile's room (pull_room; tests of what follows when it ends).
+int amr_debug_pull_room(amr_ctx* c, int gen, int pairs, int tail, int group) {
+  AMR_TRY
+  if (!c || gen < 0 || pairs < 0 || tail < 0 || group < 1 || group > kFillChunk) return AMR_ERR_CONFIG;
+  c->pull_room = {gen, pairs, tail, group};
+  return AMR_OK;
   AMR_CATCH
 }
 

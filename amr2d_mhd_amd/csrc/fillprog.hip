@@ -189,17 +189,19 @@ __global__ __launch_bounds__(kThreads) void pull_size_kernel(const PullInst* __r
 
 __device__ inline int size_class(int n) { return n <= 1 ? 0 : 32 - __clz(n - 1); }
 
-// how many groups take room for each power of two
+// how many groups take room for each power of two.  (Other workgroups may set
+// kPullGroup meanwhile: a check of it could part a workgroup before its barriers.
+// The kernels after this one make it, or go by the flags of the ones before.)
 __global__ __launch_bounds__(kThreads) void pull_classes_kernel(const PullInst* __restrict__ insts) {
   const PullInst P = insts[blockIdx.y];
-  if (P.meta[kPullFlags] & ~kPullSelf) return;
+  if (P.meta[kPullFlags] & ~(kPullSelf | kPullGroup)) return;
   __shared__ int sCount[kClasses];
   if (threadIdx.x < kClasses) sCount[threadIdx.x] = 0;
   __syncthreads();
   const int k = blockIdx.x * kThreads + threadIdx.x;
   if (k < P.meta[kPullLinked] && P.root[k] == P.linked[k]) {
     const int n = P.size[P.linked[k]];
-    if (n > kFillChunk) atomicOr(&P.meta[kPullFlags], kPullGroup);
+    if (n > P.max_group) atomicOr(&P.meta[kPullFlags], kPullGroup);
     else atomicAdd(&sCount[size_class(n)], 1);
   }
   __syncthreads();

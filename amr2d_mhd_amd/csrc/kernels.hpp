@@ -109,12 +109,12 @@ void launch_ring_table(int NT, int ng, const FillOp* const* inst_ops, const int3
 // One instance whose fill program is compiled on the device (fillprog.hip): its
 // tree, slots and leaves (rank: a block's place in the leaf list), the program
 // (`main` ops, one per ring element of a leaf in order, padded to whole chunks,
-// then up to cap_tail of the linked groups), scratch of `main` entries each
-// (edges: cap_edges pairs) and the counters.
+// then up to cap_tail of the linked groups of up to max_group <= kFillChunk ops),
+// scratch of `main` entries each (edges: cap_edges pairs) and the counters.
 enum { kPullKinds = 0, kPullGen = 3, kPullLinked = 4, kPullEdges = 5, kPullFlags = 6, kPullTail = 7,
        kPullCount = 8, kPullNext = 20, kPullMeta = 32 };
-// flags: a restriction of a restriction, out of space, a group larger than a
-// chunk (the host compiles instead); an op that reads its own destination
+// flags: a restriction of a restriction, out of space, a group larger than
+// max_group (the host compiles instead); an op that reads its own destination
 enum { kPullNested = 1, kPullSpace = 2, kPullGroup = 4, kPullSelf = 8 };
 struct PullInst {
   const int32_t* lp;
@@ -123,7 +123,7 @@ struct PullInst {
   FillOp* ops;
   FillGen* gen;
   int32_t *uf, *size, *linked, *root, *edges, *meta;
-  int32_t nleaf, main, cap_tail, cap_gen, cap_edges;
+  int32_t nleaf, main, cap_tail, cap_gen, cap_edges, max_group;
 };
 // max_main, max_ops: the largest main and main + cap_tail of the n instances
 void launch_pull(int NT, int ng, const PullInst* insts, int n, int max_main, int max_ops, hipStream_t s);

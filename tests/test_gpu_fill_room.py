@@ -48,3 +48,43 @@ def test_group_larger_than_allowed():
     find one at once)."""
     device, host, again = _run((BIG, BIG, BIG, 1))
     assert device == 0 and again > 1 and host >= again
+
+
+@pytest.mark.parametrize("room", [(BIG, 0, BIG, 256), (BIG, 100, BIG, 256), (BIG, BIG, 0, 256), (BIG, BIG, 256, 256)],
+                         ids=["no pairs", "few pairs", "no tail", "one chunk of tail"])
+def test_out_of_room(room):
+    """No room for pairs of ops or linked ops, or for the first of them only.  (The
+    trees of these runs need no explicit operands.)"""
+    device, host, again = _run(room)
+    assert 0 < again <= host
+
+
+@pytest.mark.parametrize("cfg,steps", [
+    (dict(ic="rotor", limiter="minmod", flux="HLLC", cfl=0.5, nx=16, nghosts=2, maxlevs=5), 18),
+    (CFG, 27),
+    (dict(ic="OT", limiter="WENO5", flux="HLLD", cfl=0.4, nx=16, nghosts=4, maxlevs=5, periodic=True, rk_stages=3), 6),
+], ids=["20x20", "12x12", "24x24 periodic"])
+def test_every_large_tree_on_the_device(cfg, steps):
+    """With its own room the device compiles every changed tree of 8192 ring
+    elements or more, and the host every smaller one."""
+    import amr2d_mhd_amd as A
+
+    nt = cfg["nx"] + 2 * cfg["nghosts"]
+    ring = nt * nt - cfg["nx"] ** 2
+    sim = A.Simulation(cfg)
+    sim.init()
+    sim.set_fill_cache(0)
+    want = np.zeros(2, np.int64)
+    tree = sim.get_tree()[2].tobytes()
+    sim.step()  # (the initial tree's program)
+    before = _compiled(sim)
+    for _ in range(steps):
+        now = sim.get_tree()[2].tobytes()
+        if now != tree:  # compiled by the step that follows
+            want[0 if sim.info()["nleaf"] * ring >= 8192 else 1] += 1
+        tree = now
+        sim.step()
+    got = _compiled(sim) - before
+    sim.close()
+    assert want[0] > 1
+    assert got[2] == 0 and (got[:2] == want).all(), (got, want)

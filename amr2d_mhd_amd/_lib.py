@@ -128,7 +128,8 @@ _SIGS = {
     "amr_debug_compile": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int,
                                     C.c_void_p, C.c_void_p]),
     "amr_debug_compiled": (C.c_int, [C.c_void_p, C.c_void_p]),
-    "amr_debug_pull_room": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int]),
+    "amr_debug_pull_room": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]),
+    "amr_debug_drop_ct_tables": (C.c_int, [C.c_void_p]),
     "amr_debug_pull_fill": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "amr_debug_schedule": (C.c_int, [C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]),
     "amr_debug_stage_flops": (C.c_int, [C.c_void_p, C.c_int, C.c_void_p]),

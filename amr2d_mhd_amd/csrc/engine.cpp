@@ -460,7 +460,7 @@ struct amr_ctx {
   // compiled fill programs kept per instance besides the current one (LRU)
   int prog_cache_max = 4;
   // fill programs by destination and scratch of the fused CT launches, which
-  // serve the current trees when ct_fused
+  // serve the current trees when ct_fused (null where memory had no room for them)
   RingTable ring;
   bool ct_fused = false;
   int32_t* h_pull = nullptr;  // staging and scratch of the compiles on the device
@@ -468,9 +468,9 @@ struct amr_ctx {
   int64_t cap_pull_h = 0, cap_pull = 0;
   // programs compiled on the device, on the host, and of those after the device
   // had tried; tests may lower the device's room {FillGen, pairs, linked ops, ops
-  // of a group}
+  // of a group, words of scratch}
   int64_t compiled[3] = {0, 0, 0};
-  std::array<int32_t, 4> pull_room = {INT32_MAX, INT32_MAX, INT32_MAX, kFillChunk};
+  std::array<int32_t, 5> pull_room = {INT32_MAX, INT32_MAX, INT32_MAX, kFillChunk, INT32_MAX};
   char* slot_mem = nullptr;  // the allocation of all per-slot arrays (F, ring)
   // a step launched by step_begin and not yet completed by step_end
   bool in_flight = false;
@@ -2133,7 +2133,8 @@ constexpr int64_t kPullElements = 8192;
 
 // Compiles the programs of those `dirty` instances whose device trees are current
 // and of the form the look-up by destination takes; takes out of `dirty` those
-// that are done (the others the host compiles).
+// that are done (the others the host compiles, all of them where memory has no
+// room for the scratch or for programs with the device's margins).
 int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
   if (!c->regrid_device || dirty.empty()) return 0;
   const int R = ring_cells(c->NT, c->ng);
@@ -2147,6 +2148,11 @@ int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
   }
   if (todo.empty() || total < kPullElements || total > INT32_MAX / 4) return 0;
   auto chunks = [](int n) { return (n + kFillChunk - 1) / kFillChunk * kFillChunk; };
+  auto no_room = [](auto& p) {  // an allocation failed: clears its error
+    p = nullptr;
+    (void)hipGetLastError();
+    return 0;
+  };
   // staging: [instances | leaves, ranks, slots of each], then on the device only
   // the counters and the scratch
   const int n = (int)todo.size();
@@ -2164,15 +2170,16 @@ int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
     c->h_pull = nullptr;
     c->cap_pull_h = 0;
     const size_t cap = words + words / 2;
-    HIPCHK(hipHostMalloc((void**)&c->h_pull, sizeof(int32_t) * cap));
+    if (hipHostMalloc((void**)&c->h_pull, sizeof(int32_t) * cap) != hipSuccess) return no_room(c->h_pull);
     c->cap_pull_h = (int64_t)cap;
   }
   const size_t need = words + (size_t)n * kPullMeta + scratch;
+  if (need > (size_t)c->pull_room[4]) return 0;
   if (need > (size_t)c->cap_pull) {
     hipFree(c->d_pull);
     c->d_pull = nullptr;
     c->cap_pull = 0;
-    HIPCHK(hipMalloc((void**)&c->d_pull, sizeof(int32_t) * (need + need / 2)));
+    if (hipMalloc((void**)&c->d_pull, sizeof(int32_t) * (need + need / 2)) != hipSuccess) return no_room(c->d_pull);
     c->cap_pull = (int64_t)(need + need / 2);
   }
   PullInst* P = (PullInst*)c->h_pull;
@@ -2193,8 +2200,8 @@ int compile_on_device(amr_ctx* c, std::vector<int>& dirty) {
     p.cap_gen = std::min(p.main / 4 + 1024, c->pull_room[0]);
     p.cap_edges = std::min(p.main, c->pull_room[1]);
     p.max_group = c->pull_room[3];
-    if (int e = ensure(I.d_ops, I.cap_ops, p.main + p.cap_tail)) return e;
-    if (int e = ensure(I.d_gen, I.cap_gen, p.cap_gen)) return e;
+    if (ensure(I.d_ops, I.cap_ops, p.main + p.cap_tail)) return no_room(I.d_ops);
+    if (ensure(I.d_gen, I.cap_gen, p.cap_gen)) return no_room(I.d_gen);
     p.ops = I.d_ops;
     p.gen = I.d_gen;
     p.meta = meta + (size_t)t * kPullMeta;
@@ -2427,7 +2434,7 @@ int rebuild_topology(amr_ctx* c) {
   c->d_rgi = (RegridInst*)(c->d_topo + off_rgi);
   c->d_leaves = (LeafItem*)(c->d_topo + off_leaf);
   // the programs by destination, for the fused CT launches
-  c->ct_fused = true;
+  c->ct_fused = c->ring.entries != nullptr;
   for (const Instance& I : c->inst) c->ct_fused &= I.done || leaf_neighbours(I);
   if (c->ct_fused) {
     if (++c->ring.version == kRingVersions) {
@@ -3129,17 +3136,30 @@ int amr_create(int n_inst, const amr_sim_config* cfgs, int64_t slot_capacity, am
   auto place = [&](size_t n) { return std::exchange(bytes, bytes + (n + 4095) / 4096 * 4096); };
   size_t at[kNumFields];
   for (int f = 0; f < kNumFields; f++) at[f] = place(cell * kFieldVars[f]);
+  const size_t field_bytes = bytes;
   const size_t at_ring = place(ring_bytes(c)), at_emf = place(cell), at_old = place(2 * cell),
                at_rdx = place(sizeof(double) * c->cap_slots);
-  if (hipMalloc((void**)&c->slot_mem, bytes) != hipSuccess || hipMemset(c->slot_mem, 0, bytes) != hipSuccess) {
+  // slots that fill the memory go without the tables (9% of it): the CT then takes
+  // its separate launches
+  bool tables = true;
+  if (hipMalloc((void**)&c->slot_mem, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    c->slot_mem = nullptr;
+    tables = false;
+    bytes = field_bytes;
+    if (hipMalloc((void**)&c->slot_mem, bytes) != hipSuccess) c->slot_mem = nullptr;
+  }
+  if (!c->slot_mem || hipMemset(c->slot_mem, 0, bytes) != hipSuccess) {
     amr_destroy(c);
     return AMR_ERR_HIP;
   }
   for (int f = 0; f < kNumFields; f++) c->F.f[f] = (double*)(c->slot_mem + at[f]);
-  c->ring.entries = (uint64_t*)(c->slot_mem + at_ring);
-  c->ring.emf = (double*)(c->slot_mem + at_emf);
-  c->ring.old = (double*)(c->slot_mem + at_old);
-  c->ring.rdx = (double*)(c->slot_mem + at_rdx);
+  if (tables) {
+    c->ring.entries = (uint64_t*)(c->slot_mem + at_ring);
+    c->ring.emf = (double*)(c->slot_mem + at_emf);
+    c->ring.old = (double*)(c->slot_mem + at_old);
+    c->ring.rdx = (double*)(c->slot_mem + at_rdx);
+  }
   // error records, then the step kernel's barrier-failure flag
   c->rec_err_bytes = (sizeof(DevError) * n_inst + sizeof(int32_t) + 255) & ~size_t(255);
   // [error records | regrid records | op log | per-leaf CFL bounds and indicators]
@@ -4259,11 +4279,23 @@ int amr_debug_compiled(amr_ctx* c, int64_t* out) {
 }
 
 // Lowers the device compile's room (pull_room; tests of what follows when it ends).
-int amr_debug_pull_room(amr_ctx* c, int gen, int pairs, int tail, int group) {
+int amr_debug_pull_room(amr_ctx* c, int gen, int pairs, int tail, int group, int words) {
   AMR_TRY
-  if (!c || gen < 0 || pairs < 0 || tail < 0 || group < 1 || group > kFillChunk) return AMR_ERR_CONFIG;
-  c->pull_room = {gen, pairs, tail, group};
+  if (!c || gen < 0 || pairs < 0 || tail < 0 || group < 1 || group > kFillChunk || words < 0) return AMR_ERR_CONFIG;
+  c->pull_room = {gen, pairs, tail, group, words};
   return AMR_OK;
+  AMR_CATCH
+}
+
+// Leaves the context as amr_create does where memory has no room for the tables of
+// the fused CT; returns whether it had them, negative on error.
+int amr_debug_drop_ct_tables(amr_ctx* c) {
+  AMR_TRY
+  if (!c || c->in_flight) return -1;
+  const int had = c->ring.entries != nullptr;
+  c->ring = RingTable{};
+  c->ct_fused = false;
+  return had;
   AMR_CATCH
 }
 

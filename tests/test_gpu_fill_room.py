@@ -1,5 +1,6 @@
-"""The device compile of fill programs (fillprog.hip) out of room: the host
-compiles instead, with the same results, bitwise against the oracle."""
+"""The device compile of fill programs (fillprog.hip) and the tables of the fused
+constrained transport out of room: the host compiles, the separate launches run
+instead, with the same results, bitwise against the oracle."""
 import numpy as np
 import pytest
 
@@ -20,7 +21,7 @@ def _compiled(sim):
     return out
 
 
-def _run(room, cfg=CFG, steps=27):
+def _run(room, cfg=CFG, steps=27, tables=True):
     """Steps in lockstep with the oracle; the programs compiled on the device, on
     the host, and on the host after the device."""
     import amr2d_mhd_amd as A
@@ -30,7 +31,10 @@ def _run(room, cfg=CFG, steps=27):
     sim.init()
     assert dom.init() == 0
     sim.set_fill_cache(0)
-    assert lib().amr_debug_pull_room(sim.h, *room) == 0
+    assert lib().amr_debug_pull_room(sim.h, *(room + (BIG,))[:5]) == 0
+    if not tables:
+        assert lib().amr_debug_drop_ct_tables(sim.h) == 1
+        assert lib().amr_debug_drop_ct_tables(sim.h) == 0
     before = _compiled(sim)
     for step in range(steps):
         sim.step()
@@ -88,3 +92,17 @@ def test_every_large_tree_on_the_device(cfg, steps):
     sim.close()
     assert want[0] > 1
     assert got[2] == 0 and (got[:2] == want).all(), (got, want)
+
+
+@pytest.mark.parametrize("words", [0, 20000])
+def test_no_scratch(words):
+    """Memory without room for the device compile's scratch, for that of any tree
+    or of the larger ones."""
+    device, host, again = _run((BIG, BIG, BIG, 256, words))
+    assert again == 0 and host > 1 and (words or device == 0)
+
+
+@pytest.mark.parametrize("extra", [dict(), dict(ct_type=2, flux="HLLC"), dict(rk_stages=3)], ids=["RK2", "type 2", "RK3"])
+def test_no_tables(extra):
+    """A context whose memory had no room for the fused CT's tables."""
+    _run((BIG, BIG, BIG, 256), cfg=dict(CFG, maxlevs=5, **extra), steps=12, tables=False)

@@ -476,11 +476,13 @@ struct amr_ctx {
   bool in_flight = false;
   uint64_t prog_clock = 0;
   // stage-kernel variant: fixed (0..kStageVariants-1), or (-1) by stage_rule
-  // unless one was imported for the bucket of the leaf count
+  // unless one was imported for the bucket of a launch's leaf count
   int stage_variant = -1;
   struct StageBucket {
     int chosen = -1;    // imported
     bool used = false;  // stages have been launched in the bucket
+    double us[kStageVariants] = {0};  // sum of the timed launches' times per leaf
+    int64_t n[kStageVariants] = {0};
   };
   StageBucket stage_buckets[kStageSpecs][24];  // per stage-kernel specialisation
   int stage_spec = kStageGeneric;   // of the running instances (set at each topology rebuild)
@@ -544,7 +546,11 @@ struct amr_ctx {
   int64_t prof_seen[PF_COUNT] = {};
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::vector<std::array<hipEvent_t, 2>> ev_pool;
-  std::vector<std::pair<int, int>> ev_pending;  // (family, pool index)
+  struct TimedLaunch {
+    int family, slot;                          // slot: pool index
+    int variant = -1, nleaf = 0, bucket = 0, spec = 0;  // of a stage launch
+  };
+  std::vector<TimedLaunch> ev_pending;
 };
 
 namespace {
@@ -602,6 +608,7 @@ struct Timed {
   amr_ctx* c;
   int fam, slot = -1;
   bool attached;
+  amr_ctx::TimedLaunch launch{};
   Timed(amr_ctx* c_, int f, bool attached_ = false) : c(c_), fam(f), attached(attached_) {
     if (!(c->prof_mask & (1u << fam))) return;
     if (c->prof_seen[fam]++ % c->prof_stride) return;
@@ -619,7 +626,9 @@ struct Timed {
   ~Timed() {
     if (slot < 0) return;
     if (!attached) hipEventRecord(c->ev_pool[slot][1], c->stream);
-    c->ev_pending.push_back({fam, slot});
+    launch.family = fam;
+    launch.slot = slot;
+    c->ev_pending.push_back(launch);
   }
 };
 
@@ -650,9 +659,14 @@ void flush_profile(amr_ctx* c) {
   c->stamps_pending = 0;
   for (auto& p : c->ev_pending) {
     float ms = 0;
-    hipEventElapsedTime(&ms, c->ev_pool[p.second][0], c->ev_pool[p.second][1]);
-    c->prof[p.first].ms += ms;
-    c->prof[p.first].launches += 1;
+    hipEventElapsedTime(&ms, c->ev_pool[p.slot][0], c->ev_pool[p.slot][1]);
+    c->prof[p.family].ms += ms;
+    c->prof[p.family].launches += 1;
+    if (p.variant >= 0 && p.nleaf > 0) {
+      amr_ctx::StageBucket& B = c->stage_buckets[p.spec][p.bucket];
+      B.us[p.variant] += 1e3 * ms / p.nleaf;
+      B.n[p.variant] += 1;
+    }
   }
   c->ev_pending.clear();
 }
@@ -2476,29 +2490,31 @@ int leaf_bucket(int nleaf) {
 // that reads and writes the same field (SSP-RK3's second stage reads Us and
 // writes Us: one strip's update would race with another's loads of its halo
 // rows); such a stage runs as the wide kernel instead.
-int stage_variant_for(const amr_ctx* c, int step) {
-  const int b = c->stage_buckets[c->stage_spec][leaf_bucket(c->nleaf)].chosen;
-  const int v = c->stage_variant >= 0 ? c->stage_variant : b >= 0 ? b : stage_rule(c->nleaf);
+int stage_variant_for(const amr_ctx* c, int step, int nleaf) {
+  const int b = c->stage_buckets[c->stage_spec][leaf_bucket(nleaf)].chosen;
+  const int v = c->stage_variant >= 0 ? c->stage_variant : b >= 0 ? b : stage_rule(nleaf);
   return stage_kernel_of(v) == kStageStrips && c->rk == 3 && step == 2 ? kVariantWide : v;
 }
 
 void run_stage(amr_ctx* c, int step) {
-  const int v = stage_variant_for(c, step);
-  c->stage_buckets[c->stage_spec][leaf_bucket(c->nleaf)].used = true;
-  if (c->stage_split) {
-    // one launch per class of instances, each with its specialisation
-    for (int k = 0; k < c->split_n; k++) {
-      const int n = c->split_off[k + 1] - c->split_off[k];
-      if (n <= 0) continue;
-      Timed tm(c, PF_STAGE, true);
-      launch_stage(c->NT, c->ng, v, c->split_spec[k], c->F, c->d_split_leaves + c->split_off[k], n, c->d_ip, step,
-                   c->d_err, c->stream, tm.start(), tm.stop());
-    }
-    return;
+  // nleaf leaves in a grid for `grid`, of one specialisation
+  auto launch = [&](int spec, const LeafItem* leaves, int nleaf, int grid, const int32_t* counts) {
+    const int v = stage_variant_for(c, step, nleaf), b = leaf_bucket(nleaf);
+    c->stage_buckets[c->stage_spec][b].used = true;
+    Timed tm(c, PF_STAGE, true);
+    tm.launch.variant = v;
+    tm.launch.nleaf = nleaf;
+    tm.launch.bucket = b;
+    tm.launch.spec = c->stage_spec;
+    launch_stage(c->NT, c->ng, v, spec, c->F, leaves, grid, c->d_ip, step, c->d_err, c->stream, tm.start(), tm.stop(),
+                 counts);
+  };
+  if (!c->stage_split) return launch(c->stage_spec, c->d_leaves, c->nleaf, c->grid_leaves, c->launch_counts);
+  // one launch per class of instances, each with its specialisation
+  for (int k = 0; k < c->split_n; k++) {
+    const int n = c->split_off[k + 1] - c->split_off[k];
+    if (n > 0) launch(c->split_spec[k], c->d_split_leaves + c->split_off[k], n, n, nullptr);
   }
-  Timed tm(c, PF_STAGE, true);
-  launch_stage(c->NT, c->ng, v, c->stage_spec, c->F, c->d_leaves, c->grid_leaves, c->d_ip, step, c->d_err, c->stream,
-               tm.start(), tm.stop(), c->launch_counts);
 }
 
 // CT2D.cpp:11-124
@@ -2957,7 +2973,7 @@ int step_begin(amr_ctx* c) {
     k.epoch = c->topo_epoch;
     k.leaves = graph_capacity(c->gkey.leaves, c->nleaf, (int)std::min<int64_t>(c->cap_slots, INT32_MAX));
     k.chunks = graph_capacity(c->gkey.chunks, c->nchunks, INT32_MAX);
-    k.variant = stage_variant_for(c, 1);
+    k.variant = stage_variant_for(c, 1, c->nleaf);
     k.spec = c->stage_spec;
     c->grid_leaves = k.leaves;
     c->grid_chunks = k.chunks;
@@ -3853,7 +3869,7 @@ int amr_stage_tuning(amr_ctx* c, int nbuckets, int32_t* chosen, double* us_per_l
   const auto* buckets = c->stage_buckets[stage_spec_of(c)];
   for (int b = 0; b < nbuckets && b < 24; b++) {
     if (chosen) chosen[b] = buckets[b].chosen >= 0 || !buckets[b].used ? buckets[b].chosen : stage_rule(1 << b);
-    for (int v = 0; v < kStageVariants && us_per_leaf; v++) us_per_leaf[b * kStageVariants + v] = 0.0;
+    for (int v = 0; v < kStageVariants && us_per_leaf; v++) us_per_leaf[b * kStageVariants + v] = buckets[b].n[v] ? buckets[b].us[v] / buckets[b].n[v] : 0.0;
   }
   return AMR_OK;
   AMR_CATCH

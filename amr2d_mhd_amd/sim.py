@@ -229,7 +229,8 @@ class Simulation:
         _check(self.h, lib().amr_set_stage_variant(self.h, int(variant)))
 
     def stage_tuning(self, nbuckets=24):
-        """Variants in use: {leaf-count bucket: (variant, [zeros])}."""
+        """Variants in use: {leaf-count bucket: (variant, [mean us per leaf of each variant])}; the times are of
+        launches made while profile() timed stage kernels, 0 where there was none."""
         chosen = np.zeros(nbuckets, np.int32)
         us = np.zeros((nbuckets, STAGE_VARIANTS))
         _check(self.h, lib().amr_stage_tuning(self.h, nbuckets, chosen.ctypes.data, us.ctypes.data))

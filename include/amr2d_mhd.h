@@ -231,14 +231,17 @@ int amr_set_regrid_device(amr_ctx *ctx, int on);
  * second, runs as the wide kernel instead).  Each exists generic (solver and
  * limiter read per instance), specialised to HLLD or HLLC with a MUSCL-family
  * limiter, and, for nghosts 4, specialised to HLLD with WENO5; launches use a
- * specialisation when every running instance has its pair.  -1 (the default)
- * chooses by the number of leaf blocks: strips below 128, wide below 512,
- * narrow from there. */
+ * specialisation when every running instance has its pair, and where the pairs
+ * differ a stage is one launch a pair.  -1 (the default) chooses by the number of
+ * leaf blocks of the launch: strips below 128, wide below 512, narrow from
+ * there. */
 int amr_set_stage_variant(amr_ctx *ctx, int variant);
-/* Variants in use, per leaf-count bucket (bucket b holds 2^b <= nleaf <
- * 2^(b+1)) of the specialisation in use: chosen[b] is the imported variant,
- * or the default's where stages have run in the bucket, or -1.  us_per_leaf[b][8]
- * is filled with zeros (no launch is timed for the choice). */
+/* Variants in use, per bucket of a launch's leaf count (bucket b holds
+ * 2^b <= nleaf < 2^(b+1)) of the specialisation in use (the generic one where a stage
+ * is several launches): chosen[b] is the imported variant, or the default's where
+ * stages have run in the bucket, or -1.  us_per_leaf[b][8] are the mean
+ * microseconds per leaf block of each variant's launches while stage kernels were
+ * timed (amr_profile_enable), 0 where none was: no launch is timed for the choice. */
 int amr_stage_tuning(amr_ctx *ctx, int nbuckets, int32_t *chosen, double *us_per_leaf);
 /* Import variants: chosen[b] >= 0 fixes bucket b's variant for the
  * specialisation the context's running instances select; -1 leaves a bucket

@@ -145,3 +145,83 @@ def test_recon_batch_exponents_and_sizes(lim, ng, NT):
         assert same.all(), f"{lim}: tile {t} differs in {int((~same).sum())} entries"
     assert _same_bits(raw, out)[inside].all()
     assert (out[~inside].view(np.int64) == 0).all() and (raw[~inside] == 7.0).all()
+
+
+@pytest.mark.parametrize("lim,ng", [("1st", 2), ("noSL", 2), ("minmod", 2), ("VanLeer", 2), ("Superbee", 2),
+                                    ("MC", 2), ("Koren", 2), ("Cada3rd", 2), ("WENO3", 2), ("WENO5", 4)])
+def test_recon_batch_upper_exponents(lim, ng):
+    """Tiles on either side of the upper limit 2^100 and far beyond (WENO's weights
+    are fourth powers: 2^254 squares of squares below overflow, 2^300 beyond), whole and
+    mixed with small values."""
+    torch = pytest.importorskip("torch")
+    import amr2d_mhd_amd as A
+
+    rng = np.random.default_rng(13)
+    NT, scales = 20 if ng == 2 else 24, [98, 99, 100, 101, 200, 253, 300, 1000]
+    W = np.empty((2 * len(scales), 8, NT, NT))
+    for t, e in enumerate(scales):
+        w = rng.uniform(0.5, 2.0, (2, 8, NT, NT)) * rng.choice([-1.0, 1.0], (2, 8, NT, NT))
+        W[2 * t] = np.ldexp(w[0], e)
+        W[2 * t + 1] = np.ldexp(w[1], rng.integers(-e, e + 1, w[1].shape))
+    out = A.recon_batch(torch.from_numpy(W).cuda(), lim, ng, dx=1.0 / 30).cpu().numpy()
+    lo, hi = (ng - 1, NT - ng) if lim.startswith("WENO") else (0, NT - 2)
+    inside = np.zeros(out.shape[1:], bool)
+    inside[:, :, lo:hi + 1, lo:hi + 1] = True
+    inside[0:2, 5] = inside[2:4, 6] = False
+    compared = 0
+    for t in range(len(W)):
+        with np.errstate(all="ignore"):
+            (xl, xr, yl, yr), status = O.recon_tile(W[t], lim, ng, dx=1.0 / 30)
+        if status:  # the oracle stops at a NaN edge
+            continue
+        compared += 1
+        same = _same_bits(out[t], np.stack([xl, xr, yl, yr]))[inside]
+        assert same.all(), f"{lim}, 2^{scales[t // 2]}: tile {t} differs in {int((~same).sum())} entries"
+    assert compared >= (12 if lim.startswith("WENO") else 15)
+
+
+@pytest.mark.parametrize("lim,ng", [("minmod", 2), ("MC", 2), ("Cada3rd", 2), ("WENO3", 2), ("WENO5", 4)])
+@pytest.mark.parametrize("variant", [2, 3, 7])
+def test_stage_upper_exponents(lim, ng, variant):
+    """Stage 1 with densities around 2^+-60 and 2^+-100, momenta around 2^400, flux
+    differences around 2^480 and cells around 2^+-100, against the oracle's stage.  (Noise small enough that no edge
+    state is negative.)"""
+    import amr2d_mhd_amd as A
+
+    NT = 16 + 2 * ng
+    # exponents of density, pressure and the domain's length
+    cases = [(60, 60, 0), (-61, 59, 0), (98, 0, 0), (101, 0, 0), (-98, 0, 0), (-102, 0, 0), (99, 99, 0), (250, 540, 0),
+             (250, 560, 0), (0, 470, 0), (0, 490, 0), (0, 0, 98), (0, 0, 110), (0, 0, -92), (0, 0, -110),
+             (101, 101, -110)]
+    for er, ep, el in cases:
+        if lim.startswith("WENO") and ep > 240:  # its weights' fourth powers overflow
+            continue
+        cfg = dict(ic="rotor", limiter=lim, flux="HLLD", cfl=0.4, nx=16, nghosts=ng, maxlevs=1, lenx=2.0 ** el)
+        sim, dom = A.Simulation(cfg), O.Domain(**cfg)
+        sim.init()
+        assert dom.init() == 0
+        sim.set_stage_variant(variant)
+        rng = np.random.default_rng(abs(er) + 7)
+        v, b = 2.0 ** ((ep - er) / 2), 2.0 ** (ep / 2)
+        U = np.zeros((4, 8, NT, NT))
+        U[:, 0] = np.ldexp(rng.uniform(0.9, 1.1, (4, NT, NT)), er)
+        w = rng.normal(0, 0.1, (4, 6, NT, NT))
+        U[:, 1:4] = U[:, :1] * (w[:, :3] * v)
+        U[:, 5:8] = w[:, 3:] * b
+        U[:, 4] = np.ldexp(rng.uniform(9.5, 10.5, (4, NT, NT)), ep)
+        U[2:, [3, 7]] = 0.0  # blocks without z components
+        Bi = np.ascontiguousarray(U[:, 5:7])
+        dt = 1e-3 * 2.0 ** el / v
+        sim.upload("U", U)
+        sim.upload("Bi", Bi)
+        dom.set_field(O.U, U)
+        dom.set_field(O.BI, Bi)
+        sim.set_time(0.0, dt, dt, 1)
+        dom.set_time(0.0, dt, dt, 1)
+        sim.stage(1)
+        assert dom.stage(1) == 0
+        for f, of in (("Us", O.US), ("ff", O.FF), ("gg", O.GG)):
+            a, o = sim.download(f, nslots=4), dom.get_field(of, 4)
+            same = _same_bits(np.ascontiguousarray(a), np.ascontiguousarray(o))
+            assert same.all(), f"{lim}, rho 2^{er}, p 2^{ep}, length 2^{el}: {f} differs in {int((~same).sum())} values"
+        sim.close()

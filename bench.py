@@ -377,19 +377,6 @@ def stage_op_count(at=(1000, 2500, 4000)):
                 states=f"rotor states after steps {', '.join(str(s) for s in at)}")
 
 
-def rotor_tuning():
-    """Stage-kernel variants of the whole rotor run per leaf-count bucket, from an
-    untimed run (the timed runs import them)."""
-    import amr2d_mhd_amd as A
-
-    sim = A.Simulation(ROTOR)
-    sim.init()
-    sim.run(-1)
-    tun = {b: v[0] for b, v in sim.stage_tuning().items() if v[0] >= 0}
-    sim.close()
-    return tun
-
-
 STEP_KERNEL = 0  # engine step mode of the rotor runs (--step-kernel)
 REGRID_DEVICE = True  # regrid decided on the device (--regrid)
 FILL_STATS = False  # report the fill program's op mix at both ends of the window (--fill-stats)
@@ -398,7 +385,7 @@ FILL_STATS = False  # report the fill program's op mix at both ends of the windo
 EVENT_STRIDE = 15
 
 
-def rotor_run(warmup, steps, tuning):
+def rotor_run(warmup, steps):
     """`warmup` untimed steps of the rotor from t = 0, then `steps` timed
     steps (-1: to the end of the run) with the stage kernel's launches timed
     by HIP events on the engine's stream."""
@@ -407,7 +394,6 @@ def rotor_run(warmup, steps, tuning):
     import amr2d_mhd_amd as A
 
     sim = A.Simulation(ROTOR)
-    sim.set_stage_tuning(tuning)
     sim.set_step_kernel(STEP_KERNEL)
     sim.set_regrid_device(REGRID_DEVICE)
     sim.init()
@@ -495,9 +481,8 @@ def main():
         y.copy_(x)
         torch.cuda.synchronize()
 
-    tuning = rotor_tuning()
     steps = args.steps if args.steps >= 0 else -1
-    win = rotor_run(args.warmup, steps, tuning)
+    win = rotor_run(args.warmup, steps)
     if steps >= 0 and win["steps"] != steps:
         print(f"bench.py: run ended after {win['steps']} of {steps} timed steps", file=sys.stderr)
         return 1
@@ -529,8 +514,7 @@ def main():
                                       "persistent step kernel, 512 lanes"][args.step_kernel],
                    "regrid": ("on the device (markref, critneighup/down, updatelpup/down per instance; the host "
                               "reads back the op list)") if REGRID_DEVICE else "on the host (per-leaf indicators downloaded)",
-                   **({"fill_program": win["fill_program"]} if win["fill_program"] else {}),
-                   "stage_tuner": "variants by leaf count, imported from an untimed run"},
+                   **({"fill_program": win["fill_program"]} if win["fill_program"] else {})},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": STAGE_TRAFFIC_BYTES_PER_ZONE * zones_per_launch,
@@ -550,7 +534,7 @@ def main():
                                          note="flops_per_zone: one stage; a zone-update (one step) runs two "
                                               "stages, plus CT and the CFL reduction (not counted)")
     if not args.no_whole_run and not (args.warmup == 0 and args.steps in (-1, ROTOR_STEPS)):
-        w = rotor_run(0, -1, tuning)
+        w = rotor_run(0, -1)
         out["whole_run"] = {"workload": "the same rotor run, every step from t = 0 to t = 0.295", "steps": w["steps"],
                             "zone_updates": w["zone_updates"], "seconds": w["seconds"], "value": w["value"],
                             "ms_per_step": w["ms_per_step"], "t_reached": w["t_reached"]}
@@ -572,7 +556,7 @@ def main():
             else:
                 # the CPU times a bounded part of the GPU's window: time the GPU on that part too
                 a, b = cb["steps"]
-                g = rotor_run(a, b - a, tuning)
+                g = rotor_run(a, b - a)
                 out["gpu_on_cpu_window"] = {"steps": [a, b], "zone_updates": g["zone_updates"],
                                             "seconds": g["seconds"], "value": g["value"]}
                 out["gpu_over_cpu_same_window"] = g["value"] / cb["value"]

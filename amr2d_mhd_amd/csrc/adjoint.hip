@@ -471,12 +471,12 @@ __global__ __launch_bounds__(kT) void k_gather_prim_vjp(Grid G, const double* __
 // that read them; the normal-B adjoint of a face is added only by the tile that
 // owns the face.  Deterministic: fixed summation order, no atomics.
 // Bound by the solver reverse's arithmetic at the two wavefronts a SIMD its 250
-// registers allow.  Grids of no more tiles than CUs, which would be left half
+// registers allow (those of the plain quotients, out of line, within them).  Grids of no more tiles than CUs, which would be left half
 // idle, take 512 lanes with the y faces beside the x faces (k_stage_vjp_both);
 // others 256 lanes, the y faces after the x faces in the same LDS, two workgroups
-// a CU (k_stage_vjp).  The reverse of a step, HLLD, as 512 lanes and as 256: 54.6
-// and 63.5 us at 208 tiles (200 cells a side), 86.9 and 84.7 at 285, 220 and 203
-// at 1280 (512 a side).
+// a CU (k_stage_vjp).  The reverse of a step, HLLD, as 512 lanes and as 256: 54.5
+// and 67.5 us at 208 tiles (200 cells a side), 90.1 and 89.8 at 285, 98.0 and 95.9
+// at 456, 230 and 215 at 1280 (512 a side).
 constexpr int kVjpFaces = 256, kVjpW = 16, kVjpH = 13;
 constexpr int kVjpBothTiles = 256;  // CUs
 

@@ -46,11 +46,20 @@ bool tile_supported(int NT, int ng);
 //           update phases overlap
 //   strips  each block split into 4 row strips of 192 lanes (6, 7): four times
 //           the workgroups where the blocks alone leave CUs idle
-// stage_rule chooses by the number of leaf blocks of a launch.  Microseconds a
+// Of the narrow and strip kernels the HLLD and HLLC ones with a MUSCL limiter hold
+// their faces in the 168 VGPRs of three wavefronts a SIMD; the generic ones and
+// WENO5's spill 103 to 119 more (416 to 456 B a lane; the generic narrow one for
+// 12 x 12 tiles does not).  The wide ones take 137 to 146 and spill none.
+// stage_rule chooses by the number of leaf blocks of the launch.  Microseconds a
 // launch, rotor HLLD + MC (strips, wide, narrow): 52 blocks 10.9, 15.2, 19.3;
 // 136: 16.2, 16.0, 20.5; 196: 17.2, 16.5, 20.4; 340: 24.4, 25.7, 27.4; 436: 28.5,
 // 27.1, 28.3; 757: 41.2, 41.2, 34.3; 2352: 110, 117, 90.  HLLC + VanLeer at 100
-// blocks 15.1, 17.0, 23.6, HLLE at 340 25.7, 27.1, 28.4.
+// blocks 15.1, 17.0, 23.6, HLLE at 340 25.7, 27.1, 28.4, HLLD + WENO5 at 112 23.5,
+// 24.4, 43.0 and at 925 70.9, 69.8, 60.9.  (Between the lines strips and wide lie
+// within 6% of each other, either ahead as the blocks fill the 256 CUs.)  One rule for
+// all tiles, though blocks of 8 x 8 cells leave 606 of the wide kernel's lanes without
+// a face and do better with the narrow one from 160 blocks: 160 13.8, 11.1, 11.1; 340
+// 18.1, 18.4, 15.3; 664 20.3, 25.4, 17.4; 1918 38.7, 54.9, 31.2.
 enum { kStageWide, kStageNarrow, kStageStrips };
 constexpr int stage_kernel_of(int variant) {
   return variant >= 6 ? kStageStrips : variant == 0 || variant == 3 || variant == 4 ? kStageNarrow : kStageWide;
@@ -62,9 +71,8 @@ constexpr int kStageVariants = 8;
 // HLLD with a MUSCL-family limiter, or HLLD with WENO5 (24x24 tiles, the only
 // ones with the ghost depth WENO5 needs), fixed at compile time
 // or HLLC with a MUSCL-family limiter.  The specialised kernels are 2-7% faster
-// than the generic one with the same settings (rotor5 at 340 blocks: 25.7 and
-// 26.7 us; WENO5 narrow 28 and 40 us: the generic code overruns the
-// instruction cache).
+// than the generic one with the same settings (rotor at 340 blocks: 25.7 and
+// 26.7 us; WENO5 narrow at 925: 60.9 and 63.4).
 enum { kStageGeneric = 0, kStageHLLDMuscl = 1, kStageHLLDWeno5 = 2, kStageHLLCMuscl = 3, kStageSpecs = 4 };
 // Work-list counts on the device (counts[kCountLeaves], counts[kCountChunks]):
 // a launch given `counts` may have a larger grid than its work (a captured

@@ -354,9 +354,6 @@ __device__ inline void fill_chunk_nv(const FillProgram& P, const FillSet& set, i
   }
 }
 
-// field sets of the step (engine.cpp) with their combine kinds: {U, Bi},
-// {Bi, ff, gg}, {ff, gg}, one cell field, one face field, EMF; any other set
-// takes the per-field path
 // {U} or {U, Bi} (NB = 2) with a chunk's components over four workgroups, two each,
 // and Bi's in a fifth (blockIdx.y)
 template <int NB>
@@ -411,6 +408,9 @@ __global__ __launch_bounds__(kThreads) void fill_parts_kernel(FillProgram P, Fil
         [](int k, double a, double b, double c, double d) { return restrict_kind<kFillCell>(k, a, b, c, d); });
 }
 
+// The step's other field sets (engine.cpp) with their combine kinds: {U, Bi},
+// {Bi, ff, gg}, {ff, gg}, one cell field, one face field, EMF; any other set takes
+// the per-field path.
 template <int NV0, int NV1, int NV2, int K0, int K1, int K2>
 __global__ __launch_bounds__(kThreads) void fill_kernel_nv(FillProgram P, FillSet set, int NT,
                                                            const int32_t* __restrict__ counts) {
